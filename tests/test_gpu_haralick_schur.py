@@ -1,0 +1,70 @@
+"""GPU: the Schur kernels behind Haralick f14 at the sizes where their windows,
+bands and launch rules have edges, bit for bit against the oracle.
+
+The small-launch kernel chases a bulge in windows of 16 steps, keeps a band of
+64 columns in a wave and updates rows above a window 64 at a time, so matrix
+orders around multiples of 16 and 64 (order = number of gray tones) exercise
+its remainders; order 256 is the largest, and orders below 3 have no f14.
+Launches of up to 256 matrices, up to 6144 and beyond take different kernels."""
+import numpy as np
+import pytest
+
+import wndcharm
+from helpers import ALG_NAMES, orc_algorithm
+
+pytestmark = pytest.mark.gpu
+
+F14 = [16, 17]  # mean and range over the four angles
+
+
+def toned(ng, seed, shape=(40, 56)):
+    """an image whose quantised plane has exactly ng tones (0 and 255 among them)"""
+    rng = np.random.default_rng(1000 * ng + seed)
+    if ng == 1:
+        return np.full(shape, 7.0)
+    tones = np.concatenate([[0, 255], rng.permutation(np.arange(1, 255))[:ng - 2]]).astype(np.float64)
+    y, x = np.mgrid[0:shape[0], 0:shape[1]]
+    # smooth structure plus noise over the sorted tones, every tone at least once
+    u = (0.5 + 0.3 * np.sin(x / 5.0 + seed) * np.cos(y / 7.0) + 0.2 * rng.uniform(-1, 1, shape)).clip(0, 0.999)
+    idx = (u * ng).astype(int)
+    idx.reshape(-1)[rng.permutation(idx.size)[:ng]] = np.arange(ng)
+    return np.sort(tones)[idx]
+
+
+@pytest.mark.parametrize('ng', [1, 2, 3, 4, 5, 17, 18, 19, 20, 33, 34, 35, 63, 64, 65, 66, 80, 81, 82, 83, 127, 130,
+                                194, 195, 255, 256])
+def test_schur_orders_equal_oracle(ng):
+    img = toned(ng, 3, (64, 72) if ng > 128 else (40, 56))
+    print('schur order', ng, flush=True)
+    got = np.asarray(wndcharm.FeatureAlgorithm('Haralick Textures').execute(img))
+    assert wndcharm.last_haralick_work()[0][0] == ng
+    want = orc_algorithm(ALG_NAMES.index('Haralick Textures'), img)
+    assert np.array_equal(got[F14], want[F14], equal_nan=True), (got[F14], want[F14])
+
+
+def test_schur_low_rank_and_binary_planes_equal_oracle():
+    """matrices with zero rows, exact zeros below the diagonal and repeated
+    eigenvalues: deflations of one and two roots, reflectors of zero vectors"""
+    y, x = np.mgrid[0:48, 0:48]
+    planes = [((x // 8) % 2) * 255.0, (x % 5) * 51.0, ((x * y) % 17).astype(float), np.where(x == y, 255.0, x % 3),
+              (x // 3).astype(float)]
+    for k, img in enumerate(planes):
+        print('schur structured', k, flush=True)
+        got = np.asarray(wndcharm.FeatureAlgorithm('Haralick Textures').execute(img))
+        want = orc_algorithm(ALG_NAMES.index('Haralick Textures'), img)
+        assert np.array_equal(got[F14], want[F14], equal_nan=True), (k, got[F14], want[F14])
+
+
+def test_schur_launch_rules_agree():
+    """the same images in launches of 4 x 1, 4 x 100 and 4 x 1600 matrices (eight
+    waves, four waves and one wave per matrix) give the same bits"""
+    kinds = [toned(int(ng), s, (24, 32)) for s, ng in enumerate(np.linspace(3, 200, 100))]
+    plan = wndcharm.FeatureComputationPlan('haralick')
+    plan.add('Haralick Textures ()')
+    plan.finalize()
+    print('schur 1600 / 100 / 1', flush=True)
+    many = wndcharm.compute_features(kinds * 16, plan)
+    some = wndcharm.compute_features(kinds, plan)
+    one = np.concatenate([wndcharm.compute_features([im], plan) for im in kinds[::9]])
+    assert np.array_equal(many, np.concatenate([some] * 16), equal_nan=True)
+    assert np.array_equal(one, some[::9], equal_nan=True)

@@ -8,6 +8,7 @@
 // CPU oracle's restatement of that algorithm: every reduction that feeds a
 // decision is a per-thread sequential loop, parallelism is across the
 // independent rows / columns a reflector touches.
+#include <utility>
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -864,21 +865,14 @@ k_har_hess(const HarDesc *hd, const int *order) {
   }
 }
 
-// Francis QR on the Hessenberg matrix left in H.Q by k_har_hess.
-// NT threads per (angle, image).  The Schur iteration is a chain of
-// dependent steps, so for large batches many matrices per CU (NT = 64: a
-// small LDS window and one wave each) beat many waves per matrix.  For a
-// few matrices (a call of one or a few images) NT = 256: the chase still
-// runs on wave 0, while the strip updates after each window, whose columns
-// and rows are independent, take one round over 256 threads instead of
-// several over 64 (and the rows above the window one LDS chunk of up to 256
-// rows instead of chunks of 32).  Every entry receives the same operations
-// in the same order either way.
-template <int NT>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 64 ? 4 : 1)))
+// Francis QR on the Hessenberg matrix left in H.Q by k_har_hess, for launches
+// of many matrices: one wave per (angle, image), sixteen per CU.  The Schur
+// iteration is a chain of dependent steps, so many chains with a small LDS
+// window each keep the CU busy; k_har_schur below serves smaller launches.
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
 k_har_qr(const HarDesc *hd, const int *order) {
-  constexpr int RS = NT / 32;             // window rows per pass of the block (32 columns per row)
-  constexpr int CH = NT == 64 ? QW : NT;  // rows above the window staged per chunk
+  constexpr int RS = 2;   // window rows per pass of the wave (32 columns per row)
+  constexpr int CH = QW;  // rows above the window staged per chunk
   __shared__ double Rw[CH * QWP];
   __shared__ double rf[QB][4];
   __shared__ double sc[8];
@@ -1355,6 +1349,740 @@ k_har_qr(const HarDesc *hd, const int *order) {
 #undef AT
 }
 
+// ------------------------------------------------------- pipelined Schur form
+// The same Francis iteration as k_har_qr with a matrix's chain of dependent
+// steps on wave 0 alone, in registers, and everything off that chain on the
+// other three waves of the block, one window of PB steps behind.
+//
+//   wave 0 (chase)   lane l holds the open rows k, k+1, k+2 of column k0 + l.
+//     Per step: the reflector (the same in every lane), the left update of
+//     all 64 columns at once, then the right update of rows k+1..k+3 on the
+//     corner columns k..k+2, whose values are read from their lanes, updated
+//     in every lane and put back.  Row k goes to LDS.  A step's only LDS read
+//     is the row k+4, a step ahead; global memory is never touched.
+//   waves 1-3        left updates of the columns right of the band, one column
+//     per lane, following wave 0's reflectors through LDS (each carries its
+//     step's number) with the rows of the window loaded ahead; right updates
+//     of the previous window: its own PB rows and the rows above, through a
+//     wave-private LDS transpose; the next window's rows into LDS.
+//
+// One block barrier per window.  Every entry receives the same reflectors in
+// the same order, with the same operations, as in k_har_qr.  Subdiagonal
+// entries live in LDS (sub[i] = T(i,i-1)); the bulge below them is never
+// stored, as the iteration clears it at the end of every sweep.
+//
+// What bounds it: the chain, about 100 instructions of wave 0 per step, issued
+// one per four cycles (an FP64 instruction's rate; dependent ones gain nothing
+// on independent ones): 660 cycles per step, 28,000 steps for 240 tones.  With
+// one block of 256 threads chasing through an LDS window, as this kernel's
+// predecessor did, a step took 2,500 cycles: three LDS round trips, three IEEE
+// divisions and a square root with their scaling, and the strips in between.
+constexpr int PB = 16;        // steps per window
+constexpr int PWP = 65;       // padded row of a window buffer (64 columns)
+constexpr int PT = 64;        // rows of a transpose buffer
+constexpr int PTP = PB + 3;   // its padded row (odd)
+
+__device__ __forceinline__ double lane_value(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | lo);
+}
+
+// a / d and b / d with d's reciprocal y formed once: Newton steps to y, then
+// the quotient corrected by its exact remainder (Markstein).  Operands must
+// lie well inside the normal range (schur_in_range): the results are then the
+// correctly rounded quotients.
+__device__ __forceinline__ double recip_seed(double d) {
+  double y = __builtin_amdgcn_rcp(d);
+  double e = __builtin_fma(-d, y, 1.0);
+  y = __builtin_fma(y, e, y);
+  e = __builtin_fma(-d, y, 1.0);
+  return __builtin_fma(y, e, y);
+}
+__device__ __forceinline__ double quot(double a, double d, double y) {
+  const double q = a * y;
+  const double r = __builtin_fma(-d, q, a);
+  return __builtin_fma(r, y, q);
+}
+// sqrt(a) by a coupled Newton iteration on sqrt and 1 / (2 sqrt) with two
+// remainder corrections, for a well inside the normal range
+__device__ __forceinline__ double root(double a) {
+  const double y = __builtin_amdgcn_rsq(a);
+  double g = a * y, h = y * 0.5;
+  const double r = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  double d = __builtin_fma(-g, g, a);
+  g = __builtin_fma(d, h, g);
+  d = __builtin_fma(-g, g, a);
+  return __builtin_fma(d, h, g);
+}
+
+struct __align__(16) SchurRf {
+  double tau, e0, e1;
+  int gen, app;  // step number; whether the reflector is applied (beta != 0)
+};
+
+// steps 0, 1, .. while step(q) accepts, in groups of four up to lim (a
+// multiple of four); returns how many were done
+template <class Step, int... Q>
+__device__ __forceinline__ int schur_steps(Step &step, int lim, std::integer_sequence<int, Q...>) {
+  int done = 0;
+  (void)(((Q % 4 != 0 || Q < lim) && step(std::integral_constant<int, Q>()) && (done = Q + 1, true)) && ...);
+  return done;
+}
+typedef double schur_d2 __attribute__((ext_vector_type(2)));
+
+// Right reflectors of a window applied to one row, row[0..PB+1] = columns
+// k0..k1+1 (and on, unchanged): the steps whose bit is set in `on`, or all.
+template <bool ALL>
+__device__ __forceinline__ void schur_right(unsigned on, const SchurRf *rf, double *row) {
+  double x[PB + 2];
+#pragma unroll
+  for (int q = 0; q < PB + 2; q++) x[q] = row[q];
+  double u0 = x[0], u1 = x[1];
+  double tau = rf[0].tau, e0 = rf[0].e0, e1 = rf[0].e1;
+#pragma unroll
+  for (int q = 0; q < PB; q++) {
+    double ntau = 0, ne0 = 0, ne1 = 0;
+    if (q + 1 < PB) {  // the next step's reflector during this step
+      ntau = rf[q + 1].tau; ne0 = rf[q + 1].e0; ne1 = rf[q + 1].e1;
+    }
+    double u2 = x[q + 2];
+    double tt = u1 * e0;
+    tt += u2 * e1;
+    tt += u0;
+    const double w = tau * tt;
+    double n0 = u0 - w, n1 = u1 - w * e0, n2 = u2 - w * e1;
+    if (!ALL) {
+      __asm__ volatile("" : "+v"(n0), "+v"(n1), "+v"(n2));  // selects, no branches
+      const bool take = (int)(on << (31 - q)) < 0;
+      n0 = take ? n0 : u0;
+      n1 = take ? n1 : u1;
+      n2 = take ? n2 : u2;
+    }
+    row[q] = n0;
+    u0 = n1;
+    u1 = n2;
+    tau = ntau; e0 = ne0; e1 = ne1;
+    __asm__ volatile("" ::: "memory");
+  }
+  row[PB] = u0;
+  row[PB + 1] = u1;
+}
+
+template <int NW>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
+k_har_schur(const HarDesc *hd, const int *order) {
+  // window t's buffer (t mod 3): slot j first holds row k0+3+j, which wave 0
+  // reads at step j, then the finished row k0+j, which it writes at step j;
+  // column k0 + l at l
+  __shared__ double win[3][PB * PWP];
+  __shared__ double tbuf[NW][PT * PTP];
+  __shared__ SchurRf rf[2][PB];
+  __shared__ double hand[2][3][64];  // open rows k1, k1+1, k1+2 of the next window's columns k1..k1+63
+  __shared__ double dia[256], sup[256], sub[260];
+  __shared__ double fin[3];          // last reflector of the sweep: tau, e0, applied
+  __shared__ double dred;
+  __shared__ unsigned long long wm[NW];
+  const int angle = blockIdx.x;
+  const HarDesc H = hd[order[blockIdx.y]];
+  const int n = __builtin_amdgcn_readfirstlane(*H.ng);
+  gptr<double> A = to_global(H.Q + (long)angle * n * n);
+  // Which wave chases: two blocks share a CU (NW = 4), and their chases should
+  // not share a SIMD.  A block's waves go to the SIMDs in the order 0, 2, 1, 3
+  // from any start, so the first wave's SIMD and whether the block's LDS is the
+  // CU's first tell which wave sits where; any answer is correct.
+  __shared__ int s_rot;
+  if (NW == 4 && threadIdx.x == 0) {
+    const unsigned simd = (__builtin_amdgcn_s_getreg(4 | (31 << 11)) >> 4) & 3;   // HW_ID
+    const unsigned base = __builtin_amdgcn_s_getreg(6 | (31 << 11)) & 0xfff;      // LDS_ALLOC
+    const int pos = simd == 0 ? 0 : simd == 2 ? 1 : simd == 1 ? 2 : 3;
+    s_rot = (pos + (base ? 2 : 0)) & 3;
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  const int wave = NW == 4 ? (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) + __builtin_amdgcn_readfirstlane(s_rot)) & 3
+                           : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int t = wave * 64 + lane;
+#define AT(r, c) A[(unsigned)((r) * n + (c))]
+  // RealSchur::computeNormOfT as in k_har_qr
+  double *segs = win[0];
+  if (t < n) {
+    const int k0 = t - 1 > 0 ? t - 1 : 0;
+    gptr<const double> row = A + ((long)t * n + k0);
+    segs[t] = eigen_redux(n - k0, (int)(((long)t * n + k0) & 1), [&](int k) { return fabs(row[k]); });
+    sub[t] = t > 0 ? AT(t, t - 1) : 0.0;
+  }
+  __syncthreads();
+  if (t == 0) {
+    double sn = 0;
+    for (int j = 0; j < n; j++) sn += segs[j];
+    dred = sn;
+  }
+  if (t < 2 * PB) rf[t / PB][t % PB].gen = 0;
+  __syncthreads();
+  const double norm = dred;
+  const double eps = kDblEps;
+  // a bound on the Frobenius norm, hence on every entry: reflections keep it,
+  // and an exceptional shift s, |s| <= 2 |T|, adds at most 2 sqrt(n) of it
+  double cap = norm;
+  if (wave == 0) __builtin_amdgcn_s_setprio(3);  // the chain first where it shares its SIMD
+  // decision state: every thread keeps it, from the same LDS values
+  int iu = n - 1, iter = 0, totalIter = 0;
+  double exshift = 0;
+  double work = 0;
+  int base = 0;  // steps published so far
+  // highest thread index with a hit over the block (none: -1)
+  auto highest = [&](bool hit) {
+    const unsigned long long m = __ballot(hit);
+    if (lane == 0) wm[wave] = m;
+    __syncthreads();
+    int r = -1;
+#pragma unroll
+    for (int w = 0; w < NW; w++)
+      if (wm[w]) r = 64 * w + 63 - __clzll((long long)wm[w]);
+    return __builtin_amdgcn_readfirstlane(r);
+  };
+  bool reload = true;
+  while (norm != 0 && iu >= 0) {
+    __syncthreads();  // the previous step's stores and LDS reads are complete
+    iu = __builtin_amdgcn_readfirstlane(iu);  // the same in every thread: scalar branches and indices
+    if (reload) {
+      if (t <= iu) {
+        dia[t] = AT(t, t);
+        sup[t] = t < iu ? AT(t, t + 1) : 0.0;
+      }
+      reload = false;
+      __syncthreads();
+    }
+    // findSmallSubdiagEntry: the largest res in (0, iu] with a negligible subdiagonal entry
+    bool hit = false;
+    if (t > 0 && t <= iu) {
+      double s = fabs(dia[t - 1]) + fabs(dia[t]);
+      if (s == 0.0) s = norm;
+      hit = fabs(sub[t]) < eps * s;
+    }
+    const int il = max(highest(hit), 0);
+    if (il == iu) {  // one root
+      __syncthreads();
+      if (t == 0) {
+        const double d = dia[iu] + exshift;
+        dia[iu] = d;
+        AT(iu, iu) = d;
+        if (iu > 0) sub[iu] = 0;
+      }
+      iu--;
+      iter = 0;
+      continue;
+    }
+    if (il == iu - 1) {  // two roots (RealSchur::splitOffTwoRows)
+      const double p = 0.5 * (dia[iu - 1] - dia[iu]);
+      const double q = p * p + sub[iu] * sup[iu - 1];
+      const double a00 = dia[iu - 1] + exshift, a01 = sup[iu - 1], a10 = sub[iu], a11 = dia[iu] + exshift;
+      __syncthreads();
+      if (q >= 0) {
+        const double z = sqrt(fabs(q));
+        const double pp = (p >= 0) ? p + z : p - z, qq = a10;
+        double c, s;  // JacobiRotation::makeGivens, real case
+        if (qq == 0) { c = pp < 0 ? -1 : 1; s = 0; }
+        else if (pp == 0) { c = 0; s = qq < 0 ? 1 : -1; }
+        else if (fabs(pp) > fabs(qq)) {
+          const double tt = qq / pp;
+          double u = sqrt(1 + tt * tt);
+          if (pp < 0) u = -u;
+          c = 1 / u; s = -tt * c;
+        } else {
+          const double tt = pp / qq;
+          double u = sqrt(1 + tt * tt);
+          if (qq < 0) u = -u;
+          s = -1 / u; c = -tt * s;
+        }
+        // left on columns iu-1, iu, then right on rows 0..iu
+        const double b00 = c * a00 - s * a10, b10 = s * a00 + c * a10;
+        const double b01 = c * a01 - s * a11, b11 = s * a01 + c * a11;
+        if (t <= iu) {
+          double xv, yv;
+          if (t == iu - 1) { xv = b00; yv = b01; }
+          else if (t == iu) { xv = b10; yv = b11; }
+          else { xv = AT(t, iu - 1); yv = AT(t, iu); }
+          const double l = c * xv - s * yv, rr = s * xv + c * yv;
+          if (t < iu) AT(t, iu - 1) = l;
+          AT(t, iu) = rr;
+        }
+        if (t == 0) { sub[iu] = 0; work += 6.0 * (2 + iu + 1); }
+      } else if (t == 0) {
+        AT(iu, iu) = a11;
+        AT(iu - 1, iu - 1) = a00;
+      }
+      if (t == 0 && iu > 1) sub[iu - 1] = 0;
+      iu -= 2;
+      iter = 0;
+      reload = true;
+      continue;
+    }
+    // ---- Francis QR step (RealSchur::computeShift)
+    double sh0 = dia[iu], sh1 = dia[iu - 1], sh2 = sub[iu] * sup[iu - 1];
+    double amt = 0;
+    int shift_kind = 0;
+    if (iter == 10) {
+      exshift += sh0;
+      shift_kind = 1;
+      amt = sh0;
+      const double s = fabs(sub[iu]) + fabs(sub[iu - 1]);
+      sh0 = 0.75 * s; sh1 = 0.75 * s; sh2 = -0.4375 * s * s;
+    }
+    if (iter == 30) {
+      double s = (sh1 - sh0) / 2.0;
+      s = s * s + sh2;
+      if (s > 0) {
+        s = sqrt(s);
+        if (sh1 < sh0) s = -s;
+        s = s + (sh1 - sh0) / 2.0;
+        s = sh0 - sh2 / s;
+        exshift += s;
+        shift_kind = 2;
+        amt = s;
+        sh0 = sh1 = sh2 = 0.964;
+      }
+    }
+    iter++;
+    totalIter++;
+    if (totalIter > 40 * n) break;
+    __syncthreads();
+    if (shift_kind) {
+      cap *= 64;
+      if (t <= iu) {
+        const double d = dia[t] - amt;
+        dia[t] = d;
+        AT(t, t) = d;
+      }
+      work += iu + 1;
+      __syncthreads();
+    }
+    // initFrancisQRStep: the largest im in (il, iu-2] passing the small-subdiagonal test, else il
+    hit = false;
+    if (t > il && t <= iu - 2) {
+      const double Tmm = dia[t];
+      const double r = sh0 - Tmm, s = sh1 - Tmm;
+      const double v0 = (r * s - sh2) / sub[t + 1] + sup[t];
+      const double v1 = dia[t + 1] - Tmm - r - s;
+      const double v2 = sub[t + 2];
+      const double lhs = sub[t] * (fabs(v1) + fabs(v2));
+      const double rhs = v0 * (fabs(dia[t - 1]) + fabs(Tmm) + fabs(dia[t + 1]));
+      hit = fabs(lhs) < eps * rhs;
+    }
+    const int im = max(highest(hit), il);
+    {  // 12 operations for each of the iu-k+1 columns and min(iu, k+3)+1 rows of steps im..iu-2
+      const int a = iu - im, m = a - 2;
+      work += 12.0 * ((a + 1) * (a + 2) / 2 - 3 + m * (im + iu - 3) / 2 + 4 * m + iu + 1);
+    }
+    double x0, x1, x2;
+    {
+      const double Tmm = dia[im];
+      const double r = sh0 - Tmm, s = sh1 - Tmm;
+      x0 = (r * s - sh2) / sub[im + 1] + sup[im];
+      x1 = dia[im + 1] - Tmm - r - s;
+      x2 = sub[im + 2];
+    }
+    // ---- first window's rows im+3 .. im+PB+2 (slots 0..PB-1), columns im .. im+63; its open rows
+    {
+      const int c = im + lane, cc = min(c, iu);
+      double v[PB / NW], o = 0;
+#pragma unroll
+      for (int j = 0; j < PB / NW; j++) v[j] = AT(min(im + 3 + wave + NW * j, iu), cc);
+      if (wave < 3) o = AT(min(im + wave, iu), cc);
+#pragma unroll
+      for (int j = 0; j < PB / NW; j++) {
+        const int r = im + 3 + wave + NW * j;
+        win[0][(wave + NW * j) * PWP + lane] = c >= r ? v[j] : c == r - 1 ? sub[min(r, iu)] : 0.0;
+      }
+      if (wave < 3) {  // the bulge's columns: subdiagonal entries, then zeros
+        if (lane < wave) o = lane == wave - 1 ? sub[im + wave] : 0.0;
+        hand[0][wave][lane] = o;
+      }
+    }
+    const int sc = im + t;  // column of a lane of waves 1-3: im + 64 + (t - 64)
+    double s0 = 0, s1 = 0;  // its open rows
+    if (wave > 0 && sc <= iu) {
+      s0 = AT(im, sc);
+      s1 = AT(im + 1, sc);
+    }
+    const double subim = sub[im];
+    __syncthreads();
+    int par = 0, wcur = 0;
+    int pk0 = 0, pn = 0;  // previous window: first step, steps (0: none)
+    // right updates of the previous window on rows k1-1 down to 0, PT rows per
+    // item: its own rows (from its buffer), then the rows above (from global
+    // memory), through the wave's transpose buffer
+    auto right_items = [&](int first, int stride, bool last) {
+      const SchurRf *rp = rf[par ^ 1];
+      const double *wp = win[wcur == 0 ? 2 : wcur - 1];
+      const unsigned fon = (unsigned)__ballot(lane < pn && rp[min(lane, PB - 1)].app != 0);
+      const bool full = fon == (1u << PB) - 1;
+      const int nc = pn + 2, nrow = pk0 + pn;
+      double *tb = tbuf[wave];
+      for (int it = first; it * PT < nrow; it += stride) {
+        const int rtop = nrow - 1 - it * PT;  // row of tb's row 0; row rr holds rtop - rr
+        const int nr = min(PT, rtop + 1), own = it == 0 ? pn : 0;
+        int rb = lane >> 5;
+        asm volatile("" : "+v"(rb));  // per-row values are formed here, not hoisted
+        const int cl5 = lane & 31, cc = min(cl5, nc - 1);
+#pragma unroll
+        for (int h = 0; h < PT / 2; h += 16) {
+          double v[16];
+#pragma unroll
+          for (int j = 0; j < 16; j++) v[j] = AT(max(rtop - (rb + 2 * (h + j)), 0), pk0 + cc);
+          if (own && h == 0) {
+#pragma unroll
+            for (int j = 0; j < PB / 2; j++) {
+              const int rr = rb + 2 * j;
+              const double o = wp[max(pn - 1 - rr, 0) * PWP + cc];
+              v[j] = rr < own ? o : v[j];
+            }
+          }
+          if (cl5 < nc)
+#pragma unroll
+            for (int j = 0; j < 16; j++) tb[(rb + 2 * (h + j)) * PTP + cl5] = v[j];
+        }
+        wave_sync();
+        if (lane < nr) {
+          double *row = tb + lane * PTP;
+          if (full && !own) schur_right<true>(0, rp, row);
+          // a row of the window takes part from its own step on
+          else schur_right<false>(own ? fon & (~0u << max(pn - 1 - lane, 0)) : fon, rp, row);
+          if (last && fin[2] != 0.0) {
+            const double tau = fin[0], e0 = fin[1], u0 = row[pn], u1 = row[pn + 1];
+            double tt = u1 * e0;
+            tt += u0;
+            const double w = tau * tt;
+            row[pn] = u0 - w;
+            row[pn + 1] = u1 - w * e0;
+          }
+        }
+        wave_sync();
+        asm volatile("" : "+v"(rb));
+        if (cl5 < nc) {
+          gptr<double> g = A + ((long)(rtop - rb) * n + pk0 + cl5);
+#pragma unroll
+          for (int h = 0; h < PT / 2; h += 8) {
+            double o[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) o[j] = tb[(rb + 2 * (h + j)) * PTP + cl5];
+            if ((own == 0 || 2 * h >= own) && 2 * h + 16 <= nr) {
+#pragma unroll
+              for (int j = 0; j < 8; j++) g[-(long)(2 * (h + j)) * n] = o[j];
+            } else {  // a window row stores its columns from the diagonal on
+#pragma unroll
+              for (int j = 0; j < 8; j++) {
+                const int rr = rb + 2 * (h + j), r = rtop - rr;
+                if (r >= 0 && pk0 + cl5 >= (rr < own ? r : 0)) AT(r, pk0 + cl5) = o[j];
+              }
+            }
+          }
+        }
+        wave_sync();
+      }
+      // the window rows' columns beyond its right updates
+      if (wave == NW - 1 && lane >= nc && pk0 + lane <= iu) {
+        double o[PB];
+#pragma unroll
+        for (int j = 0; j < PB; j++) o[j] = wp[j * PWP + lane];
+#pragma unroll
+        for (int j = 0; j < PB; j++)
+          if (j < pn) AT(pk0 + j, pk0 + lane) = o[j];
+      }
+    };
+    // after the last window one round more applies its right updates, on all waves
+    for (int k0 = im;; k0 += PB) {
+      const bool chase = k0 <= iu - 2;
+      const int k1 = min(k0 + PB, iu - 1), nstep = k1 - k0;
+      const bool more = k1 < iu - 1;
+      const int wnext = wcur == 2 ? 0 : wcur + 1;
+      if (wave == 0 && chase) {
+        double *W = win[wcur];
+        double a0 = hand[par][0][lane], a1 = hand[par][1][lane], a2 = hand[par][2][lane];
+        double nv = W[lane];
+        SchurRf *R = rf[par];
+        // one step with operands well inside the normal range (false: not
+        // done).  q is a constant in each of the PB copies, so lanes, lane
+        // masks and LDS offsets are
+        const unsigned rfa = (unsigned)(uintptr_t)(__attribute__((address_space(3))) SchurRf *)R;
+        const unsigned sba = (unsigned)(uintptr_t)(__attribute__((address_space(3))) double *)(sub + k0);
+        auto fast = [&](auto qc) __attribute__((always_inline)) {
+          constexpr int q = decltype(qc)::value;
+          double least;
+          __asm__("v_min_f64 %0, |%1|, |%2|" : "=v"(least) : "v"(x1), "v"(x2));
+          if (__builtin_expect(__ballot(least >= 0x1p-350) == 0, 0)) return false;
+          double tail = x1 * x1;
+          tail += x2 * x2;
+          double bb = root(x0 * x0 + tail);
+          if (x0 >= 0) bb = -bb;
+          const double den = x0 - bb;
+          const double yd = recip_seed(den), yb = recip_seed(bb);
+          const double e0 = quot(x1, den, yd), e1 = quot(x2, den, yd);
+          const double tau = quot(-den, bb, yb);  // bb - x0 = -den exactly
+          const schur_d2 o0 = {tau, e0}, o1 = {e1, __longlong_as_double((1ll << 32) | (unsigned)(base + q + 1))};
+          // one lane writes the reflector, its step number last
+          __asm__ volatile(
+              "s_mov_b64 exec, 1\n\tds_write_b128 %0, %2 offset:%5\n\tds_write_b128 %0, %3 offset:%6\n\t"
+              "ds_write_b64 %1, %4 offset:%7\n\ts_mov_b64 exec, -1"
+              :
+              : "v"(rfa), "v"(sba), "v"(o0), "v"(o1), "v"(bb), "n"(q * (int)sizeof(SchurRf)),
+                "n"(q * (int)sizeof(SchurRf) + 16), "n"(q * 8)
+              : "memory");
+          double tt = e0 * a1;
+          tt += e1 * a2;
+          tt += a0;
+          a0 -= tau * tt;
+          a1 -= (tau * e0) * tt;
+          a2 -= (tau * e1) * tt;
+          W[q * PWP + lane] = a0;
+          const double r10 = lane_value(a1, q), r11 = lane_value(a1, q + 1), r12 = lane_value(a1, q + 2);
+          const double r20 = lane_value(a2, q), r21 = lane_value(a2, q + 1), r22 = lane_value(a2, q + 2);
+          const double s3 = lane_value(nv, q + 2);
+          tt = r11 * e0; tt += r12 * e1; tt += r10;
+          const double w1 = tau * tt;
+          x0 = r10 - w1;
+          tt = r21 * e0; tt += r22 * e1; tt += r20;
+          const double w2 = tau * tt;
+          x1 = r20 - w2;
+          tt = s3 * e1 + 0.0;  // (0 * e0 + s3 * e1) + 0 with e0 finite
+          const double w3 = tau * tt;
+          x2 = 0.0 - w3;
+          // columns k+1 (factor e0) and k+2 (e1) of rows k+1..k+3, in their own lanes
+          double f, m1, m2, m3;
+          __asm__ volatile(
+              "s_mov_b64 exec, %12\n\tv_mov_b64 %3, %10\n\ts_mov_b64 exec, %13\n\tv_mov_b64 %3, %11\n\t"
+              "s_mov_b64 exec, %14\n\tv_mul_f64 %4, %7, %3\n\tv_mul_f64 %5, %8, %3\n\tv_mul_f64 %6, %9, %3\n\t"
+              "v_add_f64 %0, %0, -%4\n\tv_add_f64 %1, %1, -%5\n\tv_add_f64 %2, %2, -%6\n\ts_mov_b64 exec, -1"
+              : "+v"(a1), "+v"(a2), "+v"(nv), "=&v"(f), "=&v"(m1), "=&v"(m2), "=&v"(m3)
+              : "v"(w1), "v"(w2), "v"(w3), "v"(e0), "v"(e1), "n"(1 << (q + 1)), "n"(1 << (q + 2)), "n"(3 << (q + 1)));
+          a0 = a1;
+          a1 = a2;
+          a2 = nv;
+          if (q + 1 < PB) nv = W[(q + 1) * PWP + lane];
+          return true;
+        };
+        // the first vector is no entry of T: its size is checked apart
+        const bool sized = __ballot(cap <= 0x1p340) && (k0 > im || __ballot(fabs(x0) <= 0x1p340 && fabs(x1) <= 0x1p340 && fabs(x2) <= 0x1p340));
+        const int done = schur_steps(fast, sized ? nstep & ~3 : 0, std::make_integer_sequence<int, PB>());
+        // the steps left: the last of a short window, or out-of-range operands
+        for (int q = done; q < nstep; q++) {
+          double tail = x1 * x1;
+          tail += x2 * x2;
+          double tau = 0, e0 = 0, e1 = 0, beta = x0;
+          if (tail != 0.0) {
+            double bb = sqrt(x0 * x0 + tail);
+            if (x0 >= 0) bb = -bb;
+            e0 = x1 / (x0 - bb);
+            e1 = x2 / (x0 - bb);
+            tau = (bb - x0) / bb;
+            beta = bb;
+          }
+          const bool app = __ballot(beta != 0) != 0;
+          if (lane == 0) {
+            R[q].tau = tau;
+            R[q].e0 = e0;
+            R[q].e1 = e1;
+            R[q].app = app;
+            sub[k0 + q] = beta;
+            __asm__ volatile("" ::: "memory");
+            R[q].gen = base + q + 1;
+          }
+          double w1 = 0, w2 = 0, w3 = 0;
+          if (app) {
+            double tt = e0 * a1;
+            tt += e1 * a2;
+            tt += a0;
+            a0 -= tau * tt;
+            a1 -= (tau * e0) * tt;
+            a2 -= (tau * e1) * tt;
+          }
+          W[q * PWP + lane] = a0;
+          x0 = lane_value(a1, q);
+          x1 = lane_value(a2, q);
+          x2 = 0.0;
+          if (app) {
+            double tt = lane_value(a1, q + 1) * e0;
+            tt += lane_value(a1, q + 2) * e1;
+            tt += x0;
+            w1 = tau * tt;
+            tt = lane_value(a2, q + 1) * e0;
+            tt += lane_value(a2, q + 2) * e1;
+            tt += x1;
+            w2 = tau * tt;
+            tt = 0.0 * e0;
+            tt += lane_value(nv, q + 2) * e1;
+            tt += 0.0;
+            w3 = tau * tt;
+            x0 -= w1;
+            x1 -= w2;
+            x2 -= w3;
+            const double f = lane == q + 1 ? e0 : e1;
+            if (lane == q + 1 || lane == q + 2) {
+              a1 -= w1 * f;
+              a2 -= w2 * f;
+              nv -= w3 * f;
+            }
+          }
+          a0 = a1;
+          a1 = a2;
+          a2 = nv;
+          if (q + 1 < PB) nv = W[(q + 1) * PWP + lane];
+        }
+        if (lane == 0 && k0 == im)  // T(im, im-1): negated where the first reflector applies above il
+          sub[im] = im > il && rf[par][0].app ? -subim : subim;
+        if (more) {
+          if (lane >= PB) {
+            hand[par ^ 1][0][lane - PB] = a0;
+            hand[par ^ 1][1][lane - PB] = a1;
+            hand[par ^ 1][2][lane - PB] = a2;
+          }
+        } else {  // the last reflector: rows iu-1, iu, columns iu-1, iu
+          double p00 = lane_value(a0, nstep), p01 = lane_value(a0, nstep + 1);
+          double p10 = lane_value(a1, nstep), p11 = lane_value(a1, nstep + 1);
+          double tail = 0;
+          tail += x1 * x1;
+          double tau = 0, e0 = 0, beta = x0;
+          if (tail != 0.0) {
+            double bb = sqrt(x0 * x0 + tail);
+            if (x0 >= 0) bb = -bb;
+            e0 = x1 / (x0 - bb);
+            tau = (bb - x0) / bb;
+            beta = bb;
+          }
+          const bool app = beta != 0;
+          if (app) {
+            const double f0 = tau * e0;
+            double tt = e0 * p10; tt += p00;
+            p00 -= tau * tt; p10 -= f0 * tt;
+            tt = e0 * p11; tt += p01;
+            p01 -= tau * tt; p11 -= f0 * tt;
+            tt = p01 * e0; tt += p00;
+            double w = tau * tt;
+            p00 -= w; p01 -= w * e0;
+            tt = p11 * e0; tt += p10;
+            w = tau * tt;
+            p10 -= w; p11 -= w * e0;
+            work += 6.0 * (2 + iu + 1);
+          }
+          if (lane == 0) {
+            sub[iu - 1] = beta;
+            sub[iu] = p10;
+            AT(iu - 1, iu - 1) = p00;
+            AT(iu - 1, iu) = p01;
+            AT(iu, iu) = p11;
+            fin[0] = tau;
+            fin[1] = e0;
+            fin[2] = app ? 1.0 : 0.0;
+          }
+        }
+      } else {
+        const int cE = k0 + 64;  // first column right of the band
+        const bool act = sc >= cE && sc <= iu;
+        // the window's rows of this lane's column, and the next window's rows, in flight
+        constexpr int NX = (PB + NW - 1) / (NW - 1);  // PB + 1 rows over the NW - 1 waves
+        double w[PB], nx[NX];
+        const int c2 = k1 + lane, cc2 = min(c2, iu), ccol = min(sc, iu);
+        if (more) {
+#pragma unroll
+          for (int q = 0; q < PB; q++) w[q] = AT(min(k0 + 2 + q, iu), ccol);
+#pragma unroll
+          for (int j = 0; j < NX; j++) nx[j] = AT(min(k1 + 2 + wave - 1 + (NW - 1) * j, iu), cc2);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // waves 5-7, which have no columns of the left strip, come first, and
+        // wave 4, which shares its SIMD with the chase, last
+        if (pn) {
+          const int first = !chase ? wave : NW == 4 ? wave - 1 : wave > 4 ? wave - 5 : wave + 2;
+          right_items(first, chase ? NW - 1 : NW, !chase);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) {
+#pragma unroll
+          for (int j = 0; j < NX; j++) {
+            const int i = wave - 1 + (NW - 1) * j;  // row k1 + 2 + i
+            if (i == 0) {
+              if (c2 >= cE) hand[par ^ 1][2][lane] = nx[j];
+            } else if (i <= PB) {
+              const int r = k1 + 2 + i;
+              win[wnext][(i - 1) * PWP + lane] = c2 >= r ? nx[j] : c2 == r - 1 ? sub[min(r, iu)] : 0.0;
+            }
+          }
+          if (__ballot(act) != 0) {
+            const SchurRf *R = rf[par];
+            // wave 0 publishes every step of its window
+            auto await = [&](int q) {
+              for (int spin = 0; spin < (1 << 24); spin++) {
+                if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(&R[q].gen, __ATOMIC_RELAXED,
+                                                                     __HIP_MEMORY_SCOPE_WORKGROUP)) == base + q + 1)
+                  break;
+                __builtin_amdgcn_s_sleep(1);
+              }
+              __asm__ volatile("" ::: "memory");
+            };
+#pragma unroll
+            for (int q = 0; q < PB; q++) {
+              if (q % 4 == 0) await(q + 3);  // four steps at a time
+              const double tau = R[q].tau, e0 = R[q].e0, e1 = R[q].e1;
+              double u2 = w[q];
+              if (__builtin_amdgcn_readfirstlane(R[q].app)) {
+                double tt = e0 * s1;
+                tt += e1 * u2;
+                tt += s0;
+                s0 -= tau * tt;
+                s1 -= (tau * e0) * tt;
+                u2 -= (tau * e1) * tt;
+              }
+              if (act) AT(k0 + q, sc) = s0;
+              s0 = s1;
+              s1 = u2;
+            }
+            if (act && sc < cE + PB) {
+              hand[par ^ 1][0][sc - k1] = s0;
+              hand[par ^ 1][1][sc - k1] = s1;
+            }
+          }
+        }
+      }
+      if (!chase) break;
+      __syncthreads();
+      base += nstep;
+      pk0 = k0;
+      pn = nstep;
+      par ^= 1;
+      wcur = wnext;
+    }
+    reload = true;
+  }
+  __syncthreads();
+  // eigenvalue 2 in Schur-diagonal order (EigenSolver::compute, EigenSolver.h:364-381)
+  if (t == 0) {
+    double f = 0.0;
+    if (n >= 3) {
+      int i = 0;
+      double re2 = 0, im2 = 0;
+      while (i < n && i <= 2) {
+        if (i == n - 1 || sub[i + 1] == 0) {
+          if (i == 2) { re2 = AT(i, i); im2 = 0; }
+          ++i;
+        } else {
+          const double p = 0.5 * (AT(i, i) - AT(i + 1, i + 1));
+          const double z = sqrt(fabs(p * p + sub[i + 1] * AT(i, i + 1)));
+          if (i == 2) { re2 = AT(i + 1, i + 1) + p; im2 = z; }
+          if (i + 1 == 2) { re2 = AT(i + 1, i + 1) + p; im2 = -z; }
+          i += 2;
+        }
+      }
+      f = (im2 == 0) ? sqrt(re2) : 0.0;
+    }
+    H.feat[angle * 14 + 13] = f;
+    H.work[angle] = work;
+  }
+#undef AT
+}
+
 // mean and range over the 4 angles, reference output order (haralick.cpp:96-143)
 __global__ void k_har_final(const HarDesc *hd, OutRef o) {
   const HarDesc H = hd[blockIdx.x];
@@ -1439,10 +2167,18 @@ void launch_haralick_hess(const HarDesc *hd, const int *order, int nimg, hipStre
   k_har_hess<<<dim3(4, nimg), 256, 0, s>>>(hd, order);
 }
 void launch_haralick_qr(const HarDesc *hd, const int *order, int nimg, hipStream_t s) {
-  // up to 1024 matrices: one 256-thread block each (all resident at once);
-  // beyond, one wavefront each
-  if (4 * nimg <= 1024) k_har_qr<256><<<dim3(4, nimg), 256, 0, s>>>(hd, order);
-  else k_har_qr<64><<<dim3(4, nimg), 64, 0, s>>>(hd, order);
+  // Up to 256 matrices every CU has at most one, and the launch lasts as long
+  // as the longest chain of steps: eight waves per matrix.  Up to 6144, four
+  // waves per matrix, two matrices per CU.  Beyond, one wave per matrix and
+  // sixteen matrices per CU: its chain is three times slower, but it does less
+  // work per step, and with that many the work counts.  Nodes of 256 x 256
+  // images (tones 10..256, mean 128), this rule's kernel against the other:
+  // 48 matrices 13.2 against 30.6 ms (four waves: 17.5), 1200 18.3 against
+  // 48.4, 2400 33.0 against 51.6, 4800 62.9 against 69.0; 7200 88.2 against
+  // 93.9, 9600 112.0 against 124.8, 19200 201 against 259.
+  if (4 * nimg <= 256) k_har_schur<8><<<dim3(4, nimg), 512, 0, s>>>(hd, order);
+  else if (4 * nimg <= 6144) k_har_schur<4><<<dim3(4, nimg), 256, 0, s>>>(hd, order);
+  else k_har_qr<<<dim3(4, nimg), 64, 0, s>>>(hd, order);
 }
 void launch_haralick_final(const HarDesc *hd, OutRef o, int nimg, hipStream_t s) {
   k_har_final<<<nimg, 64, 0, s>>>(hd, o);
