@@ -475,394 +475,586 @@ constexpr int QWP = QW + 1;  // padded LDS row of the window
 // window and strip tiles are loaded as two rows of 32 lanes per wave instruction
 static_assert(QW <= 32 && QW % 2 == 0 && QB + 2 <= QW, "QR window tiles must fit 32-lane rows");
 static_assert(QW * QWP >= 256, "the window buffer also holds the n <= 256 row sums of the Schur norm");
-constexpr int HT = 32;       // Hessenberg: columns per row-dot tile (n x HT in LDS)
-constexpr int HTP = HT + 1;  // padded tile row (bank-conflict free row reads)
-constexpr int HS = 256 / HT; // row stride of the tile-loading threads; each loads HT rows
-constexpr int HR = 16;       // rows in flight per thread in the column pass (a multiple of 4)
-
-// Reflector of column s below the diagonal (Eigen makeHouseholderInPlace),
-// x[0..rm-1] in LDS: one thread's sequential squared norm of the tail (the
-// column is strided in row-major storage, so Eigen sums it in order), then
-// the essential part element-parallel.  Writes beta and the zeros of the
-// Hessenberg form into column s, and the reflector into row s of `store`
-// (essential part, tau in column n-1) for the rows above the active block.
-// Returns tau.
-__device__ __forceinline__ double hess_reflector(gptr<double> A, int n, int s, int rm, const double *x, double *ess,
-                                                 double *sc, gptr<double> store) {
-  const int t = threadIdx.x;
-  if (t == 0) {
-    double tail = 0;
-    for (int k = 1; k < rm; k++) tail += x[k] * x[k];
-    const double c0 = x[0];
-    if (tail == 0.0) {
-      sc[0] = 0; sc[1] = c0; sc[2] = 0; sc[3] = 0;
-    } else {
-      double b = sqrt(c0 * c0 + tail);
-      if (c0 >= 0) b = -b;
-      sc[0] = (b - c0) / b;
-      sc[1] = b;
-      sc[2] = c0 - b;
-      sc[3] = 1;
-    }
-  }
-  __syncthreads();
-  const double tau = sc[0];
-  const bool nz = sc[3] != 0;
-  const double den = sc[2];
-  for (int k = 1 + t; k < rm; k += blockDim.x) {
-    const double e = nz ? x[k] / den : 0.0;
-    ess[k - 1] = e;
-    store[(long)s * n + k - 1] = e;
-  }
-  if (t == 0) {
-    A[(long)(s + 1) * n + s] = sc[1];
-    store[(long)s * n + n - 1] = tau;
-  }
-  for (int k = 1 + t; k < rm; k += blockDim.x) A[(long)(s + 1 + k) * n + s] = 0.0;  // matrixH(): Hessenberg part only
-  __syncthreads();
-  return tau;
+// The value of the neighbouring lane (lane ^ 1).
+__device__ __forceinline__ double lane_xor1(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_mov_dpp((int)b, 0xB1, 0xf, 0xf, true);  // quad_perm 1,0,3,2
+  const unsigned hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), 0xB1, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | lo);
 }
 
-// Column pass after step i (columns c = i+2..n-1, one thread per column;
-// threads left over split the rows above the dot region):
-//   upd  A = H A and A = A H of step i on rows i+1..n-1 (the rows above are
-//        deferred).  The tile pass computed H A only in LDS, so the left
-//        update is applied here to the stored values first, with the same
-//        operations: A(r,c) -= fac(r) * twold[c] (fac = tau for row i+1,
-//        tau * ess[r-i-2] below; twold = the left dot of step i), then
-//        A(r,c) -= tu[r] * ess[c-i-2], with
-//        tu[r] = tau * (row dot), Eigen's (tau * tmp) * essential^T
-//   dot  the left dot of step i+1 on the updated column, in Eigen's ColMajor
-//        GEMV order on bottom^T (general_matrix_vector_product<ColMajor>,
-//        GeneralMatrixVector.h:31-285): inner terms (rows i+3..n-1 times nx)
-//        in groups of four (g, g+o1, g+2, g+o3), added pairwise for outputs
-//        in the packet range and left to right for an odd last output;
-//        leftover terms one by one; a skipped leading term last; then
-//        + A(i+2, c) (applyHouseholderOnTheLeft's tmp += row(0)).  -> tw[c]
-__device__ __forceinline__ void hess_colpass(gptr<double> A, int n, int i, bool upd, const double *ess,
-                                             const double *tu, double tau, const double *twold, bool dot,
-                                             const double *nx, double *tw) {
-  const int t = threadIdx.x;
-  const int mB = n - i - 2;
-  if (mB <= 0) return;
-  const int k = min(8, (int)blockDim.x / mB);
-  const int cc = t % mB, sub = t / mB;
-  if (sub >= k) return;
-  const int c = i + 2 + cc;
-  const double f = upd ? ess[cc] : 0.0;
-  const double wl = upd ? twold[c] : 0.0;  // left dot of step i for this column
-  // left factor of row r (r >= i+1) of step i: tau * (1, ess)
-  auto lfac = [&](int r) { return r == i + 1 ? tau : tau * ess[r - i - 2]; };
-  const int d0 = dot ? i + 2 : n;  // first row of the dot region
-  if (upd && !(dot && k > 1 && sub == 0)) {
-    const int parts = (dot && k > 1) ? k - 1 : k, ps = (dot && k > 1) ? sub - 1 : sub;
-    const int base = i + 1;  // upd implies i >= 0
-    const int ra = base + (d0 - base) * ps / parts, rb = base + (d0 - base) * (ps + 1) / parts;
-    unsigned o = (unsigned)(ra * n + c);
-    int r = ra;
-    for (; r + HR <= rb; r += HR, o += HR * n) {
-      double v[HR];
-#pragma unroll
-      for (int q = 0; q < HR; q++) v[q] = A[o + q * n];
-#pragma unroll
-      for (int q = 0; q < HR; q++) A[o + q * n] = (v[q] - lfac(r + q) * wl) - tu[r + q] * f;
-    }
-    for (; r < rb; r++, o += n) A[o] = (A[o] - lfac(r) * wl) - tu[r] * f;
-  }
-  if (!dot || sub != 0) return;
-  const int s = i + 1;       // the step whose left dot this is
-  const int ms = n - s - 2;  // its inner terms: rows s+2..n-1
-  const bool odd_n = n & 1;
-  const long L = (long)(s + 2) * n + (s + 1);  // bottom^T(0,0) in row-major storage
-  const int skip = ((L & 1) && odd_n && ms > 0) ? 1 : 0;
-  const bool packet = cc < ((n - s - 1) & ~1);
-  const int bound = ((ms - skip) / 4) * 4 + skip;
-  const unsigned ot = (unsigned)((s + 1) * n + c);
-  double top = A[ot];
-  if (upd) { top = (top - lfac(s + 1) * wl) - tu[s + 1] * f; A[ot] = top; }
-  // rows s+2+j are addressed as A[o0 + j*n]: a uniform base and a 32-bit
-  // offset per load (one register per address)
-  const unsigned o0 = ot + n;  // row s+2: term 0
-  double x0 = 0.0;
-  if (skip) {
-    double v = A[o0];
-    if (upd) { v = (v - lfac(s + 2) * wl) - tu[s + 2] * f; A[o0] = v; }
-    x0 = v * nx[0];
-  }
-  double acc = 0.0;
-  int g = skip;
-  for (; g + HR <= bound; g += HR) {
-    double v[HR];
-#pragma unroll
-    for (int q = 0; q < HR; q++) v[q] = A[o0 + (g + q) * n];
-    if (upd) {
-#pragma unroll
-      for (int q = 0; q < HR; q++) {
-        v[q] = (v[q] - lfac(s + 2 + g + q) * wl) - tu[s + 2 + g + q] * f;
-        A[o0 + (g + q) * n] = v[q];
-      }
-    }
-#pragma unroll
-    for (int h = 0; h < HR; h += 4) {
-      const double a = v[h] * nx[g + h], p1 = v[h + 1] * nx[g + h + 1];
-      const double c2 = v[h + 2] * nx[g + h + 2], p3 = v[h + 3] * nx[g + h + 3];
-      const double b = odd_n ? p3 : p1, d = odd_n ? p1 : p3;
-      if (packet) acc = acc + ((a + b) + (c2 + d));
-      else acc = (((acc + a) + b) + c2) + d;
-    }
-  }
-  for (; g < bound; g += 4) {
-    double v[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) v[q] = A[o0 + (g + q) * n];
-    if (upd) {
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        v[q] = (v[q] - lfac(s + 2 + g + q) * wl) - tu[s + 2 + g + q] * f;
-        A[o0 + (g + q) * n] = v[q];
-      }
-    }
-    const double a = v[0] * nx[g], p1 = v[1] * nx[g + 1], c2 = v[2] * nx[g + 2], p3 = v[3] * nx[g + 3];
-    const double b = odd_n ? p3 : p1, d = odd_n ? p1 : p3;
-    if (packet) acc = acc + ((a + b) + (c2 + d));
-    else acc = (((acc + a) + b) + c2) + d;
-  }
-  for (int j = bound; j < ms; j++) {
-    double v = A[o0 + j * n];
-    if (upd) { v = (v - lfac(s + 2 + j) * wl) - tu[s + 2 + j] * f; A[o0 + j * n] = v; }
-    acc = acc + v * nx[j];
-  }
-  if (skip) acc = acc + x0;
-  tw[c] = acc + top;
-}
+constexpr int HT8 = 9;          // padded row of a wave's 32 x 8 staging tile
+constexpr int HTW = 32 * HT8;   // a wave's tile
+constexpr int HCAP = 16384;     // doubles of the matrix kept in LDS
+// all waves' LDS accesses complete; global stores may be in flight
+__device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // One block per (angle, image): HessenbergDecomposition::_compute
 // (Eigenvalues/HessenbergDecomposition.h:292-318) of Q (n x n, row-major, in
 // place).  Rows 0..i only ever receive the right reflectors of steps >= i,
-// and nothing else reads them, so step i works on the active rows
-// i+1..n-1 and the rows above are brought up to date at the end (deferred
-// pass); every element still receives the same operations in the same
-// order.  Two passes over the active block per step:
-//   tile pass    columns i+1..n-1 in HT-column LDS tiles of the active rows.
-//                The loading thread applies A = H A of step i (row i+1 -=
-//                tau*tw, bottom -= (tau*ess)*tw; tw = the left dot from the
-//                previous column pass) in LDS only (the column pass applies
-//                it again to the stored values, so the block is written once
-//                per step); the row's thread
-//                then accumulates the row dot in Eigen's RowMajor GEMV order
+// and nothing else reads them, so step i works on the active rows and columns
+// i+1..n-1 and the rows above are brought up to date by k_har_hess_rows; every element still receives the same operations in the same order.
+// Two passes over the active block per step:
+//   row pass     A = H A of step i (row i+1 -= tau*tw, the rows below -=
+//                (tau*ess)*tw; tw = the left dot of the column pass before),
+//                then the row dots in Eigen's RowMajor GEMV order
 //                (general_matrix_vector_product<RowMajor>,
 //                GeneralMatrixVector.h:289-552): even and odd terms in two
-//                lanes, the lanes added, an odd last term, + A(r, i+1).
-//   column i+1   A = A H on column i+1 (factor 1), then the reflector of
-//                step i+1 from it (kept in the co-occurrence buffer, free
-//                once Q is built, for the deferred pass).
-//   column pass  A = A H on columns i+2..n-1 fused with the left dot of
-//                step i+1 (hess_colpass).
+//                lanes, the lanes added, an odd last term, + A(r, i+1).  The
+//                two lanes are two threads: 32 rows per wave.
+//   column i+1   A = A H on column i+1 (factor 1), then the reflector of step
+//                i+1 from it (kept in the co-occurrence buffer, free once Q is
+//                built, for k_har_hess_rows).
+//   column pass  A = A H on columns i+2..n-1 and the left dot of step i+1 on
+//                them, in Eigen's ColMajor GEMV order on bottom^T
+//                (general_matrix_vector_product<ColMajor>,
+//                GeneralMatrixVector.h:31-285): inner terms (rows i+3..n-1) in
+//                groups of four (g, g+o1, g+2, g+o3), added pairwise for
+//                outputs in the packet range and left to right for an odd last
+//                output; leftover terms one by one; a skipped leading term
+//                last; then + A(i+2, c).  Two threads per column take two rows
+//                of each group.
+// The last K columns of the active rows live in LDS (K = 64, 96, then all 128
+// once 128 rows are left); the columns before them are streamed from global
+// memory, the row pass through a wave-private tile with the next 32 columns in
+// flight.  Column c of resident row r lies at c ^ (r & 31) within its 32, so
+// that neither walking rows nor walking columns conflicts.
+//
+// What bounds it: per step the latency of the two passes over the streamed
+// columns (15,000 and 19,000 cycles at 190 rows) and four barriers; with all
+// columns resident a step takes 13,000 cycles, its serial dots, the reflector's
+// norm and LDS round trips.  The kernel before, 256 threads with every column
+// streamed and the rows above updated by the same block, took 8.5 ms for one
+// 256 x 256 image's 48 matrices, now 3.3 with k_har_hess_rows, and 167 ms for
+// 19,200 (0.77 TB at the fabric's 4.6 TB/s), now 132.
 // Eigen's last step (one row below the diagonal) scales by 1 - tau with
 // tau = 0 (a one-element reflector): an exact no-op, not performed.
-// Two blocks per CU (waves_per_eu 2): the ~500 matrices in flight then fit
-// in the MALL, which serves the re-reads of later steps.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_har_hess(const HarDesc *hd, const int *order) {
-  __shared__ double tile[256 * HTP];
-  __shared__ double essb[2][256];  // reflector of step i and of step i+1
-  __shared__ double twb[2][256];   // left dots by column: current step, next step
-  __shared__ double tu[256];       // tau * right dot of the current step, by row
-  __shared__ double xcol[256];
+  __shared__ double res[HCAP];          // resident columns
+  __shared__ __align__(16) double tile[8 * HTW];  // per wave: staging; then the squares of its rows' x
+  __shared__ __align__(16) double2 twe[256];      // by column: left dot, essential element of step i
+  __shared__ __align__(16) double2 tun[256];      // by row: tau * right dot of step i, essential of step i (row pass) / i+1 (column pass)
+  __shared__ double lf[256];            // by row: left factor of step i
+  __shared__ double xc[256];            // by row: column i+1 after step i
   __shared__ double sc[4];
   const int angle = blockIdx.x;
   const HarDesc H = hd[order[blockIdx.y]];
-  const int n = *H.ng;
+  const int n = __builtin_amdgcn_readfirstlane(*H.ng);
   if (n < 2) return;
   gptr<double> A = to_global(H.Q + (long)angle * n * n);
   gptr<double> Rf = to_global(H.P + (long)angle * n * n);  // reflector store
-  const int t = threadIdx.x;
-  for (int k = t; k < n - 1; k += blockDim.x) xcol[k] = A[(long)(1 + k) * n];
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const bool odd_n = n & 1;
+  int K = 0, cK = n, r0 = 0;  // resident: columns cK.., rows r0.. (row r at (r - r0) * K)
+#define AT(r, c) A[(unsigned)((r) * n + (c))]
+#define RES(r, c) res[((r) - r0) * K + (((c) - cK) ^ ((r) & 31))]
+
+  // Reflector of column s below the diagonal (Eigen makeHouseholderInPlace)
+  // from xc[s+1..n-1] and the squares of xc (row base + k at tile row k): the
+  // column is strided in row-major storage, so Eigen sums the tail in order.
+  // Writes beta and the zeros of the Hessenberg form into column s, the
+  // reflector into row s of Rf (essential part, tau in column n-1) and tun.y.
+  auto reflector = [&](int s, int base) {
+    if (wave == 0) {
+      const double c0 = xc[s + 1];
+      double tail = 0;
+      for (int w = 0; w * 32 < n - base; w++) {
+        const int k0 = s + 2 - base - 32 * w, k1 = min(32, n - base - 32 * w);  // tile rows k0..k1-1 of this wave
+        const double2 *q = (const double2 *)(tile + w * HTW);
+        double2 v[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) v[k] = q[k];
+        if (k0 <= 0 && k1 == 32) {
+#pragma unroll
+          for (int k = 0; k < 16; k++) {
+            tail += v[k].x;
+            tail += v[k].y;
+          }
+        } else {
+#pragma unroll
+          for (int k = 0; k < 16; k++) {
+            if (2 * k >= k0 && 2 * k < k1) tail += v[k].x;
+            if (2 * k + 1 >= k0 && 2 * k + 1 < k1) tail += v[k].y;
+          }
+        }
+      }
+      double tau = 0, beta = c0, den = 0, nz = 0;
+      if (tail != 0.0) {
+        double b = sqrt(c0 * c0 + tail);
+        if (c0 >= 0) b = -b;
+        tau = (b - c0) / b;
+        beta = b;
+        den = c0 - b;
+        nz = 1;
+      }
+      if (lane == 0) {
+        sc[0] = tau;
+        sc[1] = den;
+        sc[2] = nz;
+        AT(s + 1, s) = beta;
+        Rf[(unsigned)(s * n + n - 1)] = tau;
+      }
+    }
+    lds_barrier();
+    const double den = sc[1];
+    const int r = s + 2 + t;
+    if (r < n) {
+      const double e = sc[2] != 0.0 ? xc[r] / den : 0.0;
+      tun[r].y = e;
+      Rf[(unsigned)(s * n + t)] = e;
+      AT(r, s) = 0.0;  // matrixH(): Hessenberg part only
+    }
+    return sc[0];
+  };
+
+  // the resident columns back to global memory, rows from r1 on
+  auto flush = [&](int r1) {
+    for (int r = r1 + wave; r < n; r += 8)
+      for (int c = max(cK, r1) + lane; c < n; c += 64) AT(r, c) = RES(r, c);
+  };
+  // residency for rows r1..n-1
+  auto reside = [&](int r1) {
+    const int R = n - r1;
+    K = R <= 128 ? 128 : R <= 170 ? 96 : 64;
+    cK = max(n - K, 0);
+    r0 = r1;
+    for (int ra = r1 + wave; ra < n; ra += 32) {
+      double v[4][2];
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) v[k][j] = AT(min(ra + 8 * k, n - 1), min(cK + lane + 64 * j, n - 1));
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          if (ra + 8 * k < n && cK + lane + 64 * j < n && lane + 64 * j < K) RES(ra + 8 * k, cK + lane + 64 * j) = v[k][j];
+    }
+  };
+
+  // Column pass after step i (i = -1: the left dot of step 0 alone, with
+  // zero factors).
+  auto colpass = [&](int i) {
+    const int s = i + 1;                   // the step whose left dot this is
+    const int ms = n - s - 2;              // its inner terms: rows s+2..n-1
+    const int ns = max(cK - (i + 2), 0);   // streamed columns, whole waves ending at cK
+    const int nsw = (ns + 31) / 32;
+    const bool stream = wave < nsw;
+    const int c = stream ? cK - 32 * (nsw - wave) + (lane >> 1) : max(cK, i + 2) + 32 * (wave - nsw) + (lane >> 1);
+    const int h = lane & 1;
+    const bool act = c >= i + 2 && c < n;
+    if (__ballot(act) == 0) return;
+    const int cs = min(max(c, i + 2), n - 1);  // in range; lanes without a column compute along
+    const double2 own = twe[cs];
+    const double wl = i >= 0 ? own.x : 0.0, f = i >= 0 ? own.y : 0.0;
+    const bool packet = cs - (i + 2) < ((n - s - 1) & ~1);
+    const bool np = __ballot(!packet) != 0;
+    const long L = (long)(s + 2) * n + (s + 1);  // bottom^T(0,0) in row-major storage
+    const int skip = ((L & 1) && odd_n && ms > 0) ? 1 : 0;
+    const int bound = ms > 0 ? ((ms - skip) / 4) * 4 + skip : 0;
+    double acc = 0.0, top = 0.0, x0 = 0.0;
+    const int ro = s + 2;  // row of inner term 0
+    auto run = [&](auto st) __attribute__((always_inline)) {
+      constexpr bool S = decltype(st)::value;
+      // one row: A = H A (streamed; the row pass has done it for resident
+      // columns), A = A H; stored
+      auto upd = [&](int r, double v, double tu) {
+        if (S) v = v - lf[r] * wl;
+        return v - tu * f;
+      };
+      auto get = [&](int r) { return S ? (double)AT(r, cs) : RES(r, cs); };
+      auto put = [&](int r, double v) {
+        if (!act) return;
+        if (S) AT(r, cs) = v;
+        else RES(r, cs) = v;
+      };
+      // both lanes of a pair compute the rows outside the groups; lane 0 stores
+      if (i >= 0) {
+        const double v = upd(i + 1, get(i + 1), tun[i + 1].x);  // this row leaves the active block
+        if (act && h == 0) AT(i + 1, cs) = v;
+      }
+      top = get(s + 1);
+      if (i >= 0) {
+        top = upd(s + 1, top, tun[s + 1].x);
+        if (h == 0) put(s + 1, top);
+      }
+      if (skip) {
+        const double2 q = tun[ro];
+        const double v = upd(ro, get(ro), q.x);
+        if (h == 0) put(ro, v);
+        x0 = v * q.y;
+      }
+      auto group = [&](const double *p) {  // the pair's four products in Eigen's order
+        if (np) {  // a wave with the odd last column
+          const double q0 = lane_xor1(p[0]), q1 = lane_xor1(p[1]);
+          const double sh = p[0] + (odd_n ? q1 : p[1]);
+          const double sp = acc + (sh + lane_xor1(sh));
+          // lane 0's view: its own first pair, the other lane's second pair
+          const double a = p[0], b = odd_n ? q1 : p[1], c2 = q0, d = odd_n ? p[1] : q1;
+          const double sl = (((acc + a) + b) + c2) + d;
+          acc = packet ? sp : sl;
+        } else {
+          const double sh = p[0] + (odd_n ? lane_xor1(p[1]) : p[1]);
+          acc = acc + (sh + lane_xor1(sh));
+        }
+      };
+      int g = skip;
+      for (; g + 16 <= bound; g += 16) {
+        double v[8], p[8];
+        double2 q[8];
+        const int rr = ro + g + 2 * h;
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = get(rr + (k >> 1) * 4 + (k & 1));
+#pragma unroll
+        for (int k = 0; k < 8; k++) q[k] = tun[rr + (k >> 1) * 4 + (k & 1)];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+          v[k] = upd(rr + (k >> 1) * 4 + (k & 1), v[k], q[k].x);
+          p[k] = v[k] * q[k].y;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++) put(rr + (k >> 1) * 4 + (k & 1), v[k]);
+#pragma unroll
+        for (int k = 0; k < 8; k += 2) group(p + k);
+      }
+      for (; g < bound; g += 4) {
+        double v[2], p[2];
+        const int rr = ro + g + 2 * h;
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+          const double2 q = tun[rr + k];
+          v[k] = upd(rr + k, get(rr + k), q.x);
+          p[k] = v[k] * q.y;
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) put(rr + k, v[k]);
+        group(p);
+      }
+      for (int j = bound; j < ms; j++) {
+        const double2 q = tun[ro + j];
+        const double v = upd(ro + j, get(ro + j), q.x);
+        if (h == 0) put(ro + j, v);
+        acc = acc + v * q.y;
+      }
+    };
+    if (stream) run(std::true_type());
+    else run(std::false_type());
+    if (skip) acc = acc + x0;
+    if (act && h == 0) twe[c] = double2{acc + top, tun[c].y};
+  };
+
+  // step 0's reflector and left dot
+  for (int r = t; r < 256; r += 512) tun[r] = double2{0.0, 0.0};
+  for (int r = t; r < n; r += 512) {
+    const double x = AT(r, 0);
+    xc[r] = x;
+    if (r >= 1) tile[((r - 1) >> 5) * HTW + ((r - 1) & 31)] = x * x;
+    lf[r] = 0.0;
+  }
+  reside(1);
   __syncthreads();
-  double tau = hess_reflector(A, n, 0, n - 1, xcol, essb[0], sc, Rf);
-  if (n - 1 >= 2) hess_colpass(A, n, -1, false, nullptr, nullptr, 0.0, nullptr, true, essb[0], twb[0]);
+  double tau = reflector(0, 1);
   __syncthreads();
-  int pp = 0;
-  const int lc = t % HT, lr = t / HT;
+  colpass(-1);
+  __syncthreads();
   for (int i = 0; i + 2 < n; ++i) {
     const int rem = n - i - 1, m = rem - 1, asz = m & ~1;
-    const int rb = i + 1;  // first active row; tile row k holds row rb + k
-    const double *ess = essb[pp];
-    const double *tw = twb[pp];
-    double rv[HT];
-    auto load = [&](int ct) {
-      if (ct + lc < rem) {
-        int r0 = lr;
-        asm volatile("" : "+v"(r0));  // per-row values are formed at use, not hoisted out of the column loop
-        const int c = i + 1 + ct + lc;
-        // rows past the end re-read row n-1: branch-free, so all HT loads issue back to back
-#pragma unroll
-        for (int q = 0; q < HT; q++) rv[q] = A[(unsigned)(min(rb + r0 + HS * q, n - 1) * n + c)];
-      }
-    };
-    double l0 = 0.0, l1 = 0.0, tl = 0.0, col0 = 0.0;
-    load(0);
-    for (int ct = 0; ct < rem; ct += HT) {
-      const int ncol = (rem - ct < HT) ? rem - ct : HT;
-      if (lc < ncol) {
-        const int c = i + 1 + ct + lc;
-        const double w = tw[c];
-        int r0 = lr;
-        asm volatile("" : "+v"(r0));
-        double *tl0 = tile + (r0 * HTP + lc);
-        // every LDS operand is read before the arithmetic (clamped indices,
-        // unused where clamped), so the reads are in flight together rather
-        // than one round trip per row
-        double e[HT];
-#pragma unroll
-        for (int q = 0; q < HT; q++) e[q] = ess[min(max(rb + r0 + HS * q - i - 2, 0), 255)];
-#pragma unroll
-        for (int q = 0; q < HT; q++) {
-          const int r = rb + r0 + HS * q;
-          const double fac = (r == i + 1) ? tau : tau * e[q];
-          tl0[HS * q * HTP] = (r < n) ? rv[q] - fac * w : rv[q];  // rows >= n are never read
-        }
-      }
+    const int Kn = rem <= 128 ? 128 : rem <= 170 ? 96 : 64;
+    if (Kn != K) {  // fewer rows: more resident columns
+      flush(i + 1);
       __syncthreads();
-      if (ct + HT < rem) load(ct + HT);  // next tile's loads in flight during the row sums
-      if (t < rem) {
-        const double *tr = tile + t * HTP;
+      reside(i + 1);
+      __syncthreads();
+    }
+    // ---- row pass: row r, lane parity par (terms j of that parity; parity 1 also column i+1)
+    if (i + 1 + 32 * wave < n) {
+      const int rl = lane >> 1, par = lane & 1;
+      const int r = i + 1 + 32 * wave + rl, rc = min(r, n - 1);
+      const double fac = rc == i + 1 ? tau : tau * tun[rc].y;
+      if (par == 0 && r < n) lf[r] = fac;
+      double l = 0.0, col0 = 0.0;
+      const int U = cK - (i + 1);  // streamed columns, column i+1 first
+      if (U > 0) {
+        double *tl = tile + wave * HTW;
+        const int lr = lane >> 3, lc = lane & 7;
+        // 32 rows x 32 columns from column i+1+u0: one lane offset per eight
+        // rows; the columns past U are resident ones, so still in the matrix
+        unsigned go[4];
 #pragma unroll
-        for (int h = 0; h < HT; h += HT / 2) {  // half a tile row at a time: its LDS reads in flight together
-          double tv[HT / 2], te[HT / 2];
+        for (int k = 0; k < 4; k++) go[k] = (unsigned)(min(i + 1 + 32 * wave + 8 * k + lr, n - 1) * n + i + 1 + lc);
+        auto load = [&](int u0, double *d) {
+          gptr<const double> g = A + u0;
 #pragma unroll
-          for (int u = 0; u < HT / 2; u++) {
-            tv[u] = tr[h + u];
-            te[u] = ess[min(max(ct + h + u - 1, 0), 255)];
-          }
+          for (int q = 0; q < 4; q++)
 #pragma unroll
-          for (int u = 0; u < HT / 2; u++) {
-            const int cc = h + u;
-            if (cc < ncol) {
-              const int j = ct + cc - 1;  // ct is even: j is even for odd cc
-              const double v = tv[u];
-              if (j < 0) col0 = v;
-              else if (j < asz) {
-                if (cc & 1) l0 = l0 + v * te[u];
-                else l1 = l1 + v * te[u];
-              } else tl = v * te[u];
+            for (int k = 0; k < 4; k++) d[4 * q + k] = (g + 8 * q)[go[k]];
+        };
+        double *tw = tl + lr * HT8 + lc;
+        const double *tr = tl + rl * HT8 + 1 - par;
+        const double2 *ob = twe + i + 2 - par;
+        double v[16], nx[16];
+        load(0, v);
+        for (int u0 = 0; u0 < U; u0 += 32) {
+          if (u0 + 32 < U) load(u0 + 32, nx);
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const int ub = u0 + 8 * q;
+            if (ub < U) {
+              wave_sync();
+#pragma unroll
+              for (int k = 0; k < 4; k++) tw[8 * k * HT8] = v[4 * q + k];
+              wave_sync();
+              double a[4];
+              double2 o[4];
+#pragma unroll
+              for (int x = 0; x < 4; x++) {
+                a[x] = tr[2 * x];
+                o[x] = ob[ub + 2 * x];
+              }
+              if (ub > 0 && ub + 8 <= U) {
+#pragma unroll
+                for (int x = 0; x < 4; x++) l = l + (a[x] - fac * o[x].x) * o[x].y;
+              } else {  // column i+1, which is no term; columns past U
+#pragma unroll
+                for (int x = 0; x < 4; x++) {
+                  const double w = a[x] - fac * o[x].x;
+                  const double ln = l + w * o[x].y;
+                  const int u = ub + 2 * x + 1 - par;
+                  if (x == 0) col0 = (ub == 0 && par) ? w : col0;
+                  l = (u < U && (x > 0 || ub > 0 || !par)) ? ln : l;
+                }
+              }
             }
           }
+#pragma unroll
+          for (int k = 0; k < 16; k++) v[k] = nx[k];
+        }
+      } else if (par) {
+        col0 = RES(rc, i + 1) - fac * twe[i + 1].x;
+      }
+      // resident columns: terms j0.. of this parity
+      const int j0 = max(U - 1, 0);
+      int j = j0 + ((j0 ^ par) & 1);
+      for (; j + 14 < asz; j += 16) {
+        double a[8];
+        double2 o[8];
+#pragma unroll
+        for (int x = 0; x < 8; x++) a[x] = RES(rc, i + 2 + j + 2 * x);
+#pragma unroll
+        for (int x = 0; x < 8; x++) o[x] = twe[i + 2 + j + 2 * x];
+#pragma unroll
+        for (int x = 0; x < 8; x++) {
+          a[x] = a[x] - fac * o[x].x;
+          l = l + a[x] * o[x].y;
+        }
+        if (r < n)
+#pragma unroll
+          for (int x = 0; x < 8; x++) RES(rc, i + 2 + j + 2 * x) = a[x];
+      }
+      {
+        double a[8];
+        double2 o[8];
+#pragma unroll
+        for (int x = 0; x < 8; x++) {
+          const int c = min(i + 2 + j + 2 * x, n - 1);
+          a[x] = RES(rc, c);
+          o[x] = twe[c];
+        }
+#pragma unroll
+        for (int x = 0; x < 8; x++) {
+          a[x] = a[x] - fac * o[x].x;
+          const double ln = l + a[x] * o[x].y;
+          l = j + 2 * x < asz ? ln : l;
+          if (r < n && j + 2 * x < asz) RES(rc, i + 2 + j + 2 * x) = a[x];
         }
       }
-      __syncthreads();
+      double last = 0.0;
+      if ((m & 1) && par == 0) {  // the odd last term, column n-1
+        const double2 o = twe[n - 1];
+        const double v = RES(rc, n - 1) - fac * o.x;
+        if (r < n) RES(rc, n - 1) = v;
+        last = v * o.y;
+      }
+      const double l1 = lane_xor1(l), cc0 = lane_xor1(col0);
+      wave_sync();  // the tile's reads are done: it now holds the squares
+      if (par == 0 && r < n) {
+        double tmp = 0.0;
+        if (asz > 0) tmp = tmp + (l + l1);
+        if (m & 1) tmp = tmp + last;
+        const double tt = (0.0 + tmp) + cc0;
+        const double tuv = tau * tt;
+        tun[r].x = tuv;
+        const double x = cc0 - tuv;  // column i+1 of A = A H: (tau*tmp) * 1
+        xc[r] = x;
+        tile[wave * HTW + rl] = x * x;
+        if (r == i + 1) AT(r, i + 1) = x;
+      }
     }
-    if (t < rem) {
-      const int r = rb + t;
-      double tmp = 0.0;
-      if (asz > 0) tmp = tmp + (l0 + l1);
-      if (m & 1) tmp = tmp + tl;
-      const double tt = (0.0 + tmp) + col0;
-      const double tuv = tau * tt;
-      tu[r] = tuv;
-      const double v = col0 - tuv;  // column i+1 of A = A H: (tau*tmp) * 1
-      A[(long)r * n + i + 1] = v;
-      if (r >= i + 2) xcol[r - i - 2] = v;
-    }
-    __syncthreads();
-    const double tau_n = hess_reflector(A, n, i + 1, m, xcol, essb[pp ^ 1], sc, Rf);
-    hess_colpass(A, n, i, true, ess, tu, tau, tw, m >= 2, essb[pp ^ 1], twb[pp ^ 1]);
-    __syncthreads();
-    pp ^= 1;
+    lds_barrier();
+    const double tau_n = reflector(i + 1, i + 1);
+    lds_barrier();
+    colpass(i);
+    if (cK > i + 2) __syncthreads();  // streamed columns were stored
+    else lds_barrier();
     tau = tau_n;
   }
-  // Deferred pass: row r (r <= n-3) receives the right reflectors of steps
-  // r..n-3 in order, exactly as the column passes would have applied them:
-  // row dot in the RowMajor GEMV order (lanes l0 / l1 of one row are the
-  // two threads of a pair), tu = tau * (dot + A(r, i+1)), A(r, i+1) -= tu,
-  // A(r, c) -= tu * ess[c-i-2].  Chunks of rows r0.. are staged in LDS with
-  // their live columns r0+1..n-1 only, as many rows as the tile buffer
-  // holds (at most 128); reflectors stream through a two-deep register
-  // pipeline (one element per thread) into two LDS buffers.
-  double *rows = tile;
-  const int lane = t & 63, wv = t >> 6;
-  for (int r0 = 0; r0 < n - 2;) {
-    const int cb = r0 + 1, wd = n - cb, wp = wd | 1;  // staged columns cb..n-1, odd row stride
-    int nr = (256 * HTP) / wp;
-    if (nr > 128) nr = 128;
-    if (nr > n - 2 - r0) nr = n - 2 - r0;
-    for (int rr = wv; rr < nr; rr += 4)
-      for (int c = lane; c < wd; c += 64) rows[rr * wp + c] = A[(long)(r0 + rr) * n + cb + c];
-    // reflector r0 in LDS buffer 0; reflectors r0+1..r0+4 in flight in a
-    // ring of four register slots, slot k holding reflector r0+s with
-    // s = k (mod 4): the step loop is unrolled by four so that every slot
-    // is named statically and consumed four steps after its load
-    auto fetch = [&](int i, double &e, double &tv) {
-      e = 0.0;
-      tv = 0.0;
-      if (i <= n - 3) {
-        if (t < n - i - 2) e = Rf[(long)i * n + t];
-        tv = Rf[(long)i * n + n - 1];
-      }
-    };
-    double e0, t0, e1, t1, e2, t2, e3, t3;
-    fetch(r0, e0, t0);
-    essb[0][t] = e0;
-    double ti = t0;
-    fetch(r0 + 1, e1, t1);
-    fetch(r0 + 2, e2, t2);
-    fetch(r0 + 3, e3, t3);
-    fetch(r0 + 4, e0, t0);
-    __syncthreads();
-    // step i = r0 + s; afterwards reflector i+1 (slot (s+1) mod 4) goes to
-    // LDS and that slot is refilled with reflector i+5
-    auto step = [&](int s, double &en, double &tn) {
-      const int i = r0 + s;
-      const double *eb = essb[s & 1];
-      const int m = n - i - 2, asz = m & ~1;
-      const int na = (i + 1 - r0 < nr) ? i + 1 - r0 : nr;  // rows r0..i of the chunk take part
-      if (t < 2 * na) {
-        const int rr = t >> 1, par = t & 1;
-        const double *row = rows + rr * wp + (i + 2 - cb);
-        double l = 0.0;
-#pragma unroll 8
-        for (int j = par; j < asz; j += 2) l = l + row[j] * eb[j];
-        const double l1 = __shfl_xor(l, 1);
-        if (par == 0) {
-          double tmp = 0.0;
-          if (asz > 0) tmp = tmp + (l + l1);
-          if (m & 1) tmp = tmp + row[m - 1] * eb[m - 1];
-          tu[rr] = ti * ((0.0 + tmp) + rows[rr * wp + (i + 1 - cb)]);
-        }
-      }
-      __syncthreads();
-      // column c (c = 0: column i+1, factor 1) of rows wv, wv+4, ..: the
-      // rows' entries are independent, so their LDS accesses overlap
-      for (int c = lane; c <= m; c += 64) {
-        double *col = rows + (i + 1 - cb) + c;
-        if (c == 0) {
-#pragma unroll 4
-          for (int rr = wv; rr < na; rr += 4) col[rr * wp] = col[rr * wp] - tu[rr];
-        } else {
-          const double e = eb[c - 1];
-#pragma unroll 4
-          for (int rr = wv; rr < na; rr += 4) col[rr * wp] = col[rr * wp] - tu[rr] * e;
-        }
-      }
-      essb[(s + 1) & 1][t] = en;
-      ti = tn;
-      fetch(i + 5, en, tn);
-      __syncthreads();
-    };
-    for (int s = 0; r0 + s <= n - 3; s += 4) {
-      step(s, e1, t1);
-      if (r0 + s + 1 > n - 3) break;
-      step(s + 1, e2, t2);
-      if (r0 + s + 2 > n - 3) break;
-      step(s + 2, e3, t3);
-      if (r0 + s + 3 > n - 3) break;
-      step(s + 3, e0, t0);
-    }
-    for (int rr = wv; rr < nr; rr += 4)
-      for (int c = lane; c < wd; c += 64) A[(long)(r0 + rr) * n + cb + c] = rows[rr * wp + c];
-    __syncthreads();
-    r0 += nr;
+  flush(n - 1);
+}
+#undef RES
+#undef AT
+
+// The rows above the active block, after k_har_hess: row r (r <= n-3) receives
+// the right reflectors of steps r..n-3 in order, with the operations of the
+// reduction's own rows: the row dot in the RowMajor GEMV order, tu = tau * (dot
+// + A(r, i+1)), A(r, i+1) -= tu, A(r, c) -= tu * ess[c-i-2].  Rows are
+// independent, so a wave takes 32 of them on its own, two lanes per row (the
+// even and the odd columns: the two lanes of the GEMV, which swap roles every
+// step), staged in LDS with their live columns; the update of step i-1 and the
+// dot of step i share one pass over the row.  As the last part of k_har_hess,
+// with 68 rows at a time and two block barriers per step, this took a third
+// of that kernel: 3.2M of 9.9M cycles for 238 tones.
+constexpr int RWS = 32;  // rows per wave
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1)))
+k_har_hess_rows(const HarDesc *hd, const int *order) {
+  __shared__ double rows[RWS * 257];
+  __shared__ double E[2][2][128];  // essential part of step s by column: [s & 1][c & 1][c >> 1]
+  const int angle = blockIdx.x;
+  const HarDesc H = hd[order[blockIdx.y]];
+  const int n = __builtin_amdgcn_readfirstlane(*H.ng);
+  const int r0 = RWS * blockIdx.z;
+  if (r0 >= n - 2) return;
+  gptr<double> A = to_global(H.Q + (long)angle * n * n);
+  gptr<const double> Rf = to_global((const double *)H.P + (long)angle * n * n);
+  const int lane = threadIdx.x, rr = lane >> 1, cp = lane & 1;
+  const int nr = min(RWS, n - 2 - r0), cb = r0 + 1, wd = n - cb, wp = wd | 1;
+  for (int ra = 0; ra < nr; ra += 4) {
+    double v[4][4];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int k = 0; k < 4; k++) v[q][k] = A[(unsigned)((r0 + min(ra + q, nr - 1)) * n + cb + min(lane + 64 * k, wd - 1))];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        if (ra + q < nr && lane + 64 * k < wd) rows[(ra + q) * wp + lane + 64 * k] = v[q][k];
   }
+  double *row = rows + rr * wp - cb;  // row[c]; rows past nr compute along in their own space
+  auto fetch = [&](int i, double *e, double &tau) {
+    const int m = n - i - 2;
+#pragma unroll
+    for (int k = 0; k < 4; k++) e[k] = Rf[(unsigned)(i * n + min(lane + 64 * k, max(m - 1, 0)))];
+    tau = Rf[(unsigned)(i * n + n - 1)];
+  };
+  auto deposit = [&](int i, const double *e) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int c = i + 2 + lane + 64 * k;
+      if (c < n) E[i & 1][c & 1][c >> 1] = e[k];
+    }
+  };
+  double tau, tu = 0;
+  {
+    double e[4];
+    fetch(r0, e, tau);
+    deposit(r0, e);
+  }
+  wave_sync();
+  // pass i: the update of step i-1 and the dot of step i (i = n-2: the update
+  // alone).  SEL: some rows have not started yet and keep their values.
+  auto pass = [&](int i, auto sel) __attribute__((always_inline)) {
+    constexpr bool SEL = decltype(sel)::value;
+    const bool begun = r0 + rr < i;
+    const double *ep = E[(i - 1) & 1][cp], *ec = E[i & 1][cp];
+    double en[4], tau_n = 0;
+    if (i + 1 <= n - 3) fetch(i + 1, en, tau_n);
+    auto upd = [&](double v, double e) {
+      const double w = v - tu * e;
+      return SEL ? (begun ? w : v) : w;
+    };
+    if (begun && cp == (i & 1)) row[i] = row[i] - tu;
+    double col0 = 0;
+    if (cp == ((i + 1) & 1)) {
+      col0 = upd(row[i + 1], ep[(i + 1) >> 1]);
+      row[i + 1] = col0;
+    }
+    if (i > n - 3) return;
+    double l = 0;
+    int c = i + 2 + ((i + 2 - cp) & 1);                    // this lane's first column
+    const int nb = max(n - 2 - (i + 3) + 2, 0) / 2 / 8;    // full batches of eight columns of either parity
+    struct Batch { double v[8], p[8], q[8]; };
+    auto load = [&](int c, Batch &b) {
+#pragma unroll
+      for (int x = 0; x < 8; x++) b.v[x] = row[c + 2 * x];
+#pragma unroll
+      for (int x = 0; x < 8; x++) b.p[x] = ep[(c >> 1) + x];
+#pragma unroll
+      for (int x = 0; x < 8; x++) b.q[x] = ec[(c >> 1) + x];
+    };
+    auto work = [&](int c, Batch &b) {
+#pragma unroll
+      for (int x = 0; x < 8; x++) {
+        b.v[x] = upd(b.v[x], b.p[x]);
+        l = l + b.v[x] * b.q[x];
+      }
+#pragma unroll
+      for (int x = 0; x < 8; x++) row[c + 2 * x] = b.v[x];
+    };
+    Batch a, b;
+    if (nb > 0) load(c, a);
+    for (int k = 0; k < nb; k += 2) {  // the next batch's reads in flight during this one's arithmetic
+      if (k + 1 < nb) load(c + 16, b);
+      work(c, a);
+      c += 16;
+      if (k + 1 < nb) {
+        if (k + 2 < nb) load(c + 16, a);
+        work(c, b);
+        c += 16;
+      }
+    }
+    // the rest up to column n-2 (at most eight per lane), then column n-1
+#pragma unroll
+    for (int x = 0; x < 8; x++) {
+      const int cx = min(c + 2 * x, n - 1);
+      a.v[x] = row[cx];
+      a.p[x] = ep[cx >> 1];
+      a.q[x] = ec[cx >> 1];
+    }
+    const bool own = cp == ((n - 1) & 1);
+    double vl = row[n - 1];
+    const double pl = ep[(n - 1) >> 1], ql = ec[(n - 1) >> 1];
+#pragma unroll
+    for (int x = 0; x < 8; x++) {
+      const bool in = c + 2 * x <= n - 2;
+      const double w = upd(a.v[x], a.p[x]);
+      const double ln = l + w * a.q[x];
+      l = in ? ln : l;
+      if (in) row[c + 2 * x] = w;
+    }
+    double tl = 0;
+    if (own) {
+      vl = upd(vl, pl);
+      row[n - 1] = vl;
+      tl = vl * ql;
+    }
+    const bool odd_m = (n - i - 2) & 1;  // an odd last term stays apart
+    if (own && !odd_m) l = l + tl;
+    const double lx = lane_xor1(l), tx = lane_xor1(tl), cx = lane_xor1(col0);
+    double tmp = 0.0 + (l + lx);
+    if (odd_m) tmp = tmp + (own ? tl : tx);
+    tu = tau * ((0.0 + tmp) + (cp == ((i + 1) & 1) ? col0 : cx));
+    if (i + 1 <= n - 3) deposit(i + 1, en);
+    tau = tau_n;
+    wave_sync();
+  };
+  int i = r0;
+  for (; i <= n - 2 && i < r0 + RWS; i++) pass(i, std::true_type());
+  for (; i <= n - 2; i++) pass(i, std::false_type());
+  wave_sync();
+  for (int ra = 0; ra < nr; ra++)
+    for (int c = lane; c < wd; c += 64) A[(unsigned)((r0 + ra) * n + cb + c)] = rows[ra * wp + c];
 }
 
 // Francis QR on the Hessenberg matrix left in H.Q by k_har_hess, for launches
@@ -2164,7 +2356,8 @@ void launch_haralick_order(const int *ng, int nimg, int *order, hipStream_t s) {
   k_har_order<<<1, 320, 0, s>>>(ng, nimg, order);
 }
 void launch_haralick_hess(const HarDesc *hd, const int *order, int nimg, hipStream_t s) {
-  k_har_hess<<<dim3(4, nimg), 256, 0, s>>>(hd, order);
+  k_har_hess<<<dim3(4, nimg), 512, 0, s>>>(hd, order);
+  k_har_hess_rows<<<dim3(4, nimg, (256 - 2 + RWS - 1) / RWS), 64, 0, s>>>(hd, order);
 }
 void launch_haralick_qr(const HarDesc *hd, const int *order, int nimg, hipStream_t s) {
   // Up to 256 matrices every CU has at most one, and the launch lasts as long
