@@ -1,0 +1,67 @@
+"""GPU: object features and edge medians where their blocks of pixels meet.
+
+Connected components are labelled in strips of up to 16,384 pixels and joined
+across the strips' first rows; roots are ranked and areas added in blocks of
+4,096 pixels; medians are selected from the bins that hold the middle ranks.
+Planes just below, at and above these sizes, with components that wind through
+many strips, against the oracle: counts exactly, the rest to 1e-9."""
+import numpy as np
+import pytest
+
+import wndcharm
+from helpers import ALG_NAMES, orc_algorithm
+
+pytestmark = pytest.mark.gpu
+
+OBJ_EXACT = list(range(0, 14)) + [15, 16, 17] + list(range(18, 29)) + [30, 31, 33]
+EDGE_EXACT = list(range(14)) + list(range(17, 25)) + [26]  # not the direction's mean, median and variance (atan2)
+
+
+def check(alg, img, exact):
+    got = np.asarray(wndcharm.FeatureAlgorithm(alg).execute(img))
+    want = orc_algorithm(ALG_NAMES.index(alg), np.asarray(img, np.float64))
+    assert np.array_equal(got[exact], want[exact]), (alg, img.shape, got, want)
+    assert np.allclose(got, want, rtol=1e-9, atol=1e-9), (alg, img.shape, got, want)
+
+
+def winding(h, w, seed):
+    """bands that meander down the plane, combs that join them, and specks"""
+    rng = np.random.default_rng(seed)
+    y, x = np.mgrid[0:h, 0:w]
+    a = (np.sin(x / 3.0 + 2 * np.sin(y / 9.0)) > 0.3) | ((x + y) % 23 == 0) | ((x - y) % 31 == 0)
+    a = a ^ (rng.random((h, w)) < 0.02)
+    return np.where(a, 200.0, 40.0) + rng.integers(0, 9, (h, w))
+
+
+@pytest.mark.parametrize('shape', [(16, 16), (64, 64), (64, 63), (65, 64), (16, 1024), (17, 1024), (128, 128), (127, 129),
+                                   (129, 128), (33, 4096), (4096, 17), (300, 301)])
+def test_objects_across_strips(shape):
+    print('objects', shape, flush=True)
+    for alg in ('Otsu Object Features', 'Inverse-Otsu Object Features'):
+        check(alg, winding(*shape, seed=sum(shape)), OBJ_EXACT)
+
+
+def test_objects_one_component_through_every_strip():
+    """a serpentine one pixel wide, its two halves joined only in the last row"""
+    img = np.zeros((260, 200))
+    img[:, 3] = img[:, 190] = 100.0
+    img[259, 3:191] = 100.0
+    img[::4, 10:180] = 100.0
+    img[2::8, 100] = 100.0
+    print('objects serpentine', flush=True)
+    check('Otsu Object Features', img, OBJ_EXACT)
+    check('Inverse-Otsu Object Features', img, OBJ_EXACT)
+
+
+@pytest.mark.parametrize('shape', [(16, 17), (64, 128), (91, 90), (91, 91), (64, 129), (256, 257)])
+@pytest.mark.parametrize('kind', ['noise', 'flat', 'two', 'ramp', 'skewed'])
+def test_edge_medians(shape, kind):
+    """even and odd pixel counts; all values equal; two values whose middle
+    ranks straddle a gap; a plane whose values crowd one bin"""
+    h, w = shape
+    rng = np.random.default_rng(h * w)
+    img = {'noise': rng.integers(0, 4096, shape).astype(float), 'flat': np.full(shape, 5.0),
+           'two': np.where(np.mgrid[0:h, 0:w][0] < h // 2, 1.0, 7.0),
+           'ramp': np.mgrid[0:h, 0:w][1] * 3.0, 'skewed': np.exp(rng.normal(0, 6, shape))}[kind]
+    print('edge', shape, kind, flush=True)
+    check('Edge Features', img, EDGE_EXACT)

@@ -1355,27 +1355,24 @@ static int build_batch(wndgpu_ctx *c, const wndgpu_plan *plan, const Batch &B, A
           md[2 * k + 1] = dr[k];
         }
         std::vector<uint64_t *> sb(2 * ne);
-        std::vector<long> cap(2 * ne);
-        for (int k = 0; k < 2 * ne; k++) {
-          cap[k] = (long)md[k].h * md[k].w;
-          sb[k] = A.dalloc_n<uint64_t>(2 * (size_t)cap[k]);
-        }
+        for (int k = 0; k < 2 * ne; k++) sb[k] = A.dalloc_n<uint64_t>((size_t)md[k].h * md[k].w);
         Img *mgd = A.stage(mg), *drd = A.stage(dr), *mdd = A.stage(md);
         uint64_t **sbd = A.stage(sb);
-        long *capd = A.stage(cap);
         Stats *st2 = A.dalloc_n<Stats>(2 * ne);
         double *med = A.dalloc_n<double>(2 * ne);
+        SelState *sel = A.dalloc_n<SelState>(2 * ne);
+        EdgeCounts *ec = A.dalloc_n<EdgeCounts>(ne);
         push(gn, [=](hipStream_t s) {
           launch_prewitt(ni, mgd, drd, ne, maxp, s);
           launch_stats(mdd, st2, 2 * ne, s);
-          launch_sort(mdd, sbd, capd, 2 * ne, s);
-          launch_median_gini(mdd, sbd, st2, med, OutRef{nullptr}, OutRef{nullptr}, 2 * ne, s);
-          launch_edge_final(mgd, drd, st2, med, o, ne, s);
+          launch_median(mdd, st2, sel, sbd, med, 2 * ne, maxp, s);
+          launch_edge_final(mgd, drd, st2, med, ec, o, ne, maxp, s);
         });
       } break;
       case A_OTSU:
       case A_INV_OTSU: {
         std::vector<ObjDesc> od(ne);
+        int strips = 1;
         for (int k = 0; k < ne; k++) {
           const size_t P = (size_t)E[k].N->h[E[k].i] * E[k].N->w[E[k].i];
           od[k].label = A.dalloc_n<int>(P);
@@ -1385,10 +1382,13 @@ static int build_batch(wndgpu_ctx *c, const wndgpu_plan *plan, const Batch &B, A
           od[k].keys = A.dalloc_n<uint64_t>(2 * (P + 1));
           od[k].dist = A.dalloc_n<double>(P + 1);
           od[k].count = A.dalloc_n<int>(1);
+          od[k].state = A.dalloc_n<ObjState>(1);
+          od[k].chunk = A.dalloc_n<int>(obj_chunks((long)P));
+          strips = std::max(strips, obj_strips(E[k].N->h[E[k].i], E[k].N->w[E[k].i]));
         }
         ObjDesc *odd = A.stage(od);
         const int inv = alg == A_INV_OTSU;
-        push(gn, [=](hipStream_t s) { gather(s); launch_objects(ni, nst, inv, odd, o, ne, (int)maxp, s); });
+        push(gn, [=](hipStream_t s) { gather(s); launch_objects(ni, nst, inv, odd, o, ne, maxp, strips, s); });
       } break;
       case A_GABOR: {
         const int prec = plan->precision;
@@ -1451,7 +1451,7 @@ static int build_batch(wndgpu_ctx *c, const wndgpu_plan *plan, const Batch &B, A
       push("Pixel Intensity Statistics / Gini", [=](hipStream_t s) {
         launch_gather_stats(sts, nst, ne, s);
         launch_sort(ni, sbd, capd, ne, s);
-        launch_median_gini(ni, sbd, nst, nullptr, op, og, ne, s);
+        launch_median_gini(ni, sbd, nst, op, og, ne, s);
       });
     }
   }

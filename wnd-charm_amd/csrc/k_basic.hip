@@ -87,20 +87,30 @@ __global__ void __launch_bounds__(1024) k_stats(const Img *imgs, Stats *st) {
   const long n = (long)im.h * im.w;
   double s = 0, mn = 1e308, mx = -1e308;
   long long c = 0;
-  for (long i = threadIdx.x; i < n; i += blockDim.x) {
-    double v = im.p[i];
+  // a thread adds its pixels (1024 apart) in order, eight loads in flight
+  const gptr<const double> P = to_global((const double *)im.p);
+  auto each = [&](auto f) {
+    for (long i0 = threadIdx.x; i0 < n; i0 += 8 * 1024) {
+      double v[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) v[k] = P[min(i0 + 1024 * k, n - 1)];
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        if (i0 + 1024 * k < n) f(v[k]);
+    }
+  };
+  each([&](double v) {
     if (moments_ok(v)) { s += v; c++; mn = fmin(mn, v); mx = fmax(mx, v); }
-  }
+  });
   s = block_reduce(s, SumOp(), shd);
   c = block_reduce(c, SumOp(), shl);
   mn = block_reduce(mn, MinOp(), shd);
   mx = block_reduce(mx, MaxOp(), shd);
   const double mean = c ? s / (double)c : 0.0;
   double m2 = 0;
-  for (long i = threadIdx.x; i < n; i += blockDim.x) {
-    double v = im.p[i];
+  each([&](double v) {
     if (moments_ok(v)) { double d = v - mean; m2 += d * d; }
-  }
+  });
   m2 = block_reduce(m2, SumOp(), shd);
   if (threadIdx.x == 0) {
     Stats r;
@@ -398,7 +408,7 @@ __global__ void __launch_bounds__(1024) k_sort(const Img *imgs, uint64_t *const 
 // (FeatureAlgorithms.cpp:448-489) from the sorted keys; writes the five
 // Pixel Intensity Statistics (FeatureAlgorithms.cpp:272-291) and/or Gini.
 __global__ void __launch_bounds__(1024) k_median_gini(const Img *imgs, uint64_t *const *buf, const Stats *st,
-                                                      double *median_out, OutRef pix, OutRef gini) {
+                                                      OutRef pix, OutRef gini) {
   __shared__ double shd[16];
   __shared__ long long shl[16];
   __shared__ long long first_pos;
@@ -429,7 +439,6 @@ __global__ void __launch_bounds__(1024) k_median_gini(const Img *imgs, uint64_t 
   s = block_reduce(s, SumOp(), shd);
   g = block_reduce(g, SumOp(), shd);
   if (threadIdx.x == 0) {
-    if (median_out) median_out[blockIdx.x] = med;
     if (pix.rows && pix.rows[blockIdx.x]) {
       double *o = pix.rows[blockIdx.x];
       const Stats S = st[blockIdx.x];
@@ -692,9 +701,9 @@ void launch_fft(const Img *in, double2 *const *f1, const FftPlan *plw, const Fft
 void launch_sort(const Img *imgs, uint64_t *const *buf, const long *cap, int nimg, hipStream_t s) {
   k_sort<<<nimg, 1024, 0, s>>>(imgs, buf, cap);
 }
-void launch_median_gini(const Img *imgs, uint64_t *const *buf, const Stats *st, double *median_out, OutRef pix,
+void launch_median_gini(const Img *imgs, uint64_t *const *buf, const Stats *st, OutRef pix,
                         OutRef gini, int nimg, hipStream_t s) {
-  k_median_gini<<<nimg, 1024, 0, s>>>(imgs, buf, st, median_out, pix, gini);
+  k_median_gini<<<nimg, 1024, 0, s>>>(imgs, buf, st, pix, gini);
 }
 void launch_msh(const Img *imgs, const Stats *st, OutRef o, int nimg, hipStream_t s) {
   k_msh<<<nimg, 1024, 0, s>>>(imgs, st, o);

@@ -71,6 +71,10 @@ __device__ double block_otsu(long n, double mn, double mx, ValF val, int *hist) 
 }
 
 // ------------------------------------------------------------- union-find
+// Labels point to smaller indices of their component, roots to themselves.
+// find(lab, x) reads the chain, join(lab, a, b) links two components at the
+// smaller root: in LDS within a strip of rows, by device-scope atomics between
+// strips (blocks of other XCDs take part).
 __device__ __forceinline__ int uf_find(volatile int *lab, int x) {
   while (true) {
     const int p = lab[x];
@@ -78,10 +82,18 @@ __device__ __forceinline__ int uf_find(volatile int *lab, int x) {
     x = p;
   }
 }
-__device__ void uf_union(int *lab, int a, int b) {
+__device__ __forceinline__ int uf_find_device(int *lab, int x) {
   while (true) {
-    a = uf_find(lab, a);
-    b = uf_find(lab, b);
+    const int p = __hip_atomic_load(&lab[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (p == x) return x;
+    x = p;
+  }
+}
+template <class Find>
+__device__ __forceinline__ void uf_union(int *lab, int a, int b, Find find) {
+  while (true) {
+    a = find(a);
+    b = find(b);
     if (a == b) return;
     if (a < b) { const int t = a; a = b; b = t; }
     const int old = atomicMin(&lab[a], b);
@@ -93,154 +105,328 @@ __device__ void uf_union(int *lab, int a, int b) {
 // Object features (ImageMatrix::FeatureStatistics, cmatrix.cpp:1642-1717;
 // bwlabel / GlobalCentroid / FeatureCentroid / EulerNumber,
 // FeatureStatistics.cpp:44-254; output layout FeatureAlgorithms.cpp:370-394).
-// One 1024-thread work-group per image.  invert != 0 evaluates the
-// Inverse-Otsu variant on v' = (max - v) + min (ImageMatrix::invert, cmatrix.cpp:569-572).
-__global__ void __launch_bounds__(1024) k_objects(const Img *imgs, const Stats *st, int invert, const ObjDesc *ods,
-                                                  OutRef o) {
-  __shared__ int hist[1024];
+// invert != 0 evaluates the Inverse-Otsu variant on v' = (max - v) + min
+// (ImageMatrix::invert, cmatrix.cpp:569-572).  The per-pixel steps run over
+// the whole image in blocks of OBJ_CHUNK pixels or strips of up to OBJ_STRIP,
+// the per-image ones in one block:
+//   init, hist, thresh   range of the plane, its 1024-bin histogram, Otsu
+//   strip                mask and labels of a strip of rows: 8-connected
+//                        union-find in LDS; mass and coordinate sums
+//   merge                unions across the strips' first rows
+//   flat                 every pixel its root; Euler patterns; roots per block
+//   scan, rank           rank of each root in raster order, 1-based
+//   area                 areas and coordinate sums per object
+//   final                distances, the two sorted lists, the features
+// As one 1024-thread block per image, bound by its latency through every
+// pixel, a 1388 x 1040 frame took 22 ms on one of 256 CUs.  All sums over
+// pixels are of integers, so their order does not matter.
+constexpr int OBJ_CHUNK = 4096;
+constexpr int OBJ_STRIP = 16384;  // pixels; rows of up to 4096 pixels, so at least four rows
+__host__ __device__ inline int obj_strip_rows(int W) { return OBJ_STRIP / W > 1 ? OBJ_STRIP / W : 1; }
+
+__device__ __forceinline__ double obj_value(double v, int invert, const Stats &S) {
+  return invert ? (S.mx - v) + S.mn : v;
+}
+
+__global__ void __launch_bounds__(1024) k_obj_init(const Img *imgs, const Stats *st, int invert, const ObjDesc *ods) {
   __shared__ double shd[16];
-  __shared__ long long shl[16];
-  __shared__ int scan_w[16];
-  __shared__ int s_base;
   const Img im = imgs[blockIdx.x];
-  const ObjDesc OD = ods[blockIdx.x];
   const Stats S = st[blockIdx.x];
-  const int W = im.w, H = im.h;
-  const long n = (long)W * H;
-  const int t = threadIdx.x;
-  const double smx = S.mx, smn = S.mn;
-  auto val = [&](long i) -> double { return invert ? (smx - im.p[i]) + smn : im.p[i]; };
-  // stats of the plane the features are taken on
-  double mn = smn, mx = smx;
+  ObjState *T = ods[blockIdx.x].state;
+  const long n = (long)im.w * im.h;
+  double mn = S.mn, mx = S.mx;
   if (invert) {
-    double a = 1e308, b = -1e308;
-    for (long i = t; i < n; i += 1024) {
-      const double v = val(i);
-      if (moments_ok(v)) { a = fmin(a, v); b = fmax(b, v); }
-    }
-    mn = block_reduce(a, MinOp(), shd);
-    mx = block_reduce(b, MaxOp(), shd);
-  }
-  const double thr = block_otsu(n, mn, mx, val, hist);
-  int *lab = OD.label;
-  // mask, labels, global centroid (exact integer sums).  A wave takes 64
-  // consecutive pixels (raster order); each mask pixel starts at the first
-  // pixel of its run inside that segment (a ballot), so runs need no unions
-  // within a segment and the trees stay shallow.
-  long long xm = 0, ym = 0, mass = 0, c1 = 0, c3 = 0;
-  const int lane = t & 63;
-  for (long c0 = 0; c0 < n; c0 += 1024) {
-    const long i = c0 + t;
-    const bool m = i < n && val(i) > thr;
-    const int y = (int)(i / W), x = (int)(i - (long)y * W);
-    // bit l: pixel l of the segment continues the run of pixel l - 1 (both
-    // in the mask, the same row)
-    const unsigned long long mb = __ballot(m);
-    const unsigned long long cont = __ballot(m && x > 0) & (mb << 1);
-    const unsigned long long below = lane == 63 ? ~0ull : ((2ull << lane) - 1);
-    const int head = 63 - __clzll(~cont & below);
-    if (i < n) lab[i] = m ? (int)(i - (lane - head)) : -1;
-    if (m) {
-      xm += x + 1; ym += y + 1; mass++;
+    // the inversion is monotone, so its extremes are those of the extremes,
+    // provided that every pixel counts (Moments2's rule) before and after
+    mn = (S.mx - S.mx) + S.mn;
+    mx = (S.mx - S.mn) + S.mn;
+    if (S.n != n || !moments_ok(mn) || !moments_ok(mx)) {
+      double a = 1e308, b = -1e308;
+      for (long i = threadIdx.x; i < n; i += 1024) {
+        const double v = obj_value(im.p[i], 1, S);
+        if (moments_ok(v)) { a = fmin(a, v); b = fmax(b, v); }
+      }
+      mn = block_reduce(a, MinOp(), shd);
+      mx = block_reduce(b, MaxOp(), shd);
     }
   }
+  T->hist[threadIdx.x] = 0;
+  if (threadIdx.x == 0) {
+    T->mn = mn;
+    T->mx = mx;
+    T->xm = T->ym = T->mass = T->c1 = T->c3 = 0;
+  }
+}
+
+__global__ void __launch_bounds__(256) k_obj_hist(const Img *imgs, const Stats *st, int invert, const ObjDesc *ods) {
+  __shared__ int hist[1024];
+  const Img im = imgs[blockIdx.y];
+  const long n = (long)im.w * im.h, c0 = (long)blockIdx.x * OBJ_CHUNK;
+  if (c0 >= n) return;
+  const Stats S = st[blockIdx.y];
+  ObjState *T = ods[blockIdx.y].state;
+  const double mn = T->mn, sc = hist_scale(mn, T->mx, 1024);
+  const gptr<const double> P = to_global((const double *)im.p);
+  for (int b = threadIdx.x; b < 1024; b += 256) hist[b] = 0;
+  double v[OBJ_CHUNK / 256];
+#pragma unroll
+  for (int k = 0; k < OBJ_CHUNK / 256; k++) v[k] = P[min(c0 + 256 * k + threadIdx.x, n - 1)];
   __syncthreads();
-  // 8-connected union-find; every root ends at the component's smallest
-  // index.  Of a horizontal run [s, e] the upper neighbours are s-1 .. e+1:
-  // each pixel joins its upper-right one, the run's first pixel also its
-  // upper-left and upper ones; a segment's first pixel joins its left
-  // neighbour when the run crosses the segment boundary.
-  for (long i = t; i < n; i += 1024) {
-    if (lab[i] < 0) continue;
-    const int y = i / W, x = i - (long)y * W;
-    const bool left = x > 0 && lab[i - 1] >= 0;
-    if (left && (i & 63) == 0) uf_union(lab, (int)i, (int)(i - 1));
-    if (y > 0) {
-      const long u = i - W;
-      if (x < W - 1 && lab[u + 1] >= 0) uf_union(lab, (int)i, (int)(u + 1));
-      if (!left) {
-        if (x > 0 && lab[u - 1] >= 0) uf_union(lab, (int)i, (int)(u - 1));
-        if (lab[u] >= 0) uf_union(lab, (int)i, (int)u);
+#pragma unroll
+  for (int k = 0; k < OBJ_CHUNK / 256; k++)
+    if (c0 + 256 * k + threadIdx.x < n) atomicAdd(&hist[hist_bin(obj_value(v[k], invert, S), mn, sc, 1024)], 1);
+  __syncthreads();
+  for (int b = threadIdx.x; b < 1024; b += 256)
+    if (hist[b]) atomicAdd(&T->hist[b], hist[b]);
+}
+
+__global__ void __launch_bounds__(1024) k_obj_thresh(const Img *imgs, const ObjDesc *ods) {
+  __shared__ int hist[1024];
+  const Img im = imgs[blockIdx.x];
+  ObjState *T = ods[blockIdx.x].state;
+  hist[threadIdx.x] = T->hist[threadIdx.x];
+  __syncthreads();
+  const double thr = otsu_threshold(hist, (long)im.w * im.h, T->mn, T->mx);
+  if (threadIdx.x == 0) T->thr = thr;
+}
+
+__global__ void __launch_bounds__(1024) k_obj_strip(const Img *imgs, const Stats *st, int invert, const ObjDesc *ods) {
+  __shared__ int lab[OBJ_STRIP];
+  __shared__ long long shl[16];
+  const Img im = imgs[blockIdx.y];
+  const int W = im.w, RS = obj_strip_rows(W), y0 = blockIdx.x * RS;
+  if (y0 >= im.h) return;
+  const ObjDesc OD = ods[blockIdx.y];
+  const Stats S = st[blockIdx.y];
+  ObjState *T = OD.state;
+  const double thr = T->thr;
+  const int m = min(RS, im.h - y0) * W, base = y0 * W, t = threadIdx.x, lane = t & 63;
+  const gptr<const double> P = to_global((const double *)im.p) + base;
+  // A wave takes 64 consecutive pixels (raster order); each mask pixel starts
+  // at the first pixel of its run inside that segment (a ballot), so runs need
+  // no unions within a segment and the trees stay shallow.
+  long long xm = 0, ym = 0, mass = 0;
+  for (int c0 = 0; c0 < m; c0 += 4096) {
+    double v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = P[min(c0 + 1024 * k + t, m - 1)];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const int i = c0 + 1024 * k + t;
+      const bool in = i < m && obj_value(v[k], invert, S) > thr;
+      const int y = i / W, x = i - y * W;
+      // bit l: pixel l of the segment continues the run of pixel l - 1 (both
+      // in the mask, the same row)
+      const unsigned long long mb = __ballot(in);
+      const unsigned long long cont = __ballot(in && x > 0) & (mb << 1);
+      const unsigned long long below = lane == 63 ? ~0ull : ((2ull << lane) - 1);
+      const int head = 63 - __clzll(~cont & below);
+      if (i < m) lab[i] = in ? i - (lane - head) : -1;
+      if (in) {
+        xm += x + 1;
+        ym += y0 + y + 1;
+        mass++;
       }
     }
   }
   __syncthreads();
-  __threadfence_block();
-  for (long i = t; i < n; i += 1024)
-    if (lab[i] >= 0) lab[i] = uf_find(lab, (int)i);
-  __syncthreads();
-  // Euler number patterns (EulerNumber(8): (C1 - C3) / 4; Cd is never counted)
-  for (long i = t; i < n; i += 1024) {
-    const int y = i / W, x = i - (long)y * W;
-    if (y < 1 || x < 1) continue;
-    const int c = (lab[i - W - 1] >= 0) + (lab[i - W] >= 0) + (lab[i - 1] >= 0) + (lab[i] >= 0);
-    c1 += (c == 1);
-    c3 += (c == 3);
+  // Of a horizontal run [s, e] the upper neighbours are s-1 .. e+1: each pixel
+  // joins its upper-right one, the run's first pixel also its upper-left and
+  // upper ones; a segment's first pixel joins its left neighbour when the run
+  // crosses the segment boundary.
+  auto find = [&](int x) { return uf_find(lab, x); };
+  for (int i = t; i < m; i += 1024) {
+    if (lab[i] < 0) continue;
+    const int y = i / W, x = i - y * W;
+    const bool left = x > 0 && lab[i - 1] >= 0;
+    if (left && (i & 63) == 0) uf_union(lab, i, i - 1, find);
+    if (y > 0) {
+      const int u = i - W;
+      if (x < W - 1 && lab[u + 1] >= 0) uf_union(lab, i, u + 1, find);
+      if (!left) {
+        if (x > 0 && lab[u - 1] >= 0) uf_union(lab, i, u - 1, find);
+        if (lab[u] >= 0) uf_union(lab, i, u, find);
+      }
+    }
   }
+  __syncthreads();
+  for (int i = t; i < m; i += 1024) OD.label[base + i] = lab[i] >= 0 ? base + uf_find(lab, i) : -1;
   xm = block_reduce(xm, SumOp(), shl);
   ym = block_reduce(ym, SumOp(), shl);
   mass = block_reduce(mass, SumOp(), shl);
+  if (t == 0 && mass) {
+    atomicAdd((unsigned long long *)&T->xm, (unsigned long long)xm);
+    atomicAdd((unsigned long long *)&T->ym, (unsigned long long)ym);
+    atomicAdd((unsigned long long *)&T->mass, (unsigned long long)mass);
+  }
+}
+
+__global__ void __launch_bounds__(256) k_obj_merge(const Img *imgs, const ObjDesc *ods) {
+  const Img im = imgs[blockIdx.y];
+  const int W = im.w, y = (blockIdx.x + 1) * obj_strip_rows(W);
+  if (y >= im.h) return;
+  int *lab = ods[blockIdx.y].label;
+  // a label's sign never changes, so plain reads tell the mask
+  auto find = [&](int x) { return uf_find_device(lab, x); };
+  for (int x = threadIdx.x; x < W; x += 256) {
+    const int i = y * W + x, u = i - W;
+    if (lab[i] < 0) continue;
+    const bool left = x > 0 && lab[i - 1] >= 0;
+    if (x < W - 1 && lab[u + 1] >= 0) uf_union(lab, i, u + 1, find);
+    if (!left) {
+      if (x > 0 && lab[u - 1] >= 0) uf_union(lab, i, u - 1, find);
+      if (lab[u] >= 0) uf_union(lab, i, u, find);
+    }
+  }
+}
+
+__global__ void __launch_bounds__(1024) k_obj_flat(const Img *imgs, const ObjDesc *ods) {
+  __shared__ long long shl[16];
+  const Img im = imgs[blockIdx.y];
+  const int W = im.w, n = W * im.h, c0 = blockIdx.x * OBJ_CHUNK;
+  if (c0 >= n) return;
+  const ObjDesc OD = ods[blockIdx.y];
+  int *lab = OD.label;
+  long long c1 = 0, c3 = 0, roots = 0;
+#pragma unroll
+  for (int k = 0; k < OBJ_CHUNK / 1024; k++) {
+    const int i = c0 + 1024 * k + threadIdx.x;
+    if (i >= n) break;
+    const int y = i / W, x = i - y * W;
+    const int p = lab[i];
+    if (y >= 1 && x >= 1) {  // EulerNumber(8): (C1 - C3) / 4; Cd is never counted
+      const int c = (lab[i - W - 1] >= 0) + (lab[i - W] >= 0) + (lab[i - 1] >= 0) + (p >= 0);
+      c1 += (c == 1);
+      c3 += (c == 3);
+    }
+    if (p >= 0) {  // other threads shorten the chain meanwhile: any read of it leads to the root
+      const int r = uf_find(lab, p);
+      if (r != p) lab[i] = r;
+      roots += r == i;
+    }
+  }
   c1 = block_reduce(c1, SumOp(), shl);
   c3 = block_reduce(c3, SumOp(), shl);
-  // label ids: rank of each root in raster order (1-based)
-  int *rid = (int *)OD.keys;  // reuse: rid[i] for roots, before the keys are needed
-  if (t == 0) s_base = 0;
+  roots = block_reduce(roots, SumOp(), shl);
+  if (threadIdx.x == 0) {
+    OD.chunk[blockIdx.x] = (int)roots;
+    if (c1) atomicAdd((unsigned long long *)&OD.state->c1, (unsigned long long)c1);
+    if (c3) atomicAdd((unsigned long long *)&OD.state->c3, (unsigned long long)c3);
+  }
+}
+
+// exclusive prefix of the blocks' root counts
+__global__ void __launch_bounds__(1024) k_obj_scan(const Img *imgs, const ObjDesc *ods) {
+  __shared__ int sh[1024];
+  const Img im = imgs[blockIdx.x];
+  const ObjDesc OD = ods[blockIdx.x];
+  const int nc = (int)(((long)im.w * im.h + OBJ_CHUNK - 1) / OBJ_CHUNK), t = threadIdx.x;
+  const int per = (nc + 1023) / 1024;
+  int s = 0;
+  for (int k = 0; k < per; k++)
+    if (t * per + k < nc) s += OD.chunk[t * per + k];
+  sh[t] = s;
   __syncthreads();
-  for (long c0 = 0; c0 < n; c0 += 1024) {
-    const long i = c0 + t;
-    const int isroot = (i < n && lab[i] == (int)i) ? 1 : 0;
-    // block exclusive scan of isroot
-    const int wv = t >> 6;
-    const uint64_t bal = __ballot(isroot);
-    const int pre = __popcll(bal & ((lane == 0) ? 0ull : (~0ull >> (64 - lane))));
+  for (int o = 1; o < 1024; o <<= 1) {
+    const int v = t >= o ? sh[t - o] : 0;
+    __syncthreads();
+    sh[t] += v;
+    __syncthreads();
+  }
+  int acc = sh[t] - s;
+  for (int k = 0; k < per; k++)
+    if (t * per + k < nc) {
+      const int c = OD.chunk[t * per + k];
+      OD.chunk[t * per + k] = acc;
+      acc += c;
+    }
+  if (t == 1023) OD.count[0] = sh[1023];
+}
+
+// label ids: rank of each root in raster order (1-based), in the sort buffer;
+// the per-object sums cleared
+__global__ void __launch_bounds__(1024) k_obj_rank(const Img *imgs, const ObjDesc *ods) {
+  __shared__ int scan_w[16];
+  const Img im = imgs[blockIdx.y];
+  const int n = im.w * im.h, c0 = blockIdx.x * OBJ_CHUNK, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  if (c0 >= n) return;
+  const ObjDesc OD = ods[blockIdx.y];
+  int *rid = (int *)OD.keys;
+  const int count = OD.count[0], last = c0 + OBJ_CHUNK >= n;
+  int base = OD.chunk[blockIdx.x];
+  for (int k = 0; k < OBJ_CHUNK / 1024; k++) {
+    const int i = c0 + 1024 * k + threadIdx.x;
+    const int isroot = i < n && OD.label[i] == i;
+    const unsigned long long bal = __ballot(isroot);
+    const int pre = __popcll(bal & ((1ull << lane) - 1));
+    __syncthreads();
     if (lane == 0) scan_w[wv] = __popcll(bal);
     __syncthreads();
     int woff = 0, tot = 0;
-    for (int w = 0; w < 16; w++) { if (w < wv) woff += scan_w[w]; tot += scan_w[w]; }
-    if (isroot) rid[i] = s_base + woff + pre + 1;
-    __syncthreads();
-    if (t == 0) s_base += tot;
-    __syncthreads();
-  }
-  const int count = s_base;
-  int *area = OD.area;
-  long long *axm = OD.xm, *aym = OD.ym;
-  for (long l = t; l <= count; l += 1024) { area[l] = 0; axm[l] = 0; aym[l] = 0; }
-  __syncthreads();
-  // areas and coordinate sums per object: the lanes of a wave holding one
-  // label add theirs first, then one lane adds the totals (exact integers)
-  for (long c0 = 0; c0 < n; c0 += 1024) {
-    const long i = c0 + t;
-    int l = -1;
-    long long px = 0, py = 0;
-    if (i < n) {
-      const int r = lab[i];
-      if (r >= 0) {
-        l = rid[r];
-        const int y = i / W, x = i - (long)y * W;
-        px = x + 1;
-        py = y + 1;
-      }
+    for (int w = 0; w < 16; w++) {
+      if (w < wv) woff += scan_w[w];
+      tot += scan_w[w];
     }
+    if (isroot) rid[i] = base + woff + pre + 1;
+    base += tot;
+  }
+  for (int l = c0 + threadIdx.x; l < (last ? count + 1 : min(c0 + OBJ_CHUNK, count + 1)); l += 1024) {
+    OD.area[l] = 0;
+    OD.xm[l] = 0;
+    OD.ym[l] = 0;
+  }
+}
+
+// areas and coordinate sums per object: the lanes of a wave holding one label
+// add theirs first, then one lane adds the totals (exact integers)
+__global__ void __launch_bounds__(1024) k_obj_area(const Img *imgs, const ObjDesc *ods) {
+  const Img im = imgs[blockIdx.y];
+  const int W = im.w, n = W * im.h, c0 = blockIdx.x * OBJ_CHUNK, lane = threadIdx.x & 63;
+  if (c0 >= n) return;
+  const ObjDesc OD = ods[blockIdx.y];
+  const int *rid = (const int *)OD.keys;
+  int r[OBJ_CHUNK / 1024], id[OBJ_CHUNK / 1024];
+#pragma unroll
+  for (int k = 0; k < OBJ_CHUNK / 1024; k++) {
+    const int i = c0 + 1024 * k + threadIdx.x;
+    r[k] = i < n ? OD.label[i] : -1;
+  }
+#pragma unroll
+  for (int k = 0; k < OBJ_CHUNK / 1024; k++) id[k] = r[k] >= 0 ? rid[r[k]] : -1;
+#pragma unroll
+  for (int k = 0; k < OBJ_CHUNK / 1024; k++) {
+    const int i = c0 + 1024 * k + threadIdx.x, l = id[k];
+    const int y = i / W, x = i - y * W;
+    const int px = l >= 0 ? x + 1 : 0, py = l >= 0 ? y + 1 : 0;
     for (unsigned long long pend = __ballot(l >= 0); pend;) {
       const int lead = __ffsll((long long)pend) - 1;
       const int ll = __shfl(l, lead, 64);
       const bool mine = l == ll;
       const unsigned long long mm = __ballot(mine);
-      long long sx = mine ? px : 0, sy = mine ? py : 0;
+      int sx = mine ? px : 0, sy = mine ? py : 0;  // at most 64 x 4096
       for (int off = 32; off > 0; off >>= 1) {
         sx += __shfl_xor(sx, off, 64);
         sy += __shfl_xor(sy, off, 64);
       }
       if (lane == lead) {
-        atomicAdd(&area[ll], (int)__popcll(mm));
-        atomicAdd((unsigned long long *)&axm[ll], (unsigned long long)sx);
-        atomicAdd((unsigned long long *)&aym[ll], (unsigned long long)sy);
+        atomicAdd(&OD.area[ll], (int)__popcll(mm));
+        atomicAdd((unsigned long long *)&OD.xm[ll], (unsigned long long)sx);
+        atomicAdd((unsigned long long *)&OD.ym[ll], (unsigned long long)sy);
       }
       pend &= ~mm;
     }
   }
-  __syncthreads();
+}
+
+__global__ void __launch_bounds__(1024) k_obj_final(const ObjDesc *ods, OutRef o) {
+  __shared__ int hist[20];
+  __shared__ double shd[16];
+  const ObjDesc OD = ods[blockIdx.x];
+  const ObjState &T = *OD.state;
+  const int t = threadIdx.x, count = OD.count[0];
+  const long long xm = T.xm, ym = T.ym, mass = T.mass, c1 = T.c1, c3 = T.c3;
+  int *area = OD.area;
+  const long long *axm = OD.xm, *aym = OD.ym;
   // per-object distance to the global centroid
   double cx = 0, cy = 0;
   if (mass) { cx = (double)xm / (double)mass; cy = (double)ym / (double)mass; }
@@ -316,11 +502,22 @@ __global__ void __launch_bounds__(1024) k_objects(const Img *imgs, const Stats *
   }
 }
 
-void launch_objects(const Img *imgs, const Stats *st, int invert, const ObjDesc *od, OutRef o, int nimg, int maxn,
-                    hipStream_t s) {
-  (void)maxn;
-  k_objects<<<nimg, 1024, 0, s>>>(imgs, st, invert, od, o);
+void launch_objects(const Img *imgs, const Stats *st, int invert, const ObjDesc *od, OutRef o, int nimg, long maxn,
+                    int maxstrips, hipStream_t s) {
+  const dim3 chunks((unsigned)((maxn + OBJ_CHUNK - 1) / OBJ_CHUNK), nimg);
+  k_obj_init<<<nimg, 1024, 0, s>>>(imgs, st, invert, od);
+  k_obj_hist<<<chunks, 256, 0, s>>>(imgs, st, invert, od);
+  k_obj_thresh<<<nimg, 1024, 0, s>>>(imgs, od);
+  k_obj_strip<<<dim3(maxstrips, nimg), 1024, 0, s>>>(imgs, st, invert, od);
+  if (maxstrips > 1) k_obj_merge<<<dim3(maxstrips - 1, nimg), 256, 0, s>>>(imgs, od);
+  k_obj_flat<<<chunks, 1024, 0, s>>>(imgs, od);
+  k_obj_scan<<<nimg, 1024, 0, s>>>(imgs, od);
+  k_obj_rank<<<chunks, 1024, 0, s>>>(imgs, od);
+  k_obj_area<<<chunks, 1024, 0, s>>>(imgs, od);
+  k_obj_final<<<nimg, 1024, 0, s>>>(od, o);
 }
+int obj_strips(int h, int w) { return (h + obj_strip_rows(w) - 1) / obj_strip_rows(w); }
+int obj_chunks(long n) { return (int)((n + OBJ_CHUNK - 1) / OBJ_CHUNK); }
 
 // ================================================================ Edge features
 // Prewitt magnitude / direction (cmatrix.cpp:1317-1384), x outer order of the
@@ -343,60 +540,271 @@ __global__ void k_prewitt(const Img *in, const Img *mag, const Img *dir) {
   od.p[i] = d;
 }
 
-// EdgeStatistics (cmatrix.cpp:1402-1458) + output layout (FeatureAlgorithms.cpp:314-335).
-// st2[2*i] / st2[2*i+1] and medians[2*i] / [2*i+1] belong to magnitude / direction.
-__global__ void __launch_bounds__(256) k_edge_final(const Img *mag, const Img *dir, const Stats *st2,
-                                                    const double *medians, OutRef o) {
-  __shared__ long long shl[4];
-  __shared__ int hm[8], hd[8];
-  const Img M = mag[blockIdx.x], D = dir[blockIdx.x];
-  const Stats SM = st2[2 * blockIdx.x], SD = st2[2 * blockIdx.x + 1];
-  const long n = (long)M.h * M.w;
-  if (threadIdx.x < 8) { hm[threadIdx.x] = 0; hd[threadIdx.x] = 0; }
-  __syncthreads();
-  const double level = SM.mean;
-  const double sm = hist_scale(SM.mn, SM.mx, 8), sd = hist_scale(SD.mn, SD.mx, 8);
-  long long area = 0;
-  for (long i = threadIdx.x; i < n; i += blockDim.x) {
-    const double m = M.p[i];
-    if (m > level) area++;
-    atomicAdd(&hm[hist_bin(m, SM.mn, sm, 8)], 1);
-    atomicAdd(&hd[hist_bin(D.p[i], SD.mn, sd, 8)], 1);
-  }
-  area = block_reduce(area, SumOp(), shl);
+// ------------------------------------------------------------------ medians
+// Median of each plane (ImageMatrix::get_median, cmatrix.cpp:780-800) without
+// sorting it: the values are counted in SEL_BINS bins between the plane's
+// extremes (a binning that follows the keys' order, NaN and infinities
+// included), the keys of the bin or two that hold the middle ranks are
+// collected, and one block finds the ranks among those, digit by digit.  A
+// 1388 x 1040 frame's two edge planes took 17 of 20.8 ms as one-block radix
+// sorts.
+__device__ __forceinline__ int sel_bin(double v, double mn, double mx, double scale) {
+  if (v != v) return __double_as_longlong(v) < 0 ? 0 : SEL_BINS - 1;
+  if (v <= mn) return 0;
+  if (v >= mx) return SEL_BINS - 1;
+  return min((int)((v - mn) * scale), SEL_BINS - 1);
+}
+__global__ void __launch_bounds__(1024) k_sel_init(SelState *sel) {
+  SelState &T = sel[blockIdx.x];
+  for (int b = threadIdx.x; b < SEL_BINS; b += 1024) T.hist[b] = 0;
   if (threadIdx.x == 0) {
-    double DH[8], MH[8], diff[4] = {0, 0, 0, 0}, homog = 0;
-    for (int b = 0; b < 8; b++) { DH[b] = hd[b]; MH[b] = hm[b]; }
-    for (int b = 0; b < 4; b++) diff[b] = fabs(DH[b] - DH[b + 4]);
-    double sum = 0;
-    for (int b = 0; b < 4; b++) {
-      if (DH[b] + DH[b + 4] != 0) diff[b] = diff[b] / (DH[b] + DH[b + 4]);
-      sum += (DH[b] + DH[b + 4]);
+    T.count = 0;
+    T.kmin = ~0ull;
+    T.kmax = 0;
+  }
+}
+__global__ void __launch_bounds__(256) k_sel_hist(const Img *planes, const Stats *st, SelState *sel) {
+  __shared__ int hist[SEL_BINS];
+  const Img im = planes[blockIdx.y];
+  const long n = (long)im.w * im.h, c0 = (long)blockIdx.x * SEL_CHUNK;
+  if (c0 >= n) return;
+  const Stats S = st[blockIdx.y];
+  SelState &T = sel[blockIdx.y];
+  const double scale = hist_scale(S.mn, S.mx, SEL_BINS);
+  const gptr<const double> P = to_global((const double *)im.p);
+  for (int b = threadIdx.x; b < SEL_BINS; b += 256) hist[b] = 0;
+  __syncthreads();
+  for (int r = 0; r < SEL_CHUNK; r += 256 * 16) {
+    double v[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) v[k] = P[min(c0 + r + 256 * k + threadIdx.x, n - 1)];
+#pragma unroll
+    for (int k = 0; k < 16; k++)
+      if (c0 + r + 256 * k + threadIdx.x < n) atomicAdd(&hist[sel_bin(v[k], S.mn, S.mx, scale)], 1);
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < SEL_BINS; b += 256)
+    if (hist[b]) atomicAdd(&T.hist[b], hist[b]);
+}
+// the bins of ranks (n - 1) / 2 and n / 2
+__global__ void __launch_bounds__(1024) k_sel_pick(const Img *planes, SelState *sel) {
+  __shared__ int sh[1024];
+  const Img im = planes[blockIdx.x];
+  const int n = im.w * im.h, t = threadIdx.x, r0 = (n - 1) / 2, r1 = n / 2;
+  SelState &T = sel[blockIdx.x];
+  constexpr int PER = SEL_BINS / 1024;
+  int c[PER], s = 0;
+#pragma unroll
+  for (int k = 0; k < PER; k++) s += c[k] = T.hist[t * PER + k];
+  sh[t] = s;
+  __syncthreads();
+  for (int o = 1; o < 1024; o <<= 1) {
+    const int v = t >= o ? sh[t - o] : 0;
+    __syncthreads();
+    sh[t] += v;
+    __syncthreads();
+  }
+  int acc = sh[t] - s;
+#pragma unroll
+  for (int k = 0; k < PER; k++) {
+    if (r0 >= acc && r0 < acc + c[k]) {
+      T.lo = t * PER + k;
+      T.rank = r0 - acc;
     }
-    if (sum > 0) homog = (DH[0] + DH[1]) / sum;
-    double *c = o.rows[blockIdx.x];
-    int h = 0;
-    c[h++] = (double)area;
-    for (int j = 0; j < 4; j++) c[h++] = diff[j];
-    for (int j = 0; j < 8; j++) c[h++] = DH[j];
-    c[h++] = homog;
-    c[h++] = SD.mean;
-    c[h++] = medians[2 * blockIdx.x + 1];
-    c[h++] = SD.var;
-    for (int j = 0; j < 8; j++) c[h++] = MH[j];
-    c[h++] = SM.mean;
-    c[h++] = medians[2 * blockIdx.x];
-    c[h++] = SM.var;
+    if (r1 >= acc && r1 < acc + c[k]) T.hi = t * PER + k;
+    acc += c[k];
+  }
+}
+__global__ void __launch_bounds__(256) k_sel_collect(const Img *planes, const Stats *st, SelState *sel, uint64_t *const *keys) {
+  const Img im = planes[blockIdx.y];
+  const long n = (long)im.w * im.h, c0 = (long)blockIdx.x * SEL_CHUNK;
+  if (c0 >= n) return;
+  const Stats S = st[blockIdx.y];
+  SelState &T = sel[blockIdx.y];
+  uint64_t *out = keys[blockIdx.y];
+  const int lo = T.lo, hi = T.hi, lane = threadIdx.x & 63;
+  const double scale = hist_scale(S.mn, S.mx, SEL_BINS);
+  const gptr<const double> P = to_global((const double *)im.p);
+  uint64_t kmin = ~0ull, kmax = 0;
+  for (int r = 0; r < SEL_CHUNK; r += 256 * 16) {
+    double v[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) v[k] = P[min(c0 + r + 256 * k + threadIdx.x, n - 1)];
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+      const int b = sel_bin(v[k], S.mn, S.mx, scale);
+      const bool in = c0 + r + 256 * k + threadIdx.x < n && (b == lo || b == hi);
+      const unsigned long long m = __ballot(in);
+      if (m == 0) continue;
+      int base = 0;
+      if (lane == 0) base = atomicAdd(&T.count, (int)__popcll(m));
+      base = __shfl(base, 0, 64);
+      if (in) {
+        const uint64_t key = dkey(v[k]);
+        out[base + __popcll(m & ((1ull << lane) - 1))] = key;
+        kmin = key < kmin ? key : kmin;
+        kmax = key > kmax ? key : kmax;
+      }
+    }
+  }
+  if (kmin <= kmax) {
+    atomicMin((unsigned long long *)&T.kmin, (unsigned long long)kmin);
+    atomicMax((unsigned long long *)&T.kmax, (unsigned long long)kmax);
+  }
+}
+__global__ void __launch_bounds__(1024) k_sel_final(const Img *planes, const SelState *sel, uint64_t *const *keys, double *median) {
+  __shared__ int hist[256];
+  __shared__ unsigned long long s_next;
+  __shared__ int s_digit, s_rank;
+  const Img im = planes[blockIdx.x];
+  const SelState &T = sel[blockIdx.x];
+  const int n = im.w * im.h, m = T.count, t = threadIdx.x;
+  const uint64_t *k = keys[blockIdx.x];
+  uint64_t k0 = T.kmin, k1 = T.kmin;
+  if (T.kmin != T.kmax) {
+    // the key of rank T.rank: its digits from the highest, the keys that share
+    // the digits found so far counted by the next one
+    uint64_t prefix = 0, mask = 0;
+    int rank = T.rank, equal = 0;
+    for (int sh = 56; sh >= 0; sh -= 8) {
+      if (((T.kmin ^ T.kmax) >> sh) == 0) {  // a leading part that all keys share
+        mask |= 0xffull << sh;
+        prefix |= T.kmin & (0xffull << sh);
+        equal = m;
+        continue;
+      }
+      for (int b = t; b < 256; b += 1024) hist[b] = 0;
+      __syncthreads();
+      for (int i = t; i < m; i += 1024)
+        if ((k[i] & mask) == prefix) atomicAdd(&hist[(k[i] >> sh) & 255], 1);
+      __syncthreads();
+      if (t == 0) {
+        int b = 0, r = rank;
+        while (r >= hist[b]) r -= hist[b++];
+        s_digit = b;
+        s_rank = r;
+      }
+      __syncthreads();
+      rank = s_rank;
+      equal = hist[s_digit];
+      prefix |= (uint64_t)s_digit << sh;
+      mask |= 0xffull << sh;
+      __syncthreads();
+    }
+    k0 = k1 = prefix;
+    if (n % 2 == 0 && rank + 1 >= equal) {  // the next rank is the smallest larger key
+      if (t == 0) s_next = ~0ull;
+      __syncthreads();
+      uint64_t best = ~0ull;
+      for (int i = t; i < m; i += 1024)
+        if (k[i] > k0 && k[i] < best) best = k[i];
+      if (best != ~0ull) atomicMin(&s_next, (unsigned long long)best);
+      __syncthreads();
+      k1 = s_next;
+    }
+  }
+  if (t == 0) {
+    double med;
+    if (n % 2 == 0) {
+      med = dkey_inv(k1);
+      med += dkey_inv(k0);
+      med /= 2.0;
+    } else {
+      med = dkey_inv(k0);
+    }
+    median[blockIdx.x] = med;
   }
 }
 
+// EdgeStatistics (cmatrix.cpp:1402-1458) + output layout (FeatureAlgorithms.cpp:314-335).
+// st2[2*i] / st2[2*i+1] and medians[2*i] / [2*i+1] belong to magnitude / direction.
+// Counts over blocks of pixels: each thread counts its own pixels' bins in the
+// bytes of two words, then the wave and the block add them.
+__global__ void __launch_bounds__(256) k_edge_count(const Img *mag, const Img *dir, const Stats *st2, EdgeCounts *cnt) {
+  const Img M = mag[blockIdx.y], D = dir[blockIdx.y];
+  const long n = (long)M.h * M.w, c0 = (long)blockIdx.x * SEL_CHUNK;
+  if (c0 >= n) return;
+  const Stats SM = st2[2 * blockIdx.y], SD = st2[2 * blockIdx.y + 1];
+  const double level = SM.mean;
+  const double sm = hist_scale(SM.mn, SM.mx, 8), sd = hist_scale(SD.mn, SD.mx, 8);
+  const gptr<const double> PM = to_global((const double *)M.p), PD = to_global((const double *)D.p);
+  static_assert(SEL_CHUNK / 256 < 256, "a thread's pixels are counted in bytes");
+  uint64_t wm = 0, wd = 0;
+  int area = 0;
+  for (int r = 0; r < SEL_CHUNK; r += 256 * 8) {
+    double a[8], b[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const long i = min(c0 + r + 256 * k + threadIdx.x, n - 1);
+      a[k] = PM[i];
+      b[k] = PD[i];
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+      if (c0 + r + 256 * k + threadIdx.x < n) {
+        area += a[k] > level;
+        wm += 1ull << (8 * hist_bin(a[k], SM.mn, sm, 8));
+        wd += 1ull << (8 * hist_bin(b[k], SD.mn, sd, 8));
+      }
+  }
+  EdgeCounts &T = cnt[blockIdx.y];
+  auto add = [&](int v, int *p) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+    if ((threadIdx.x & 63) == 0 && v) atomicAdd(p, v);
+  };
+  add(area, &T.area);
+#pragma unroll
+  for (int b = 0; b < 8; b++) {
+    add((int)((wm >> (8 * b)) & 255), &T.hm[b]);
+    add((int)((wd >> (8 * b)) & 255), &T.hd[b]);
+  }
+}
+__global__ void __launch_bounds__(64) k_edge_final(const EdgeCounts *cnt, const Stats *st2, const double *medians, OutRef o) {
+  if (threadIdx.x != 0) return;
+  const Stats SM = st2[2 * blockIdx.x], SD = st2[2 * blockIdx.x + 1];
+  const EdgeCounts &T = cnt[blockIdx.x];
+  double DH[8], MH[8], diff[4] = {0, 0, 0, 0}, homog = 0;
+  for (int b = 0; b < 8; b++) { DH[b] = T.hd[b]; MH[b] = T.hm[b]; }
+  for (int b = 0; b < 4; b++) diff[b] = fabs(DH[b] - DH[b + 4]);
+  double sum = 0;
+  for (int b = 0; b < 4; b++) {
+    if (DH[b] + DH[b + 4] != 0) diff[b] = diff[b] / (DH[b] + DH[b + 4]);
+    sum += (DH[b] + DH[b + 4]);
+  }
+  if (sum > 0) homog = (DH[0] + DH[1]) / sum;
+  double *c = o.rows[blockIdx.x];
+  int h = 0;
+  c[h++] = (double)T.area;
+  for (int j = 0; j < 4; j++) c[h++] = diff[j];
+  for (int j = 0; j < 8; j++) c[h++] = DH[j];
+  c[h++] = homog;
+  c[h++] = SD.mean;
+  c[h++] = medians[2 * blockIdx.x + 1];
+  c[h++] = SD.var;
+  for (int j = 0; j < 8; j++) c[h++] = MH[j];
+  c[h++] = SM.mean;
+  c[h++] = medians[2 * blockIdx.x];
+  c[h++] = SM.var;
+}
+
+void launch_median(const Img *planes, const Stats *st, SelState *sel, uint64_t *const *keys, double *median, int nplanes,
+                   long maxn, hipStream_t s) {
+  const dim3 chunks((unsigned)((maxn + SEL_CHUNK - 1) / SEL_CHUNK), nplanes);
+  k_sel_init<<<nplanes, 1024, 0, s>>>(sel);
+  k_sel_hist<<<chunks, 256, 0, s>>>(planes, st, sel);
+  k_sel_pick<<<nplanes, 1024, 0, s>>>(planes, sel);
+  k_sel_collect<<<chunks, 256, 0, s>>>(planes, st, sel, keys);
+  k_sel_final<<<nplanes, 1024, 0, s>>>(planes, sel, keys, median);
+}
 void launch_prewitt(const Img *imgs, const Img *mag, const Img *dir, int nimg, long maxn, hipStream_t s) {
   k_prewitt<<<dim3((maxn + 255) / 256, nimg), 256, 0, s>>>(imgs, mag, dir);
 }
 
-void launch_edge_final(const Img *mag, const Img *dir, const Stats *st2, const double *medians, OutRef o, int nimg,
-                       hipStream_t s) {
-  k_edge_final<<<nimg, 256, 0, s>>>(mag, dir, st2, medians, o);
+void launch_edge_final(const Img *mag, const Img *dir, const Stats *st2, const double *medians, EdgeCounts *cnt, OutRef o,
+                       int nimg, long maxn, hipStream_t s) {
+  launch_fill_int((int *)cnt, (long)nimg * (long)(sizeof(EdgeCounts) / sizeof(int)), 0, s);
+  k_edge_count<<<dim3((unsigned)((maxn + SEL_CHUNK - 1) / SEL_CHUNK), nimg), 256, 0, s>>>(mag, dir, st2, cnt);
+  k_edge_final<<<nimg, 64, 0, s>>>(cnt, st2, medians, o);
 }
 
 // ======================================================================= Gabor

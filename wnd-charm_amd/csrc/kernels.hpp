@@ -130,7 +130,7 @@ void launch_cheb_gemm(const GemmDesc *d, int nimg, int maxM, int maxN, hipStream
 void launch_fft(const Img *in, double2 *const *f1, const FftPlan *plw, const FftPlan *plh, const Img *out, int nimg,
                 int maxh, int maxw, hipStream_t s);
 void launch_sort(const Img *imgs, uint64_t *const *buf, const long *cap, int nimg, hipStream_t s);
-void launch_median_gini(const Img *imgs, uint64_t *const *buf, const Stats *st, double *median_out, OutRef pix,
+void launch_median_gini(const Img *imgs, uint64_t *const *buf, const Stats *st, OutRef pix,
                         OutRef gini, int nimg, hipStream_t s);
 void launch_msh(const Img *imgs, const Stats *st, OutRef o, int nimg, hipStream_t s);
 void launch_fractal(const Img *imgs, OutRef o, int nimg, int maxh, int maxw, hipStream_t s);
@@ -172,7 +172,14 @@ void launch_radon_certified(const Img *imgs, const double *trig, double *const *
                             double slack, hipStream_t s);
 
 // objects / edges / gabor / zernike / chebyshev-fourier (k_objects.hip, k_spectral.hip)
+struct ObjState {  // per image
+  int hist[1024];
+  double mn, mx, thr;                  // range of the plane, Otsu threshold
+  long long xm, ym, mass, c1, c3;      // sums over the mask; Euler patterns
+};
 struct ObjDesc {
+  ObjState *state;
+  int *chunk;            // [obj_chunks(n)] roots per block, then their prefix
   int *label;            // [n]
   int *area;             // [n+1] per label
   long long *xm, *ym;    // [n+1]
@@ -180,11 +187,23 @@ struct ObjDesc {
   double *dist;          // [n+1]
   int *count;            // [1]
 };
-void launch_objects(const Img *imgs, const Stats *st, int invert, const ObjDesc *od, OutRef o, int nimg, int maxn,
-                    hipStream_t s);
+int obj_strips(int h, int w);  // strips of rows of an image
+int obj_chunks(long n);        // blocks of pixels
+void launch_objects(const Img *imgs, const Stats *st, int invert, const ObjDesc *od, OutRef o, int nimg, long maxn,
+                    int maxstrips, hipStream_t s);
 void launch_prewitt(const Img *imgs, const Img *mag, const Img *dir, int nimg, long maxn, hipStream_t s);
-void launch_edge_final(const Img *mag, const Img *dir, const Stats *st2, const double *medians, OutRef o, int nimg,
-                       hipStream_t s);
+// median of each plane by counting and selection; keys: room for all of a plane's keys
+constexpr int SEL_BINS = 4096, SEL_CHUNK = 8192;
+struct SelState {
+  int hist[SEL_BINS];
+  int lo, hi, rank, count;   // bins of the middle ranks, the first one's rank within them, keys collected
+  uint64_t kmin, kmax;       // extremes of the collected keys
+};
+void launch_median(const Img *planes, const Stats *st, SelState *sel, uint64_t *const *keys, double *median, int nplanes,
+                   long maxn, hipStream_t s);
+struct EdgeCounts { int area, hm[8], hd[8]; };
+void launch_edge_final(const Img *mag, const Img *dir, const Stats *st2, const double *medians, EdgeCounts *cnt, OutRef o,
+                       int nimg, long maxn, hipStream_t s);
 void launch_gabor_post(const Img *imgs, double *const *energy, OutRef o, int nimg, hipStream_t s);
 // reduced-precision contractions (k_mixed.hip): precision 1 = FP32, 2 = BF16x3 on MFMA.
 // Gabor: FP32 takes float kernels (k0); BF16x3 takes the hi / mid / lo bf16
