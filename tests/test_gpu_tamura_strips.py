@@ -1,0 +1,45 @@
+"""GPU: Tamura textures where the summed-area table's strips and the pixel runs meet.
+
+The table is formed in strips of 64 rows, eight at once, in groups of 16
+columns; pixels are taken in runs of 64 columns x 8 rows and their histograms
+in blocks of 16,384.  Planes just below, at and above these sizes against the
+oracle.  Best scales and phi go through histograms, whose counts are whole
+numbers: a wrong table entry moves a count, i.e. a result by more than 1 / P.
+The rest are sums of P terms in another order, P * 2^-53 < 1e-9 apart."""
+import numpy as np
+import pytest
+
+import wndcharm
+from helpers import ALG_NAMES, orc_algorithm
+
+pytestmark = pytest.mark.gpu
+ALG = 'Tamura Textures'
+
+
+def check(img):
+    got = np.asarray(wndcharm.FeatureAlgorithm(ALG).execute(img))
+    want = orc_algorithm(ALG_NAMES.index(ALG), np.asarray(img, np.float64))
+    assert np.allclose(got, want, rtol=1e-9, atol=1e-12, equal_nan=True), (img.shape, got, want)
+
+
+# one strip and less, runs and groups cut short, eight strips, a wave's second
+# strip where it follows after 41 groups (narrow) and after all groups (wide)
+@pytest.mark.parametrize('shape', [(16, 16), (16, 64), (17, 65), (63, 17), (64, 64), (65, 63), (64, 256), (129, 128), (128, 129),
+                                   (511, 40), (512, 17), (513, 33), (577, 593), (576, 594), (1100, 61), (1030, 700)])
+def test_strips_and_runs(shape):
+    print('tamura', shape, flush=True)
+    rng = np.random.default_rng(sum(shape))
+    y, x = np.mgrid[0:shape[0], 0:shape[1]]
+    check(np.round(900 + 300 * np.sin(x / 5.0 + y / 11.0)) + rng.integers(0, 400, shape))
+
+
+@pytest.mark.parametrize('kind', ['flat', 'step', 'negative', 'tiny', 'float32'])
+def test_values(kind):
+    """all equal; two values; a negative maximum; differences near the smallest double; 24-bit values"""
+    print('tamura', kind, flush=True)
+    rng = np.random.default_rng(5)
+    noise = rng.normal(0, 1, (70, 150))
+    img = {'flat': np.full((70, 150), 7.0), 'step': np.where(np.arange(150) < 70, 10.0, 200.0) * np.ones((70, 1)),
+           'negative': noise - 50, 'tiny': 1.0 + np.round(noise) * 2.0 ** -52,
+           'float32': noise.astype(np.float32).astype(np.float64) + 9}[kind]
+    check(img)

@@ -1141,7 +1141,7 @@ static int build_batch(wndgpu_ctx *c, const wndgpu_plan *plan, const Batch &B, A
       case A_TAMURA: {
         std::vector<double *> sc(ne);
         for (int k = 0; k < ne; k++)
-          sc[k] = A.dalloc_n<double>(5 * (size_t)E[k].N->h[E[k].i] * E[k].N->w[E[k].i] + 8);
+          sc[k] = A.dalloc_n<double>(tamura_scratch(E[k].N->h[E[k].i], E[k].N->w[E[k].i]));
         double **scd = A.stage(sc);
         push(gn, [=](hipStream_t s) { gather(s); launch_tamura(ni, nst, scd, o, ne, mh, mw, s); });
       } break;

@@ -2378,9 +2378,7 @@ void launch_haralick_final(const HarDesc *hd, OutRef o, int nimg, hipStream_t s)
 }
 
 // ======================================================================= Tamura
-// tamura.cpp:10-299.  scratch per image (5P doubles): [0, P) normalised
-// plane, [P, 2P) summed-area table (laufendeSumme), [2P, 3P) phi,
-// [3P, 4P) per-pixel sum_r terms, [4P, 4.5P) best coarseness scale (int).
+// tamura.cpp:10-299.  The scratch's layout is given at tam_summary.
 // (x - min) / max per pixel; planes are 256-byte aligned (arena), so each
 // thread streams two double pairs through the global address space
 typedef double tam_d2 __attribute__((ext_vector_type(2)));
@@ -2406,220 +2404,423 @@ __global__ void __launch_bounds__(256) k_tam_norm(const Img *imgs, const Stats *
   }
 }
 
-// summed-area table with the reference's exact recurrence
+// the value of the lane below (lane - 1); lane 0 takes `first`
+__device__ __forceinline__ double from_lane_below(double v, double first) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(first), __double2loint(v), 0x138, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(first), __double2hiint(v), 0x138, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+// Sums over a plane that the directionality and contrast need, by wave of
+// k_tam_pix (64 columns x TAM_ROWS rows), then by block of k_tam_hist
+struct TamPart { double s, sr, pmn, pmx; int ks, kmask; };
+struct TamPart2 { double m2, m4; };
+struct TamSum { double mean, sr, pmn, pmx; long long ks; int kmn, kmx; int hk[3], hd[125]; };
+constexpr int TAM_ROWS = 8, TAM_CHUNK = 16384;
+static_assert(sizeof(TamPart) % 8 == 0 && sizeof(TamPart2) % 8 == 0, "parts are laid out in doubles");
+// scratch of a plane of P pixels, in doubles: [0, P) normalised plane, [P, 2P)
+// row differences and [3P, 4P) corner differences of the summed-area table,
+// [2P, 3P) phi, [4P, 4.5P) best scale (int), then the summary, the parts of
+// k_tam_pix and of k_tam_hist and a row of the table
+__host__ __device__ inline size_t tam_summary(long P) { return 4 * (size_t)P + ((size_t)P + 1) / 2; }
+__host__ __device__ inline size_t tam_parts(long P) { return tam_summary(P) + (sizeof(TamSum) + 7) / 8; }
+__host__ __device__ inline int tam_runs(int h, int w) { return ((w + 63) / 64) * ((h + TAM_ROWS - 1) / TAM_ROWS); }
+__host__ __device__ inline size_t tam_parts2(int h, int w) {
+  return tam_parts((long)h * w) + (size_t)tam_runs(h, w) * (sizeof(TamPart) / 8);
+}
+__host__ __device__ inline size_t tam_row(int h, int w) {
+  return tam_parts2(h, w) + ((size_t)h * w + TAM_CHUNK - 1) / TAM_CHUNK * (sizeof(TamPart2) / 8);
+}
+size_t tamura_scratch(int h, int w) { return tam_row(h, w) + w + 8; }
+
+// Summed-area table with the reference's exact recurrence
 //   S(y,x) = ((I(y,x) + S(y,x-1)) + S(y-1,x)) - S(y-1,x-1)
-// evaluated as an anti-diagonal wavefront: one wave per image, lane l owns
-// row y0+l of a 64-row strip, the value above comes from lane l-1.
-__global__ void __launch_bounds__(64) k_tam_sat(const Img *imgs, double *const *scr) {
-  extern __shared__ double rowbuf[];
+// and from it what k_tam_pix reads: R = S(y,x) - S(y,x-1) and
+// D = S(y,x) - S(y,x-1) - S(y-1,x) + S(y-1,x-1), with zeros outside the plane.
+//
+// An anti-diagonal wavefront: lane l of a wave owns row y0 + l of a 64-row
+// strip and is l columns behind lane 0; the value above comes from lane l - 1.
+// The chain is three additions and a lane shift per step, so a plane's strips
+// run at once: strip s belongs to wave s % nw and starts LAG = 5 groups of 16
+// steps behind strip s - 1, whose last row it takes from a ring of 64 values.
+// A wave's next strip begins T groups after its last, T >= 5 nw + 1, and what
+// wave 0 takes from the strip before it passes through a row in memory.  A
+// group's 64 x 16 inputs and results pass through an LDS tile, so that 16 lanes
+// access 128 consecutive bytes of a row.  Three planes of 1388 x 1040 and their
+// transforms (18 planes): 1.2 ms, 9.0 ms with one wave per plane that met at
+// two barriers per step; 4,800 planes of up to 256 x 256 (7.6 GB moved): 3.0 ms.
+constexpr int SAT_WAVES = 8;
+__global__ void __launch_bounds__(64 * SAT_WAVES) k_tam_sat(const Img *imgs, double *const *scr) {
+  constexpr int GR = 16, LAG = 5;
+  __shared__ double tiles[SAT_WAVES][64 * (GR + 1)];
+  __shared__ double rings[SAT_WAVES][64];
   const Img im = imgs[blockIdx.x];
   const int H = im.h, W = im.w;
   const long P = (long)H * W;
-  // global, not FLAT: the LDS waits of each step leave the prefetched
-  // inputs in flight
-  const gptr<const double> I = to_global((const double *)scr[blockIdx.x]);
-  const gptr<double> S = to_global(scr[blockIdx.x] + P);
-  const int l = threadIdx.x;
-  constexpr int PF = 16;  // inputs loaded ahead per lane
-  for (int y0 = 0; y0 < H; y0 += 64) {
-    const int y = y0 + l;
-    const gptr<const double> Irow = I + (long)y * W;
-    double cur = 0, up_prev = 0;
-    double nx[PF];
+  const gptr<double> N = to_global(scr[blockIdx.x]);
+  const gptr<const double> I = (gptr<const double>)N;
+  const gptr<double> R = N + P, D = N + 3 * P, last = N + tam_row(H, W);
+  const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+  double *const tile = tiles[w], *const ring = rings[w];  // ring: the row above this wave's strip
+  double *const below = rings[w + 1 < nw ? w + 1 : 0];
+  const int G = (W + 63 + GR - 1) / GR, T = max(G, LAG * nw + 1);
+  const int strips = (H + 63) / 64;
+  const int rounds = (strips - 1) / nw * T + LAG * ((strips - 1) % nw) + G;
+  const int lr = l >> 4, lc = l & 15;
+  double nx[GR], nup = 0.0;
+  // inputs of group g of strip st (and of the row above, where it is in memory)
+  auto fetch = [&](int st, int g) {
+    const int y0 = st * 64;
 #pragma unroll
-    for (int k = 0; k < PF; k++) {
-      const int x = k - l;
-      nx[k] = (y < H && x >= 0 && x < W) ? Irow[x] : 0.0;
+    for (int k = 0; k < GR; k++) {
+      const int r = 4 * k + lr, y = y0 + r, x = g * GR - r + lc;
+      nx[k] = (y < H && (unsigned)x < (unsigned)W) ? I[(long)y * W + x] : 0.0;
     }
-    for (int t0 = 0; t0 < W + 63; t0 += PF) {
-      double in[PF];
-#pragma unroll
-      for (int k = 0; k < PF; k++) in[k] = nx[k];
-#pragma unroll
-      for (int k = 0; k < PF; k++) {  // the next group's inputs, in flight during this group
-        const int x = t0 + PF + k - l;
-        nx[k] = (y < H && x >= 0 && x < W) ? Irow[x] : 0.0;
+    if (w == 0) {
+      const int x = g * GR + lc;
+      nup = (st > 0 && x < W) ? last[x] : 0.0;
+    }
+  };
+  double cur = 0, up_prev = 0;
+  for (int r = 0; r < rounds; r++) {
+    const int q = r - LAG * w;             // rounds since this wave's first strip began
+    const int pass = q >= 0 ? q / T : 0, g = q - pass * T;
+    const int st = pass * nw + w;
+    if (q >= 0 && g < G && st < strips) {  // uniform over the wave
+      if (g == 0) {
+        fetch(st, 0);
+        cur = up_prev = 0;
       }
 #pragma unroll
-      for (int k = 0; k < PF; k++) {
-        const int t = t0 + k;
-        if (t >= W + 63) break;
-        const int x = t - l;
-        const double from_left_lane = __shfl_up(cur, 1, 64);
-        double up;
-        if (l == 0) up = (y0 == 0 || x < 0 || x >= W) ? 0.0 : rowbuf[x];
-        else up = (y < 1) ? 0.0 : from_left_lane;
-        if (x >= 0 && x < W && y < H) {
-          const double links = x < 1 ? 0.0 : cur;
-          const double oben = y < 1 ? 0.0 : up;
-          const double obenlinks = (y < 1 || x < 1) ? 0.0 : up_prev;
-          const double v = in[k] + links + oben - obenlinks;
-          S[(long)y * W + x] = v;
-          cur = v;
-          up_prev = up;
+      for (int k = 0; k < GR; k++) tile[(4 * k + lr) * (GR + 1) + lc] = nx[k];
+      if (w == 0 && l < GR) ring[(q * GR + l) & 63] = nup;
+      if (g + 1 < G) fetch(st, g + 1);     // in flight during this group
+      wave_sync();
+      double v[GR], up0[GR], d[GR];
+#pragma unroll
+      for (int k = 0; k < GR; k++) {
+        v[k] = tile[l * (GR + 1) + k];
+        up0[k] = ring[(q * GR + k) & 63];
+      }
+      wave_sync();
+#pragma unroll
+      for (int k = 0; k < GR; k++) {       // columns left of the plane stay zero, those right of it are not stored
+        const double up = from_lane_below(cur, up0[k]);
+        const double s = v[k] + cur + up - up_prev;
+        v[k] = s;
+        d[k] = s - cur;
+        tile[l * (GR + 1) + k] = d[k];
+        d[k] = d[k] - up + up_prev;
+        cur = s;
+        up_prev = up;
+      }
+      if (l == 63) {                       // the strip's last row, by the round: a wave's strips follow on
+        if (w + 1 < nw) {
+#pragma unroll
+          for (int k = 0; k < GR; k++) below[(q * GR + k - 63) & 63] = v[k];
+        } else if (st + 1 < strips) {
+#pragma unroll
+          for (int k = 0; k < GR; k++) {
+            const int x = g * GR + k - 63;
+            if ((unsigned)x < (unsigned)W) last[x] = v[k];
+          }
         }
-        __syncthreads();
-        if (l == 63 && x >= 0 && x < W) rowbuf[x] = cur;
-        __syncthreads();
       }
+      auto store = [&](gptr<double> to) {
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < GR; k++) {
+          const int rr = 4 * k + lr, y = st * 64 + rr, x = g * GR - rr + lc;
+          const double o = tile[rr * (GR + 1) + lc];
+          if (y < H && (unsigned)x < (unsigned)W) to[(long)y * W + x] = o;
+        }
+        wave_sync();
+      };
+      store(R);
+#pragma unroll
+      for (int k = 0; k < GR; k++) tile[l * (GR + 1) + k] = d[k];
+      store(D);
     }
+    __syncthreads();
   }
 }
 
-// The window's pixel count is a power of two 2^e away from the borders;
-// there the quotient is formed as a product with 2^-e, which is exact, so
-// both are the correctly rounded value of the same real number.
-__device__ __forceinline__ double local_mean(int x, int y, int k, gptr<const double> S, int dimx, int dimy) {
-  const int k2 = k / 2;
-  int starty = y - k2, startx = x - k2, stopy = y + k2 - 1, stopx = x + k2 - 1;
-  if (starty < 0) starty = 0;
-  if (startx < 0) startx = 0;
-  if (stopx > dimx - 1) stopx = dimx - 1;
-  if (stopy > dimy - 1) stopy = dimy - 1;
-  const long r1 = (long)stopy * dimx, r0 = r1 - dimx;
-  const double links = (startx - 1 < 0) ? 0 : S[r1 + startx - 1];
-  const double oben = (starty - 1 < 0) ? 0 : S[r0 + startx];
-  const double obenlinks = ((starty - 1 < 0) || (startx - 1 < 0)) ? 0 : S[r0 + startx - 1];
-  const double unten = S[r1 + startx];
-  const int counter = (stopy - starty + 1) * (stopx - startx + 1);
-  const double num = unten - links - oben + obenlinks;
-  if ((counter & (counter - 1)) == 0) {
-    const int e = __builtin_ctz((unsigned)counter);
-    return num * __longlong_as_double((long long)(1023 - e) << 52);  // 2^-e
-  }
-  return num / counter;
+// |a0 / c0 - a1 / c1| for whole numbers c <= 2^14 and r within a few units in
+// the last place of 1 / c.  A quotient is the product with r with the
+// remainder's quotient added, which rounds as the division does because a / c is
+// nowhere nearer than 1 / (2c) units in the last place to the middle between two
+// doubles; an infinite a, whose remainder is no number, is its own quotient.
+__device__ __forceinline__ double mean_diff(double a0, double c0, double r0, double a1, double c1, double r1) {
+  const double q0 = a0 * r0, q1 = a1 * r1;
+  const double m0 = __builtin_fma(__builtin_fma(-c0, q0, a0), r0, q0);
+  const double m1 = __builtin_fma(__builtin_fma(-c1, q1, a1), r1, q1);
+  double v = fabs(m0 - m1);
+  if (__any(v != v)) v = fabs((__builtin_isinf(a0) ? a0 : m0) - (__builtin_isinf(a1) ? a1 : m1));
+  return v;
 }
 
-// coarseness per pixel (best scale), directionality phi and the sums
-struct TamAcc {
-  double sum_r, m2, m4, mean;
-  long long ksum;
-  int kmin, kmax;
-};
-
-__global__ void __launch_bounds__(256) k_tam_pix(const Img *imgs, double *const *scr, int nimg, int per_img) {
+// Coarseness per pixel (best scale), directionality phi and the sums.
+//
+// The reference's window mean (efficientLocalMean, tamura.cpp) takes its four
+// table entries from two adjacent rows and columns: stop row and the row above,
+// start column and the one to its left.  Its numerator is thus an entry of D at
+// (stop row, start column), of R where the window starts in row 0: one load.
+// Its divisor is full, a power of two, away from the borders.
+//
+// Bound by instruction issue, so a wave takes 64 columns and goes down TAM_ROWS
+// rows: what depends on the row alone is scalar, and the rows' neighbours stay in
+// registers.  4,800 planes of up to 256 x 256: 9.9 ms; 18.0 ms with four table
+// entries per mean, 12.9 ms with one thread per pixel.
+__global__ void __launch_bounds__(256, 3) k_tam_pix(const Img *imgs, double *const *scr, int nimg, int per_img) {
+  __shared__ double recip[129];
   int ent, blk;
-  if (!xcd_item(per_img, nimg, ent, blk)) return;  // one plane's SAT stays in one L2
+  if (!xcd_item(per_img, nimg, ent, blk)) return;  // one plane's tables stay in one L2
+  if (threadIdx.x < 129) recip[threadIdx.x] = 1.0 / threadIdx.x;
+  __syncthreads();
   const Img im = imgs[ent];
   const int H = im.h, W = im.w;
   const long P = (long)H * W;
-  const long i = blk * (long)blockDim.x + threadIdx.x;
-  if (i >= P) return;
+  const int run = __builtin_amdgcn_readfirstlane(blk * 4 + (threadIdx.x >> 6));
+  if (run >= tam_runs(H, W)) return;
+  const int nc = (W + 63) / 64, y0 = run / nc * TAM_ROWS, x0 = run % nc * 64 + (threadIdx.x & 63);
+  const bool own = x0 < W;
+  const int x = min(x0, W - 1);
   const gptr<double> N = to_global(scr[ent]);  // global, not FLAT: vector-memory waits only
-  const gptr<const double> S = (gptr<const double>)(N + P);
-  const gptr<double> phi = N + 2 * P;
-  const int y = i / W, x = i - (long)y * W;
-  // coarseness: argmax over scales of E_h / E_v (tamura.cpp:183-238)
-  double maxE = 0;
-  int maxk = 0;
-  int len = 1;
-  for (int k = 1; k <= 7; ++k) {
-    const int k2 = len;
-    len *= 2;
-    double eh = 0, ev = 0;
-    if (x + k2 < W && x - k2 >= 0)
-      eh = fabs(local_mean(x + k2, y, len, S, W, H) - local_mean(x - k2, y, len, S, W, H));
-    if (y + k2 < H && y - k2 >= 0)
-      ev = fabs(local_mean(x, y + k2, len, S, W, H) - local_mean(x, y - k2, len, S, W, H));
-    if (eh > maxE) { maxE = eh; maxk = k; }
-    if (ev > maxE) { maxE = ev; maxk = k; }
+  const gptr<const double> Nc = (gptr<const double>)N, R = Nc + P, D = Nc + 3 * P;
+  const double ctl = x, ctr = W - x;  // widths of the windows beside it where the border cuts them
+  const double rtl = recip[min(x, 128)], rtr = recip[min(W - x, 128)];
+  const bool xm = x >= 1, xp = x + 1 < W;
+  const unsigned xl = max(x - 1, 0), xr = min(x + 1, W - 1);
+  // rows y - 1 and y of the normalised plane around column x
+  double a0 = 0, a1 = 0, a2 = 0, b0, b1, b2;
+  if (y0 >= 1) {
+    const gptr<const double> q = Nc + (long)(y0 - 1) * W;
+    a0 = xm ? q[xl] : 0.0;
+    a1 = q[(unsigned)x];
+    a2 = xp ? q[xr] : 0.0;
   }
-  ((gptr<int>)(N + 4 * P))[i] = maxk;
-  // directionality filters after the reference's assignments (tamura.cpp:50-57):
-  // H = [-1 2 1; -2 0 2; -1 -2 -1], V = [1 0 0; 0 0 0; -1 0 0], correlation order
-  // (column offset outer, row offset inner), zero weights skipped (exact).
-  auto px = [&](int yy, int xx) -> double { return N[(long)yy * W + xx]; };
-  double dh = 0.0, dv = 0.0;
-  const bool xm = x - 1 >= 0, xp = x + 1 < W, ym = y - 1 >= 0, yp = y + 1 < H;
-  if (xm) {
-    if (ym) dh += -1 * px(y - 1, x - 1);
-    dh += -2 * px(y, x - 1);
-    if (yp) dh += -1 * px(y + 1, x - 1);
+  {
+    const gptr<const double> q = Nc + (long)y0 * W;
+    b0 = xm ? q[xl] : 0.0;
+    b1 = q[(unsigned)x];
+    b2 = xp ? q[xr] : 0.0;
   }
-  if (ym) dh += 2 * px(y - 1, x);
-  if (yp) dh += -2 * px(y + 1, x);
-  if (xp) {
-    if (ym) dh += 1 * px(y - 1, x + 1);
-    dh += 2 * px(y, x + 1);
-    if (yp) dh += -1 * px(y + 1, x + 1);
+  TamPart T = {0, 0, 1e308, -1e308, 0, 0};
+#pragma unroll 1
+  for (int y = y0; y < min(y0 + TAM_ROWS, H); y++) {
+    int xi = x;
+    __asm__ volatile("" : "+v"(xi));  // formed anew per row: registers held through the loop cost more waves
+    // coarseness: argmax over scales of E_h / E_v (tamura.cpp:183-238); the four
+    // windows of each scale, all loads in flight
+    double d[7][4], c0 = 0, c1 = 0, c2 = 0;
+#pragma unroll
+    for (int k = 0; k < 7; k++) {
+      const int k2 = 1 << k;
+      const gptr<const double> h = (y <= k2 ? R : D) + (long)min(y + k2 - 1, H - 1) * W;
+      const gptr<const double> v0 = D + (long)min(y + 2 * k2 - 1, H - 1) * W;  // y >= k2: starts in row y
+      const gptr<const double> v1 = (y <= 2 * k2 ? R : D) + (long)max(y - 1, 0) * W;
+      d[k][0] = h[(unsigned)xi];
+      d[k][1] = h[(unsigned)max(xi - 2 * k2, 0)];
+      d[k][2] = v0[(unsigned)max(xi - k2, 0)];
+      d[k][3] = v1[(unsigned)max(xi - k2, 0)];
+    }
+    if (y + 1 < H) {
+      const gptr<const double> q = Nc + (long)(y + 1) * W;
+      c0 = xm ? q[xl] : 0.0;
+      c1 = q[(unsigned)xi];
+      c2 = xp ? q[xr] : 0.0;
+    }
+    double maxE = 0;
+    int maxk = 0;
+#pragma unroll
+    for (int k = 0; k < 7; k++) {
+      const int k2 = 1 << k;
+      const double full = 1.0 / (4 * k2 * k2);  // a power of two: the product is the quotient
+      const bool okh = xi + k2 < W && xi - k2 >= 0;
+      double eh = 0, ev = 0;
+      if (__any(okh)) {
+        const int n = min(y + k2, H) - max(y - k2, 0);
+        const bool cl = xi < 2 * k2, cr = W - xi < 2 * k2;
+        if (n == 2 * k2 && !__any(okh && (cl || cr))) {
+          eh = fabs(d[k][0] * full - d[k][1] * full);
+        } else {
+          const double r = recip[n], c = n;
+          eh = mean_diff(d[k][0], c * (cr ? ctr : 2.0 * k2), r * (cr ? rtr : 0.5 / k2), d[k][1],
+                         c * (cl ? ctl : 2.0 * k2), r * (cl ? rtl : 0.5 / k2));
+        }
+        eh = okh ? eh : 0.0;
+      }
+      if (y + k2 < H && y - k2 >= 0) {
+        const int n0 = min(2 * k2, H - y), n1 = min(2 * k2, y), wc = min(xi + k2, W) - max(xi - k2, 0);
+        if (n0 == 2 * k2 && n1 == 2 * k2 && __all(wc == 2 * k2)) {
+          ev = fabs(d[k][2] * full - d[k][3] * full);
+        } else {
+          const double r = recip[wc], c = wc;
+          ev = mean_diff(d[k][2], n0 * c, recip[n0] * r, d[k][3], n1 * c, recip[n1] * r);
+        }
+      }
+      if (eh > maxE) { maxE = eh; maxk = k + 1; }
+      if (ev > maxE) { maxE = ev; maxk = k + 1; }
+    }
+    // directionality filters after the reference's assignments (tamura.cpp:50-57):
+    // H = [-1 2 1; -2 0 2; -1 -2 -1], V = [1 0 0; 0 0 0; -1 0 0], correlation order
+    // (column offset outer, row offset inner), zero weights skipped (exact); what
+    // lies outside the plane is zero, and adding it changes nothing
+    double dh = 0.0, dv = 0.0;
+    dh += -1 * a0;
+    dh += -2 * b0;
+    dh += -1 * c0;
+    dh += 2 * a1;
+    dh += -2 * c1;
+    dh += 1 * a2;
+    dh += 2 * b2;
+    dh += -1 * c2;
+    dv += 1 * a0;
+    dv += -1 * c0;
+    double ph = 0.0;
+    if (dh >= 0.0001) ph = atan(dv / dh) + (M_PI / 2.0 + 0.001);
+    if (own) {
+      const unsigned i = (unsigned)y * (unsigned)W + (unsigned)x;
+      ((gptr<int>)(N + 4 * P))[i] = maxk;
+      (N + 2 * P)[i] = ph;
+      T.s += b1;
+      if (dh >= 0.0001) T.sr += (dh * dh + dv * dv) + ph * ph;
+      T.ks += maxk;
+    }
+    T.kmask |= 1 << maxk;
+    T.pmn = fmin(T.pmn, ph);
+    T.pmx = fmax(T.pmx, ph);
+    a0 = b0; a1 = b1; a2 = b2;
+    b0 = c0; b1 = c1; b2 = c2;
   }
-  if (xm) {
-    if (ym) dv += 1 * px(y - 1, x - 1);
-    if (yp) dv += -1 * px(y + 1, x - 1);
+  for (int o = 32; o > 0; o >>= 1) {
+    T.s += __shfl_down(T.s, o, 64);
+    T.sr += __shfl_down(T.sr, o, 64);
+    T.pmn = fmin(T.pmn, __shfl_down(T.pmn, o, 64));
+    T.pmx = fmax(T.pmx, __shfl_down(T.pmx, o, 64));
+    T.ks += __shfl_down(T.ks, o, 64);
+    T.kmask |= __shfl_down(T.kmask, o, 64);
   }
-  double ph = 0.0;
-  if (dh >= 0.0001) ph = atan(dv / dh) + (M_PI / 2.0 + 0.001);
-  phi[i] = ph;
-  N[3 * P + i] = (dh >= 0.0001) ? (dh * dh + dv * dv) + ph * ph : 0.0;
+  if ((threadIdx.x & 63) == 0) ((TamPart *)(scr[ent] + tam_parts(P)))[run] = T;
 }
 
-__global__ void __launch_bounds__(1024) k_tam_final(const Img *imgs, double *const *scr, OutRef o) {
+// the plane's sums from its parts; clears the histograms
+__global__ void __launch_bounds__(1024) k_tam_mid(const Img *imgs, double *const *scr) {
   __shared__ double shd[16];
   __shared__ long long shl[16];
-  __shared__ int hk[3];
-  __shared__ int hd[125];
+  __shared__ int shi[16];
   const Img im = imgs[blockIdx.x];
-  const int H = im.h, W = im.w;
-  const long P = (long)H * W;
-  const double *N = scr[blockIdx.x];
-  const double *phi = N + 2 * P;
-  const double *srt = N + 3 * P;
-  const int *kb = (const int *)(N + 4 * P);
-  const int t = threadIdx.x;
-  // contrast: Moments4 of the normalised plane (tamura.cpp:10-28)
-  double s = 0;
-  for (long i = t; i < P; i += blockDim.x) s += N[i];
-  s = block_reduce(s, SumOp(), shd);
-  const double mean = s / P;
-  double m2 = 0, m4 = 0;
-  for (long i = t; i < P; i += blockDim.x) { const double d = N[i] - mean, d2 = d * d; m2 += d2; m4 += d2 * d2; }
-  m2 = block_reduce(m2, SumOp(), shd);
-  m4 = block_reduce(m4, SumOp(), shd);
-  // coarseness sums and min/max of best scale
+  const long P = (long)im.h * im.w;
+  TamSum &T = *(TamSum *)(scr[blockIdx.x] + tam_summary(P));
+  const TamPart *part = (const TamPart *)(scr[blockIdx.x] + tam_parts(P));
+  double s = 0, sr = 0, pmn = 1e308, pmx = -1e308;
   long long ks = 0;
-  int kmn = 99, kmx = -1;
-  double pmn = 1e308, pmx = -1e308, sr = 0;
-  for (long i = t; i < P; i += blockDim.x) {
-    const int k = kb[i];
-    ks += k;
-    kmn = min(kmn, k);
-    kmx = max(kmx, k);
-    pmn = fmin(pmn, phi[i]);
-    pmx = fmax(pmx, phi[i]);
-    sr += srt[i];
+  int km = 0;
+  for (int b = threadIdx.x; b < tam_runs(im.h, im.w); b += 1024) {
+    const TamPart q = part[b];
+    s += q.s;
+    sr += q.sr;
+    pmn = fmin(pmn, q.pmn);
+    pmx = fmax(pmx, q.pmx);
+    ks += q.ks;
+    km |= q.kmask;
   }
-  ks = block_reduce(ks, SumOp(), shl);
-  kmn = (int)block_reduce((long long)kmn, MinOp(), shl);
-  kmx = (int)block_reduce((long long)kmx, MaxOp(), shl);
+  s = block_reduce(s, SumOp(), shd);
+  sr = block_reduce(sr, SumOp(), shd);
   pmn = block_reduce(pmn, MinOp(), shd);
   pmx = block_reduce(pmx, MaxOp(), shd);
-  sr = block_reduce(sr, SumOp(), shd);
-  if (t < 3) hk[t] = 0;
-  if (t < 125) hd[t] = 0;
-  __syncthreads();
-  const double ksc = hist_scale((double)kmn, (double)kmx, 3), psc = hist_scale(pmn, pmx, 125);
-  // the 3-bin coarseness histogram by ballot per wave (counts in scalar
-  // registers, one LDS add per bin and wave); the 125-bin one by LDS atomics
-  int wk0 = 0, wk1 = 0, wk2 = 0;
-  for (long i0 = 0; i0 < P; i0 += blockDim.x) {
-    const long i = i0 + t;
-    const bool ok = i < P;
-    int b = -1;
-    if (ok) {
-      b = hist_bin((double)kb[i], (double)kmn, ksc, 3);
-      atomicAdd(&hd[hist_bin(phi[i], pmn, psc, 125)], 1);
-    }
-    wk0 += __popcll(__ballot(b == 0));
-    wk1 += __popcll(__ballot(b == 1));
-    wk2 += __popcll(__ballot(b == 2));
+  ks = block_reduce(ks, SumOp(), shl);
+  const int kmn = block_reduce(km ? __builtin_ctz(km) : 99, MinOp(), shi);
+  const int kmx = block_reduce(km ? 31 - __builtin_clz(km) : -1, MaxOp(), shi);
+  if (threadIdx.x < 125) T.hd[threadIdx.x] = 0;
+  if (threadIdx.x < 3) T.hk[threadIdx.x] = 0;
+  if (threadIdx.x == 0) {
+    T.mean = s / P;
+    T.sr = sr;
+    T.pmn = pmn;
+    T.pmx = pmx;
+    T.ks = ks;
+    T.kmn = kmn;
+    T.kmx = kmx;
   }
-  if ((t & 63) == 0) {
+}
+
+// contrast moments about the mean (Moments4, tamura.cpp:10-28) and the two
+// histograms, by block of TAM_CHUNK pixels
+__global__ void __launch_bounds__(256) k_tam_hist(const Img *imgs, double *const *scr) {
+  __shared__ double shd[4];
+  __shared__ int hk[3], hd[125];
+  const Img im = imgs[blockIdx.y];
+  const long P = (long)im.h * im.w, c0 = (long)blockIdx.x * TAM_CHUNK;
+  if (c0 >= P) return;
+  const gptr<const double> N = to_global((const double *)scr[blockIdx.y]);
+  const gptr<const double> phi = N + 2 * P;
+  const gptr<const int> kb = (gptr<const int>)(N + 4 * P);
+  TamSum &T = *(TamSum *)(scr[blockIdx.y] + tam_summary(P));
+  const double mean = T.mean, pmn = T.pmn, kmn = T.kmn;
+  const double ksc = hist_scale(kmn, (double)T.kmx, 3), psc = hist_scale(pmn, T.pmx, 125);
+  if (threadIdx.x < 3) hk[threadIdx.x] = 0;
+  if (threadIdx.x < 125) hd[threadIdx.x] = 0;
+  __syncthreads();
+  double m2 = 0, m4 = 0;
+  int wk0 = 0, wk1 = 0, wk2 = 0;
+  for (int r = 0; r < TAM_CHUNK; r += 256 * 4) {
+    double v[4], p[4];
+    int kk[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const long i = min(c0 + r + 256 * k + threadIdx.x, P - 1);
+      v[k] = N[i];
+      p[k] = phi[i];
+      kk[k] = kb[i];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const bool ok = c0 + r + 256 * k + threadIdx.x < P;
+      int b = -1;
+      if (ok) {
+        const double d = v[k] - mean, d2 = d * d;
+        m2 += d2;
+        m4 += d2 * d2;
+        b = hist_bin((double)kk[k], kmn, ksc, 3);
+        atomicAdd(&hd[hist_bin(p[k], pmn, psc, 125)], 1);
+      }
+      wk0 += __popcll(__ballot(b == 0));
+      wk1 += __popcll(__ballot(b == 1));
+      wk2 += __popcll(__ballot(b == 2));
+    }
+  }
+  if ((threadIdx.x & 63) == 0) {
     atomicAdd(&hk[0], wk0);
     atomicAdd(&hk[1], wk1);
     atomicAdd(&hk[2], wk2);
   }
   __syncthreads();
-  if (t == 0) {
+  if (threadIdx.x < 3 && hk[threadIdx.x]) atomicAdd(&T.hk[threadIdx.x], hk[threadIdx.x]);
+  if (threadIdx.x < 125 && hd[threadIdx.x]) atomicAdd(&T.hd[threadIdx.x], hd[threadIdx.x]);
+  m2 = block_reduce(m2, SumOp(), shd);
+  m4 = block_reduce(m4, SumOp(), shd);
+  if (threadIdx.x == 0) ((TamPart2 *)(scr[blockIdx.y] + tam_parts2(im.h, im.w)))[blockIdx.x] = TamPart2{m2, m4};
+}
+
+__global__ void __launch_bounds__(64) k_tam_final(const Img *imgs, double *const *scr, OutRef o) {
+  __shared__ double shd[1];
+  const Img im = imgs[blockIdx.x];
+  const int H = im.h, W = im.w;
+  const long P = (long)H * W;
+  const TamSum &T = *(const TamSum *)(scr[blockIdx.x] + tam_summary(P));
+  const TamPart2 *part = (const TamPart2 *)(scr[blockIdx.x] + tam_parts2(im.h, im.w));
+  double m2 = 0, m4 = 0;
+  for (long b = threadIdx.x; b < (P + TAM_CHUNK - 1) / TAM_CHUNK; b += 64) {
+    m2 += part[b].m2;
+    m4 += part[b].m4;
+  }
+  m2 = block_reduce(m2, SumOp(), shd);
+  m4 = block_reduce(m4, SumOp(), shd);
+  if (threadIdx.x == 0) {
+    const int *hk = T.hk, *hd = T.hd;
+    const long long ks = T.ks;
+    const double sr = T.sr;
     double *out = o.rows[blockIdx.x];
     // coarseness (tamura.cpp:240-262); the divisor is unsigned arithmetic
     const unsigned xD = W, yD = H;
@@ -2653,12 +2854,14 @@ __global__ void __launch_bounds__(1024) k_tam_final(const Img *imgs, double *con
 void launch_tamura(const Img *imgs, const Stats *st, double *const *scratch, OutRef o, int nimg, int maxh, int maxw,
                    hipStream_t s) {
   const long maxn = (long)maxh * maxw;
-  int blocks = (int)((maxn + 255) / 256);
+  const int blocks = (tam_runs(maxh, maxw) + 3) / 4;
   const int nblocks = (int)((maxn / 4 + 255) / 256);
   k_tam_norm<<<dim3(nblocks < 1 ? 1 : (nblocks > 1024 ? 1024 : nblocks), nimg), 256, 0, s>>>(imgs, st, scratch);
-  k_tam_sat<<<nimg, 64, maxw * sizeof(double), s>>>(imgs, scratch);
+  k_tam_sat<<<nimg, 64 * std::min((maxh + 63) / 64, SAT_WAVES), 0, s>>>(imgs, scratch);
   k_tam_pix<<<xcd_grid(blocks, nimg), 256, 0, s>>>(imgs, scratch, nimg, blocks);
-  k_tam_final<<<nimg, 1024, 0, s>>>(imgs, scratch, o);
+  k_tam_mid<<<nimg, 1024, 0, s>>>(imgs, scratch);
+  k_tam_hist<<<dim3((unsigned)((maxn + TAM_CHUNK - 1) / TAM_CHUNK), nimg), 256, 0, s>>>(imgs, scratch);
+  k_tam_final<<<nimg, 64, 0, s>>>(imgs, scratch, o);
 }
 
 // ================================================================= Comb moments

@@ -160,6 +160,7 @@ void launch_haralick_order(const int *ng, int nimg, int *order, hipStream_t s);
 void launch_haralick_hess(const HarDesc *hd, const int *order, int nimg, hipStream_t s);
 void launch_haralick_qr(const HarDesc *hd, const int *order, int nimg, hipStream_t s);
 void launch_haralick_final(const HarDesc *hd, OutRef o, int nimg, hipStream_t s);
+size_t tamura_scratch(int h, int w);  // doubles per plane
 void launch_tamura(const Img *imgs, const Stats *st, double *const *scratch, OutRef o, int nimg, int maxh, int maxw,
                    hipStream_t s);
 void launch_comb(const Img *imgs, const double *iis, OutRef o, int nimg, hipStream_t s);
