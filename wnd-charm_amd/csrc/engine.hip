@@ -305,7 +305,7 @@ struct wndgpu_ctx {
   std::map<std::pair<int, double>, DevTable> dspos;
   std::map<std::tuple<int, double, int>, DevTable> dsdense;  // (len, dx, nout): dense Downsample passes
   std::map<int, DevTable> comb;
-  DevTable gabor, zern, rtrig;
+  DevTable gabor, gabor_fac, zern, rtrig;
   DevTable color_lut;  // fuzzy colour class of every (h, s, v) byte triple, built on first use
   // Size-dependent bases (Chebyshev, Chebyshev-Fourier geometry) take libm
   // calls on the host per new image size: the sizing pass of a batch lists
@@ -1404,13 +1404,13 @@ static int build_batch(wndgpu_ctx *c, const wndgpu_plan *plan, const Batch &B, A
         float **bdd = cert ? A.stage(bd) : nullptr;
         double *gprm = cert ? A.dalloc_n<double>(32 * (size_t)ne) : nullptr;  // per entry: max, min, base count
         int *gflag = cert ? A.dalloc_n<int>(8 * 64 * (size_t)ne) : nullptr;  // per entry and filter: open energies
-        const double *gk = (const double *)c->gabor.p;
+        const double *gk = (const double *)c->gabor.p, *gf = (const double *)c->gabor_fac.p;
         const void *k0 = prec == 1 ? c->gabor_f32.p : c->gabor_bhi.p, *k1 = c->gabor_bmd.p, *k2 = c->gabor_blo.p;
         const double *wsum = (const double *)c->gabor_wsum.p;
         const double gslack = c->gabor_slack;
         push_late(gn, [=](hipStream_t s) {
           if (prec) launch_gabor_mixed(prec, ni, k0, k1, k2, wsum, gk, end_, bdd, gprm, gflag, o, ne, mh, mw, s);
-          else if (cert) launch_gabor_certified(ni, gk, wsum, gslack, end_, bdd, gprm, gflag, o, ne, mh, mw, s);
+          else if (cert) launch_gabor_certified(ni, gk, gf, wsum, gslack, end_, bdd, gprm, gflag, o, ne, mh, mw, s);
           else launch_gabor(ni, gk, end_, o, ne, mh, mw, s);
         });
       } break;
@@ -1461,7 +1461,8 @@ static int build_batch(wndgpu_ctx *c, const wndgpu_plan *plan, const Batch &B, A
 static int ensure_tables(wndgpu_ctx *c) {
   if (c->gabor.p) return 0;
   int r;
-  std::vector<double> g = gabor_kernels(), z = zernike_h(), t = radon_trig();
+  std::vector<double> g = gabor_kernels(), gf = gabor_factors(), z = zernike_h(), t = radon_trig();
+  if ((r = upload(c, c->gabor_fac, gf.data(), gf.size() * sizeof(double)))) return r;
   if ((r = upload(c, c->gabor, g.data(), g.size() * sizeof(double)))) return r;
   if ((r = upload(c, c->zern, z.data(), z.size() * sizeof(double)))) return r;
   if ((r = upload(c, c->rtrig, t.data(), t.size() * sizeof(double)))) return r;
@@ -1854,7 +1855,7 @@ void wndgpu_destroy(wndgpu_ctx *c) {
   for (auto &kv : c->dspos) fr(kv.second);
   for (auto &kv : c->dsdense) fr(kv.second);
   for (auto &kv : c->comb) fr(kv.second);
-  fr(c->gabor); fr(c->zern); fr(c->rtrig);
+  fr(c->gabor); fr(c->gabor_fac); fr(c->zern); fr(c->rtrig);
   fr(c->gabor_f32); fr(c->gabor_bhi); fr(c->gabor_bmd); fr(c->gabor_blo); fr(c->gabor_wsum);
   release_check(hipStreamSynchronize(c->stream), "hipStreamSynchronize");
   if (c->color_lut.p) release_check(hipFree(c->color_lut.p), "hipFree");

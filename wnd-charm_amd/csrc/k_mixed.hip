@@ -31,7 +31,7 @@ __device__ __forceinline__ unsigned bf16_split(float f) {
 
 // ---------------------------------------------------------------- Gabor
 // Both reduced forms write, beside each energy E, an a-priori bound D on
-// |E - E64|, E64 being the FP64 kernel's value (k_gabor_conv_t<false>), so that the
+// |E - E64|, E64 being the FP64 kernel's value (k_gabor_conv), so that the
 // exact post-processing (k_gabor_post_exact) can certify every count:
 //   re, im = sum_{j,i} x w over the 38 x 38 taps, S = sum |x| (|wr| + |wi|)
 //   <= maxwin(|x|) * wsum_f (maxwin: the largest |x| in the pixel's window,

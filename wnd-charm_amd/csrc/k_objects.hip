@@ -823,22 +823,9 @@ void launch_edge_final(const Img *mag, const Img *dir, const Stats *st2, const d
 // a group needs for the thread's 8 outputs are read from LDS once into
 // registers, and every output still adds its taps in the reference's (j, i)
 // order (conv2comp, gabor.cpp:19-52).
-//   CERT = false: separate multiply and add, the reference's rounding.
-//   CERT = true: fused multiply-adds (half the instructions), and beside
-// each energy E an a-priori bound D on its distance from the CERT = false
-// value E64, for k_gabor_post_exact to certify every count (k_gabor_repair
-// recomputes in the CERT = false order each energy a count leaves open).
-// Both sums of a component are within gamma_1444 S of the exact sum,
-// S = sum |x| |w| <= (largest |x| of the block's input tile) x wsum_f, and
-// the two magnitudes round by at most 2u each, so |E - E64| <= 2 gamma_1444
-// S + 4u E: D = coef * tmax * wsum_f + 1e-14 E, coef = 4e-13 (2 gamma_1444
-// = 3.21e-13) times the context's slack, rounded up.
-template <bool CERT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) k_gabor_conv_t(const Img *imgs, const double *kernels, double *const *energy,
-                                                      const double *wsum, float *const *bound, double coef) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) k_gabor_conv(const Img *imgs, const double *kernels, double *const *energy) {
   __shared__ double tile[GB_TR + GB_N - 1][GB_LD];
   __shared__ double2 wk[GB_N * GB_N];
-  __shared__ double shd[4];
   const Img im = imgs[blockIdx.z];
   const int f = blockIdx.y % 8;
   const int tilesx = (im.w + GB_TC - 1) / GB_TC, tilesy = (im.h + GB_TR - 1) / GB_TR;
@@ -848,18 +835,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   const double *K = kernels + (long)f * GB_N * GB_N * 2;
   for (int e = t; e < GB_N * GB_N; e += 256) wk[e] = make_double2(K[2 * e], K[2 * e + 1]);
   // input rows b0-18 .. b0+GB_TR+18, columns a0-18 .. a0+GB_TC+18
-  double tmax = 0.0;
   for (int r = t / 64; r < GB_TR + GB_N - 1; r += 4) {
     const int y = b0 - 18 + r;
     for (int c = t % 64; c < GB_TC + GB_N - 1; c += 64) {
       const int x = a0 - 18 + c;
-      const double v = (y >= 0 && y < im.h && x >= 0 && x < im.w) ? im.p[(long)y * im.w + x] : 0.0;
-      tile[r][c] = v;
-      if (CERT) tmax = fmax(tmax, fabs(v));
+      tile[r][c] = (y >= 0 && y < im.h && x >= 0 && x < im.w) ? im.p[(long)y * im.w + x] : 0.0;
     }
   }
-  if (CERT) tmax = block_reduce(tmax, MaxOp(), shd);  // (synchronises the block)
-  else __syncthreads();
+  __syncthreads();
   const int ty = t / 8, tx = t % 8;
   const int b = b0 + ty, a = a0 + tx * 8;
   double re[8], imv[8];
@@ -885,13 +868,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
           for (int q = 0; q < 8; q++) {
             const double v = u[q - di + 7];
-            if (CERT) {
-              re[q] = fma(v, w.x, re[q]);
-              imv[q] = fma(v, w.y, imv[q]);
-            } else {
-              re[q] += v * w.x;
-              imv[q] += v * w.y;
-            }
+            re[q] += v * w.x;
+            imv[q] += v * w.y;
           }
         }
       }
@@ -901,13 +879,147 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
   if (b < im.h)
 #pragma unroll
     for (int q = 0; q < 8; q++)
-      if (a + q < im.w) {
-        const double e = sqrt(re[q] * re[q] + imv[q] * imv[q]);
-        E[(long)b * im.w + a + q] = e;
-        if (CERT)
-          bound[blockIdx.z][(long)f * im.h * im.w + (long)b * im.w + a + q] =
-              (float)((coef * tmax * wsum[f] + 1e-14 * e) * 1.000001);
+      if (a + q < im.w) E[(long)b * im.w + a + q] = sqrt(re[q] * re[q] + imv[q] * imv[q]);
+}
+
+// The energies E with an a-priori bound D on each one's distance from
+// k_gabor_conv's value E64, for k_gabor_post_exact to certify every count
+// (k_gabor_repair recomputes in k_gabor_conv's order each energy a count leaves
+// open).
+//
+// A filter is, to 4e-16 of the sum of its taps' magnitudes, the sum of two
+// products of a row and a column: w(j, i) = b0(j) a0(i) + b1(j) a1(i), a real and
+// b complex, the second for the filter's angle, which is not quite pi / 2.  So
+// the image is filtered along its rows twice and along its columns with two
+// complex filters: 228 fused multiply-adds per energy (and 1.4 times the first
+// 76, for the rows around the block's) instead of 2,888.
+//
+// Bound: E64's components are within gamma_1445 S of the exact sum, S =
+// sum |x| |w| <= (largest |x| of the block's input tile) x wsum_f; these within
+// (gamma_39 + gamma_80 + 4e-16) (1 + 1e-8) S; the magnitudes round by at most 2u
+// each: |E - E64| <= 1.8e-13 S + 4u E.  D = coef * tmax * wsum_f + 1e-14 E with
+// coef = 4e-13 times the context's slack, rounded up.  Where a block's largest
+// |x| is so small that D would leave float's range, so large that a sum could
+// overflow, or infinite, its energies are the plain sums over the 1,444 taps.
+//
+// A block takes 27 x 64 outputs, i.e. 64 rows of 101 inputs, and `per` filters.
+// Each of 512 threads forms eight adjacent row sums of both kinds from a sliding
+// window of registers, then a wave four rows of 64 energies; the taps are uniform
+// and come through the scalar cache.  400 images of 256 x 256: 6.7 ms, 21.8 ms
+// with 1,444 complex taps per energy; three of 1388 x 1040: 1.2 ms, 4.6 ms.
+#define GS_TR 27
+#define GS_IN (GS_TR + GB_N - 1)
+constexpr int GS_F = 6 * GB_N;  // factors of a filter: a0, a1, re b0, im b0, re b1, im b1
+static_assert(GS_IN == 64, "eight threads per input row");
+__global__ void __launch_bounds__(512) k_gabor_sep(const Img *imgs, const double *__restrict__ factors,
+                                                   const double *__restrict__ kernels, double *const *energy,
+                                                   const double *__restrict__ wsum, float *const *bound, double coef,
+                                                   int per) {
+  __shared__ double tile[GS_IN][GB_LD + 1];
+  __shared__ double rows[2][GS_IN][GB_TC + 1];
+  __shared__ double shd[8];
+  const Img im = imgs[blockIdx.z];
+  const int tilesx = (im.w + GB_TC - 1) / GB_TC, tilesy = (im.h + GS_TR - 1) / GS_TR;
+  if ((int)blockIdx.x >= tilesx * tilesy) return;
+  const int b0 = (blockIdx.x / tilesx) * GS_TR, a0 = (blockIdx.x % tilesx) * GB_TC;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const long plane = (long)im.h * im.w;
+  // input rows b0-18 .. b0+45, columns a0-18 .. a0+82
+  double tmax = 0.0;
+  for (int r = wave; r < GS_IN; r += 8) {
+    const int y = b0 - 18 + r;
+    for (int c = lane; c < GB_TC + GB_N - 1; c += 64) {
+      const int x = a0 - 18 + c;
+      const double v = (y >= 0 && y < im.h && x >= 0 && x < im.w) ? im.p[(long)y * im.w + x] : 0.0;
+      tile[r][c] = v;
+      tmax = fmax(tmax, fabs(v));
+    }
+  }
+  tmax = block_reduce(tmax, MaxOp(), shd);  // (synchronises the block)
+  const bool sized = tmax == 0.0 || (tmax >= 1e-24 && tmax <= 1e290);
+  for (int f = blockIdx.y * per; f < (int)(blockIdx.y + 1) * per; f++) {
+    double *E = energy[blockIdx.z] + f * plane;
+    float *D = bound[blockIdx.z] + f * plane;
+    const double db = coef * tmax * wsum[f];
+    auto put = [&](int y, int x, double re, double imv) {
+      if (y >= im.h || x >= im.w) return;
+      const double e = sqrt(re * re + imv * imv);
+      E[(long)y * im.w + x] = e;
+      D[(long)y * im.w + x] = (float)((db + 1e-14 * e) * 1.000001);
+    };
+    if (!sized) {
+      const double *K = kernels + (long)f * GB_N * GB_N * 2;
+      for (int r = wave; r < GS_TR; r += 8) {
+        double re = 0.0, imv = 0.0;
+        for (int j = 0; j < GB_N; j++)
+          for (int i = 0; i < GB_N; i++) {
+            const double v = tile[r + 37 - j][lane + 37 - i];
+            re = fma(v, K[2 * (j * GB_N + i)], re);
+            imv = fma(v, K[2 * (j * GB_N + i) + 1], imv);
+          }
+        put(b0 + r, a0 + lane, re, imv);
       }
+      continue;
+    }
+    const double *F = factors + f * GS_F;
+    {
+      const int r = t >> 3, c0 = (t & 7) * 8;
+      double h0[8], h1[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) h0[q] = h1[q] = 0.0;
+      // output c0 + q takes tap i from input column c0 + q + 37 - i
+#pragma unroll
+      for (int i0 = 0; i0 < GB_N; i0 += 8) {
+        const int nt = GB_N - i0 < 8 ? GB_N - i0 : 8;
+        double u[15];
+#pragma unroll
+        for (int k = 0; k < 15; k++) u[k] = k >= 8 - nt ? tile[r][c0 + 30 - i0 + k] : 0.0;
+#pragma unroll
+        for (int di = 0; di < nt; di++) {
+          const double w0 = F[i0 + di], w1 = F[GB_N + i0 + di];
+#pragma unroll
+          for (int q = 0; q < 8; q++) {
+            h0[q] = fma(u[q - di + 7], w0, h0[q]);
+            h1[q] = fma(u[q - di + 7], w1, h1[q]);
+          }
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        rows[0][r][c0 + q] = h0[q];
+        rows[1][r][c0 + q] = h1[q];
+      }
+    }
+    __syncthreads();
+    if (wave * 4 < GS_TR) {
+      double re[4] = {0, 0, 0, 0}, imv[4] = {0, 0, 0, 0};
+      const int r0 = wave * 4;  // output r0 + q takes tap j from row r0 + q + 37 - j
+#pragma unroll
+      for (int p = 0; p < 2; p++) {
+        const double *B = F + (2 + 2 * p) * GB_N;
+#pragma unroll
+        for (int j0 = 0; j0 < GB_N; j0 += 8) {
+          const int nt = GB_N - j0 < 8 ? GB_N - j0 : 8;
+          double u[11];
+#pragma unroll
+          for (int k = 0; k < 11; k++) u[k] = k >= 8 - nt ? rows[p][min(r0 + 30 - j0 + k, GS_IN - 1)][lane] : 0.0;
+#pragma unroll
+          for (int dj = 0; dj < nt; dj++) {
+            const double wr = B[j0 + dj], wi = B[GB_N + j0 + dj];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+              re[q] = fma(u[q - dj + 7], wr, re[q]);
+              imv[q] = fma(u[q - dj + 7], wi, imv[q]);
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        if (r0 + q < GS_TR) put(b0 + r0 + q, a0 + lane, re[q], imv[q]);
+    }
+    __syncthreads();  // the next filter's row sums overwrite these
+  }
 }
 
 __global__ void __launch_bounds__(1024) k_gabor_post(const Img *imgs, double *const *energy, OutRef o) {
@@ -953,11 +1065,11 @@ __global__ void __launch_bounds__(1024) k_gabor_post(const Img *imgs, double *co
 }
 
 // The Gabor ratios from energies E with bounds D (|E - E64| <= D, E64 =
-// k_gabor_conv_t<false>'s value: the fused multiply-add, FP32 and BF16
+// k_gabor_conv's value: the fused multiply-add, FP32 and BF16
 // forms), equal to k_gabor_post on the FP64 energies.  Every decision whose
 // interval [E - D, E + D] leaves it open is taken on E64: the pixels
 // concerned are marked (D < 0), and the repairs recompute them in
-// k_gabor_conv_t<false>'s tap order (E = E64, D = 0).  Five phases of
+// k_gabor_conv's tap order (E = E64, D = 0).  Five phases of
 // k_gabor_post_exact, one block per (image, filter), each followed by the
 // repairs except the last:
 //   1  mark the candidates for the maximum (upper end >= largest lower end)
@@ -972,8 +1084,8 @@ __global__ void __launch_bounds__(1024) k_gabor_post(const Img *imgs, double *co
 constexpr int GP_STRIDE = 4;
 
 // the marked pixels (D < 0) of one 32 x 64 tile of one filter's map: the
-// input window staged in LDS as k_gabor_conv_t does, each marked output then
-// summed in k_gabor_conv_t<false>'s tap order by one lane
+// input window staged in LDS as k_gabor_conv does, each marked output then
+// summed in k_gabor_conv's tap order by one lane
 __device__ void gabor_repair_tile(const Img &im, int tile, const double *K, double *E, float *D,
                                   double (*tile_px)[GB_LD], double2 *wk, int *list, int *nlist) {
   const int tilesx = (im.w + GB_TC - 1) / GB_TC;
@@ -1032,7 +1144,7 @@ constexpr int GR_CAP = 63;
 constexpr int GR_STRIDE = GR_CAP + 1;
 // One wavefront per (image, filter); per listed energy the lanes form the
 // 1444 tap products (each rounded once, as in the sum) into LDS, and lane 0
-// adds them in k_gabor_conv_t<false>'s (and the tile repair's) order: tap
+// adds them in k_gabor_conv's (and the tile repair's) order: tap
 // (j, i) reads input (y + 19 - j, x + 19 - i), +0 outside the image.
 __global__ void __launch_bounds__(64) k_gabor_repair_list(const Img *imgs, const double *kernels, double *const *energy,
                                                           float *const *bound, const int *flags) {
@@ -1268,14 +1380,18 @@ void launch_gabor_post_exact(const Img *imgs, double *const *energy, float *cons
 void launch_gabor(const Img *imgs, const double *kernels, double *const *energy, OutRef o, int nimg, int maxh,
                   int maxw, hipStream_t s) {
   const int tiles = ((maxw + GB_TC - 1) / GB_TC) * ((maxh + GB_TR - 1) / GB_TR);
-  k_gabor_conv_t<false><<<dim3(tiles, 8, nimg), 256, 0, s>>>(imgs, kernels, energy, nullptr, nullptr, 0.0);
+  k_gabor_conv<<<dim3(tiles, 8, nimg), 256, 0, s>>>(imgs, kernels, energy);
   k_gabor_post<<<nimg, 1024, 0, s>>>(imgs, energy, o);
 }
-void launch_gabor_certified(const Img *imgs, const double *kernels, const double *wsum, double slack,
-                            double *const *energy, float *const *bound, double *params, int *flags, OutRef o,
-                            int nimg, int maxh, int maxw, hipStream_t s) {
-  const int tiles = ((maxw + GB_TC - 1) / GB_TC) * ((maxh + GB_TR - 1) / GB_TR);
-  k_gabor_conv_t<true><<<dim3(tiles, 8, nimg), 256, 0, s>>>(imgs, kernels, energy, wsum, bound, 4e-13 * slack);
+void launch_gabor_certified(const Img *imgs, const double *kernels, const double *factors, const double *wsum,
+                            double slack, double *const *energy, float *const *bound, double *params, int *flags,
+                            OutRef o, int nimg, int maxh, int maxw, hipStream_t s) {
+  const int tiles = ((maxw + GB_TC - 1) / GB_TC) * ((maxh + GS_TR - 1) / GS_TR);
+  // a CU holds one block: from two blocks per CU on, the input tile is read once
+  // for all filters, below that the filters go to blocks of their own (one image
+  // of 128 x 128: 10 blocks or 80)
+  const int per = (long)tiles * nimg >= 512 ? 8 : 1;
+  k_gabor_sep<<<dim3(tiles, 8 / per, nimg), 512, 0, s>>>(imgs, factors, kernels, energy, wsum, bound, 4e-13 * slack, per);
   launch_gabor_post_exact(imgs, energy, bound, kernels, params, flags, slack <= 1.0, o, nimg, maxh, maxw, s);
 }
 void launch_gabor_post(const Img *imgs, double *const *energy, OutRef o, int nimg, hipStream_t s) {

@@ -222,11 +222,12 @@ void launch_gabor_post_exact(const Img *imgs, double *const *energy, float *cons
                              hipStream_t s);
 void launch_gabor(const Img *imgs, const double *kernels, double *const *energy, OutRef o, int nimg, int maxh,
                   int maxw, hipStream_t s);
-// the plain form's default: FP64 fused multiply-adds with per-energy bounds
+// the plain form's default: FP64 row and column filters (factors: gabor_factors)
+// with per-energy bounds
 // (scaled by slack >= 1), every count certified by the exact post-processing
-void launch_gabor_certified(const Img *imgs, const double *kernels, const double *wsum, double slack,
-                            double *const *energy, float *const *bound, double *params, int *flags, OutRef o,
-                            int nimg, int maxh, int maxw, hipStream_t s);
+void launch_gabor_certified(const Img *imgs, const double *kernels, const double *factors, const double *wsum,
+                            double slack, double *const *energy, float *const *bound, double *params, int *flags,
+                            OutRef o, int nimg, int maxh, int maxw, hipStream_t s);
 void launch_zernike(const Img *imgs, double *partial, int nchunk, const double *htab, OutRef o, int nimg,
                     hipStream_t s, int precision = 0);
 // Chebyshev-Fourier histograms: matrix-core sums certified against an

@@ -137,7 +137,7 @@ std::vector<double> ds_dense(unsigned len, double dx, unsigned nout) {
 
 // Gabor filters (gabor.cpp:103-162), theta = 3.14159265/2, gamma 0.5,
 // sig2lam 0.56, n = 38; index 0: f0 = 0.1, 1..7: f0 = 1..7
-std::vector<double> gabor_kernels() {
+std::vector<double> gabor_kernels(std::vector<double> *sums) {
   const double gamma = 0.5, sig2lam = 0.56, theta = 3.14159265 / 2, fi = 0;
   const int n = 38;
   std::vector<double> all;
@@ -166,6 +166,42 @@ std::vector<double> gabor_kernels() {
     for (int y = 0; y < n; y++)
       for (int x = 0; x < n * 2; x++) G[y * n * 2 + x] = G[y * n * 2 + x] / sum;
     all.insert(all.end(), G.begin(), G.end());
+    if (sums) sums->push_back(sum);
+  }
+  return all;
+}
+
+// Each filter as b0(y) a0(x) + b1(y) a1(x), per filter a0, a1, re b0, im b0,
+// re b1, im b1 of 38 values.  With c, s the cosine and sine of theta,
+//   G = exp(-(x^2 (c^2 + g^2 s^2) + y^2 (s^2 + g^2 c^2) + 2 x y c s (1 - g^2)) / (2 sig^2))
+//       * exp(i f0 (x c + y s)),  c = 1.8e-9,
+// and the two factors that mix x and y or turn the phase with x are expanded to
+// first order in c: 1 + x (i f0 c - y c s (1 - g^2) / sig^2).  What is left out
+// is of order c^2; the sum of |G - b0 a0 - b1 a1| is below 4e-16 of sum |G|.
+std::vector<double> gabor_factors() {
+  const long double gamma = 0.5, theta = 3.14159265 / 2;
+  const int n = 38;
+  const double f0s[8] = {0.1, 1, 2, 3, 4, 5, 6, 7};
+  std::vector<double> sums;
+  gabor_kernels(&sums);
+  std::vector<double> all((size_t)8 * 6 * n);
+  for (int f = 0; f < 8; f++) {
+    const long double f0 = f0s[f], sig = 0.56 * (2 * M_PI / f0s[f]);
+    const long double ct = cos((double)theta), st = sin((double)theta);
+    const long double kap = ct * st * (1 - gamma * gamma) / (sig * sig);
+    double *o = &all[(size_t)f * 6 * n];
+    for (int i = 0; i < n; i++) {
+      const long double x = i - n / 2;
+      const long double a = expl(-x * x * (ct * ct + gamma * gamma * st * st) / (2 * sig * sig));
+      const long double e = expl(-x * x * (st * st + gamma * gamma * ct * ct) / (2 * sig * sig)) / sums[f];
+      const long double re = e * cosl(f0 * st * x), im = e * sinl(f0 * st * x);
+      o[i] = (double)a;
+      o[n + i] = (double)(x * a);
+      o[2 * n + i] = (double)re;
+      o[3 * n + i] = (double)im;
+      o[4 * n + i] = (double)(-kap * x * re - f0 * ct * im);
+      o[5 * n + i] = (double)(-kap * x * im + f0 * ct * re);
+    }
   }
   return all;
 }

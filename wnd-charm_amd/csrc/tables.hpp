@@ -16,7 +16,8 @@ CfTable cf_table(int w, int h);
 
 std::vector<double> ds_positions(unsigned len, double dx);
 std::vector<double> ds_dense(unsigned len, double dx, unsigned nout);
-std::vector<double> gabor_kernels();
+std::vector<double> gabor_kernels(std::vector<double> *sums = nullptr);
+std::vector<double> gabor_factors();
 std::vector<double> zernike_h();
 std::vector<double> radon_trig();
 std::vector<double> comb_offsets(int m);
