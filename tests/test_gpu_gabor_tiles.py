@@ -1,8 +1,8 @@
 """GPU: Gabor energies as sums of two row x column filters, where blocks meet.
 
-A block forms 27 x 64 energies; up to 512 blocks it takes one filter, beyond
+A block forms 27 x 64 energies; below 512 blocks it takes one filter, beyond
 all eight; and where its pixels are outside [1e-24, 1e290] (or infinite) it
-adds the 1,444 taps.  Counts are certified against the reference's sums, so
+adds the 1,444 taps.  The counts are taken over blocks of 8,192 pixels.  They are certified against the reference's sums, so
 every ratio equals the direct path's (WNDGPU_GABOR_DIRECT=1) exactly."""
 import numpy as np
 import pytest
@@ -28,7 +28,7 @@ def image(shape, seed):
     return 40 + 20 * np.sin(y / 3.0 + x / 17.0) + rng.normal(0, 6, shape)
 
 
-@pytest.mark.parametrize('shape', [(16, 16), (26, 63), (27, 64), (28, 65), (54, 128), (55, 129), (300, 70)])
+@pytest.mark.parametrize('shape', [(16, 16), (26, 63), (27, 64), (28, 65), (54, 128), (55, 129), (64, 128), (127, 129), (300, 70)])
 def test_block_edges(shape):
     print('gabor tiles', shape, flush=True)
     check([image(shape, 1), image(shape[::-1], 2)])

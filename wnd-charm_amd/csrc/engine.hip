@@ -1402,15 +1402,15 @@ static int build_batch(wndgpu_ctx *c, const wndgpu_plan *plan, const Batch &B, A
         }
         double **end_ = A.stage(en);
         float **bdd = cert ? A.stage(bd) : nullptr;
-        double *gprm = cert ? A.dalloc_n<double>(32 * (size_t)ne) : nullptr;  // per entry: max, min, base count
+        GaborState *gst = cert ? A.dalloc_n<GaborState>(8 * (size_t)ne) : nullptr;
         int *gflag = cert ? A.dalloc_n<int>(8 * 64 * (size_t)ne) : nullptr;  // per entry and filter: open energies
         const double *gk = (const double *)c->gabor.p, *gf = (const double *)c->gabor_fac.p;
         const void *k0 = prec == 1 ? c->gabor_f32.p : c->gabor_bhi.p, *k1 = c->gabor_bmd.p, *k2 = c->gabor_blo.p;
         const double *wsum = (const double *)c->gabor_wsum.p;
         const double gslack = c->gabor_slack;
         push_late(gn, [=](hipStream_t s) {
-          if (prec) launch_gabor_mixed(prec, ni, k0, k1, k2, wsum, gk, end_, bdd, gprm, gflag, o, ne, mh, mw, s);
-          else if (cert) launch_gabor_certified(ni, gk, gf, wsum, gslack, end_, bdd, gprm, gflag, o, ne, mh, mw, s);
+          if (prec) launch_gabor_mixed(prec, ni, k0, k1, k2, wsum, gk, end_, bdd, gst, gflag, o, ne, mh, mw, s);
+          else if (cert) launch_gabor_certified(ni, gk, gf, wsum, gslack, end_, bdd, gst, gflag, o, ne, mh, mw, s);
           else launch_gabor(ni, gk, end_, o, ne, mh, mw, s);
         });
       } break;

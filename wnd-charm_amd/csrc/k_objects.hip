@@ -883,7 +883,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 }
 
 // The energies E with an a-priori bound D on each one's distance from
-// k_gabor_conv's value E64, for k_gabor_post_exact to certify every count
+// k_gabor_conv's value E64, for launch_gabor_post_exact to certify every count
 // (k_gabor_repair recomputes in k_gabor_conv's order each energy a count leaves
 // open).
 //
@@ -1070,8 +1070,7 @@ __global__ void __launch_bounds__(1024) k_gabor_post(const Img *imgs, double *co
 // interval [E - D, E + D] leaves it open is taken on E64: the pixels
 // concerned are marked (D < 0), and the repairs recompute them in
 // k_gabor_conv's tap order (E = E64, D = 0).  Five phases of
-// k_gabor_post_exact, one block per (image, filter), each followed by the
-// repairs except the last:
+// launch_gabor_post_exact, each followed by the repairs except the last:
 //   1  mark the candidates for the maximum (upper end >= largest lower end)
 //   2  max M; filter 0: mark the pixels open at 0.4 M; other filters: mark
 //      the candidates for the minimum of e / M
@@ -1079,9 +1078,6 @@ __global__ void __launch_bounds__(1024) k_gabor_post(const Img *imgs, double *co
 //      pixels whose Otsu bin is open
 //   4  Otsu histogram and threshold; mark the pixels open at the threshold
 //   5  the counts above the threshold, the ratios
-// Per image and filter, params holds M, a, b, the threshold (and the base
-// count in filter 0's slot).
-constexpr int GP_STRIDE = 4;
 
 // the marked pixels (D < 0) of one 32 x 64 tile of one filter's map: the
 // input window staged in LDS as k_gabor_conv does, each marked output then
@@ -1219,162 +1215,182 @@ __global__ void __launch_bounds__(256) k_gabor_repair(const Img *imgs, const dou
   }
 }
 
-__global__ void __launch_bounds__(1024) k_gabor_post_exact(int phase, const Img *imgs, double *const *energy,
-                                                           float *const *bound, double *params, OutRef o,
-                                                           int *flags) {
-  __shared__ int hist[1024];
-  __shared__ double shd[16];
-  __shared__ long long shl[16];
-  __shared__ int marks[8];            // energies marked per filter in this phase
-  __shared__ int mlist[8][GR_CAP];    // the first GR_CAP of them
-  if (threadIdx.x < 8) marks[threadIdx.x] = 0;
-  __syncthreads();
-  const Img im = imgs[blockIdx.x];
-  const long n = (long)im.h * im.w;
-  double *const E0 = energy[blockIdx.x];
-  float *const D0 = bound[blockIdx.x];
-  double *prm = params + (long)blockIdx.x * 8 * GP_STRIDE;
-  const int f = blockIdx.y;  // one block per (image, filter)
-  if (!(phase >= 4 && f == 0)) do {
-    const double *E = E0 + (long)f * n;
-    float *D = D0 + (long)f * n;
-    double *P = prm + f * GP_STRIDE;
-    auto mark = [&](long i) {
-      D[i] = -D[i];
-      const int k = atomicAdd(&marks[f], 1);
-      if (k < GR_CAP) mlist[f][k] = (int)i;
-    };
-    if (phase == 1) {
-      double lo = -1e308;
-#pragma unroll 4
-      for (long i = threadIdx.x; i < n; i += 1024) lo = fmax(lo, E[i] - (double)D[i]);
-      lo = block_reduce(lo, MaxOp(), shd);
-#pragma unroll 4
-      for (long i = threadIdx.x; i < n; i += 1024)
-        if (D[i] != 0.0f && E[i] + (double)D[i] >= lo) mark(i);
-      break;
+// What the phases of the post-processing pass on, per (image, filter); values
+// that are minima or maxima over blocks are kept by their order-preserving keys.
+// GaborState is declared in kernels.hpp, for the caller's scratch.
+//
+// A phase first forms what it needs over the plane and then marks: two steps
+// (phase 2 three, filter 0 going straight on), each over blocks of GP_CHUNK
+// pixels.  Bound by memory: 12 bytes per pixel and filter and step.  Three planes
+// of 1388 x 1040: 0.8 ms for all steps, 10.1 ms with one block per (image,
+// filter); 64 planes of 64..1024 pixels a side: 2.6, 8.1 ms; 400 of 256 x 256:
+// 4.3, 4.5 ms; one of 128 x 128: 0.13, 0.12 ms (the threshold's chain of 1,024
+// bins and the launches).
+enum GaborStep { GP_LOW, GP_MARK_TOP, GP_MAX, GP_LEVEL, GP_MARK_LOW, GP_RANGE, GP_MARK_BIN, GP_HIST, GP_MARK_THR, GP_COUNT };
+constexpr int GP_CHUNK = 8192;
+
+__global__ void __launch_bounds__(1024) k_gabor_init(GaborState *state, int *flags, int count) {
+  for (int e = blockIdx.x; e < count; e += gridDim.x) {
+    GaborState &S = state[e];
+    S.hist[threadIdx.x] = 0;
+    if (threadIdx.x == 0) {
+      S.lo = S.mx = S.b = dkey(-1e308);
+      S.hi_min = S.a = dkey(1e308);
+      S.base = S.above = 0;
+      flags[(long)e * GR_STRIDE] = 0;
     }
-    if (phase == 2) {
-      double mx = -1e308;  // the candidates are exact now; nothing else can reach them
-#pragma unroll 4
-      for (long i = threadIdx.x; i < n; i += 1024)
-        if (D[i] == 0.0f) mx = fmax(mx, E[i]);
-      mx = block_reduce(mx, MaxOp(), shd);
-      if (threadIdx.x == 0) P[0] = mx;
-      if (!(mx > 0)) {  // no energy: every value exact, then the FP64 rules as written
-#pragma unroll 4
-        for (long i = threadIdx.x; i < n; i += 1024)
-          if (D[i] != 0.0f) mark(i);
-        break;
-      }
-      if (f == 0) {
-        const double lvl = mx * 0.4;
-#pragma unroll 4
-        for (long i = threadIdx.x; i < n; i += 1024) {
-          const double d = D[i];
-          if (d != 0.0 && E[i] - d <= lvl && E[i] + d > lvl) mark(i);
-        }
-        break;
-      }
-      double hi_min = 1e308;
-#pragma unroll 4
-      for (long i = threadIdx.x; i < n; i += 1024) {
-        const double v = (E[i] + (double)D[i]) / mx;
-        if (moments_ok(v)) hi_min = fmin(hi_min, v);
-      }
-      hi_min = block_reduce(hi_min, MinOp(), shd);
-#pragma unroll 4
-      for (long i = threadIdx.x; i < n; i += 1024)
-        if (D[i] != 0.0f && (E[i] - (double)D[i]) / mx <= hi_min) mark(i);
-      break;
-    }
-    const double mx = P[0];
-    if (phase == 3) {
-      if (f == 0) {
-        const double lvl = mx * 0.4;
-        long long c = 0;
-#pragma unroll 4
-        for (long i = threadIdx.x; i < n; i += 1024) {
-          const double d = D[i];
-          c += d == 0.0 ? E[i] > lvl : E[i] - d > lvl;  // open pixels were recomputed
-        }
-        c = block_reduce(c, SumOp(), shl);
-        if (threadIdx.x == 0) P[3] = (double)c;
-        break;
-      }
-      double a = 1e308, b = -1e308;
-#pragma unroll 4
-      for (long i = threadIdx.x; i < n; i += 1024) {
-        const double v = E[i] / mx;
-        if (D[i] == 0.0f && moments_ok(v)) { a = fmin(a, v); b = fmax(b, v); }
-      }
-      a = block_reduce(a, MinOp(), shd);
-      b = block_reduce(b, MaxOp(), shd);
-      if (threadIdx.x == 0) { P[1] = a; P[2] = b; }
-      const double sc = hist_scale(a, b, 1024);
-#pragma unroll 4
-      for (long i = threadIdx.x; i < n; i += 1024) {
-        const double d = D[i];
-        if (d == 0.0) continue;
-        // the true value lies in [a, b]: clamp the interval's ends there
-        const double vl = fmax((E[i] - d) / mx, a), vh = fmin((E[i] + d) / mx, b);
-        if (hist_bin(vl, a, sc, 1024) != hist_bin(vh, a, sc, 1024)) mark(i);
-      }
-      break;
-    }
-    const double a = P[1], b = P[2];
-    if (phase == 4) {
-      for (int k = threadIdx.x; k < 1024; k += 1024) hist[k] = 0;
-      __syncthreads();
-      const double sc = hist_scale(a, b, 1024);
-#pragma unroll 4
-      for (long i = threadIdx.x; i < n; i += 1024) {
-        const double e = E[i], d = D[i];
-        // d > 0: the bin was decided by the interval (both ends give it)
-        const double v = d == 0.0 ? e / mx : fmax((e - d) / mx, a);
-        atomicAdd(&hist[hist_bin(v, a, sc, 1024)], 1);
-      }
-      __syncthreads();
-      const double thr = otsu_threshold(hist, n, a, b);
-      if (threadIdx.x == 0) P[3] = thr;
-#pragma unroll 4
-      for (long i = threadIdx.x; i < n; i += 1024) {
-        const double d = D[i];
-        if (d != 0.0 && (E[i] - d) / mx <= thr && (E[i] + d) / mx > thr) mark(i);
-      }
-      __syncthreads();  // hist is reused by the next filter
-      break;
-    }
-    // phase 5
-    const double thr = P[3];
-    long long c = 0;
-#pragma unroll 4
-    for (long i = threadIdx.x; i < n; i += 1024) {
-      const double d = D[i];
-      c += d == 0.0 ? (E[i] / mx) > thr : (E[i] - d) / mx > thr;
-    }
-    c = block_reduce(c, SumOp(), shl);
-    if (threadIdx.x == 0) o.rows[blockIdx.x][f - 1] = (double)c / prm[3];
-  } while (0);
-  __syncthreads();
-  int *fl = flags + (long)(blockIdx.x * 8 + f) * GR_STRIDE;
-  for (int k = threadIdx.x; k < GR_STRIDE; k += blockDim.x) {
-    if (k == 0) fl[0] = marks[f];
-    else if (k - 1 < marks[f] && k - 1 < GR_CAP) fl[k] = mlist[f][k - 1];
   }
 }
 
-void launch_gabor_post_exact(const Img *imgs, double *const *energy, float *const *bound, const double *taps,
-                             double *params, int *flags, bool loop_tiles, OutRef o, int nimg, int maxh, int maxw,
-                             hipStream_t s) {
-  const int tiles = loop_tiles ? 1 : ((maxw + GB_TC - 1) / GB_TC) * ((maxh + GB_TR - 1) / GB_TR);
-  for (int phase = 1; phase <= 5; phase++) {
-    k_gabor_post_exact<<<dim3(nimg, 8), 1024, 0, s>>>(phase, imgs, energy, bound, params, o, flags);
-    if (phase < 5) {
-      k_gabor_repair_list<<<dim3(1, 8, nimg), 64, 0, s>>>(imgs, taps, energy, bound, flags);
-      k_gabor_repair<<<dim3(tiles, 8, nimg), 256, 0, s>>>(imgs, taps, energy, bound, flags, loop_tiles);
+template <int STEP>
+__global__ void __launch_bounds__(256) k_gabor_step(const Img *imgs, double *const *energy, float *const *bound,
+                                                    GaborState *state, int *flags) {
+  __shared__ int hist[STEP == GP_HIST ? 1024 : 1];
+  __shared__ double shd[4];
+  __shared__ int shi[4];
+  constexpr bool MARKS = STEP == GP_MARK_TOP || STEP == GP_LEVEL || STEP == GP_MARK_LOW || STEP == GP_MARK_BIN || STEP == GP_MARK_THR;
+  const Img im = imgs[blockIdx.z];
+  const long n = (long)im.h * im.w, c0 = (long)blockIdx.x * GP_CHUNK;
+  if (c0 >= n) return;
+  const int f = blockIdx.y, e = blockIdx.z * 8 + f;
+  GaborState &S = state[e];
+  int *fl = flags + (long)e * GR_STRIDE;
+  // the marks of the last phase are repaired; the next ones come in a later step
+  if ((STEP == GP_MAX || STEP == GP_RANGE || STEP == GP_HIST) && c0 == 0 && threadIdx.x == 0) fl[0] = 0;
+  if ((STEP == GP_MARK_LOW || STEP == GP_MARK_BIN || STEP == GP_HIST || STEP == GP_MARK_THR || STEP == GP_COUNT) && f == 0) return;
+  const gptr<const double> E = to_global((const double *)(energy[blockIdx.z] + f * n));
+  float *const Dp = bound[blockIdx.z] + f * n;
+  const gptr<const float> Dg = to_global((const float *)Dp);
+  const double mx = STEP >= GP_LEVEL ? dkey_inv(S.mx) : 0.0;
+  const double lo = STEP == GP_MARK_TOP ? dkey_inv(S.lo) : 0.0, hi_min = STEP == GP_MARK_LOW ? dkey_inv(S.hi_min) : 0.0;
+  const double a = STEP >= GP_MARK_BIN ? dkey_inv(S.a) : 0.0, b = STEP >= GP_MARK_BIN ? dkey_inv(S.b) : 0.0;
+  const double thr = STEP >= GP_MARK_THR ? S.thr : 0.0;
+  const double sc = STEP == GP_MARK_BIN || STEP == GP_HIST ? hist_scale(a, b, 1024) : 0.0;
+  if (STEP == GP_MARK_LOW && !(mx > 0)) return;
+  if (STEP == GP_HIST) {
+    for (int k = threadIdx.x; k < 1024; k += 256) hist[k] = 0;
+    __syncthreads();
+  }
+  double vmax = -1e308, vmin = 1e308;
+  int cnt = 0;
+  const long end = min(n, c0 + GP_CHUNK);
+  for (long i0 = c0 + threadIdx.x; i0 < end; i0 += 256 * 4) {
+    double ev[4];
+    float dv[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const long i = min(i0 + 256 * k, end - 1);
+      ev[k] = E[i];
+      dv[k] = Dg[i];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const long i = i0 + 256 * k;
+      if (i >= end) continue;
+      const double x = ev[k], d = dv[k];
+      const bool exact = dv[k] == 0.0f;
+      bool mark = false;
+      if (STEP == GP_LOW) vmax = fmax(vmax, x - d);
+      if (STEP == GP_MARK_TOP) mark = !exact && x + d >= lo;
+      if (STEP == GP_MAX && exact) vmax = fmax(vmax, x);  // nothing else can reach the candidates
+      if (STEP == GP_LEVEL) {
+        if (!(mx > 0)) mark = !exact;  // no energy: every value exact, then the FP64 rules as written
+        else if (f == 0) mark = !exact && x - d <= mx * 0.4 && x + d > mx * 0.4;
+        else {
+          const double v = (x + d) / mx;
+          if (moments_ok(v)) vmin = fmin(vmin, v);
+        }
+      }
+      if (STEP == GP_MARK_LOW) mark = !exact && (x - d) / mx <= hi_min;
+      if (STEP == GP_RANGE) {
+        if (f == 0) cnt += exact ? x > mx * 0.4 : x - d > mx * 0.4;  // open pixels were recomputed
+        else {
+          const double v = x / mx;
+          if (exact && moments_ok(v)) { vmin = fmin(vmin, v); vmax = fmax(vmax, v); }
+        }
+      }
+      if (STEP == GP_MARK_BIN && !exact) {
+        // the true value lies in [a, b]: clamp the interval's ends there
+        const double vl = fmax((x - d) / mx, a), vh = fmin((x + d) / mx, b);
+        mark = hist_bin(vl, a, sc, 1024) != hist_bin(vh, a, sc, 1024);
+      }
+      if (STEP == GP_HIST) {
+        // d > 0: the bin was decided by the interval (both ends give it)
+        const double v = exact ? x / mx : fmax((x - d) / mx, a);
+        atomicAdd(&hist[hist_bin(v, a, sc, 1024)], 1);
+      }
+      if (STEP == GP_MARK_THR) mark = !exact && (x - d) / mx <= thr && (x + d) / mx > thr;
+      if (STEP == GP_COUNT) cnt += exact ? (x / mx) > thr : (x - d) / mx > thr;
+      if (MARKS && mark) {
+        Dp[i] = -dv[k];
+        const int q = atomicAdd(fl, 1);
+        if (q < GR_CAP) fl[1 + q] = (int)i;
+      }
     }
   }
+  if (STEP == GP_LOW || STEP == GP_MAX || STEP == GP_RANGE) vmax = block_reduce(vmax, MaxOp(), shd);
+  if (STEP == GP_LEVEL || STEP == GP_RANGE) vmin = block_reduce(vmin, MinOp(), shd);
+  if (STEP == GP_RANGE || STEP == GP_COUNT) cnt = block_reduce(cnt, SumOp(), shi);
+  if (threadIdx.x == 0) {
+    if (STEP == GP_LOW) atomicMax(&S.lo, (unsigned long long)dkey(vmax));
+    if (STEP == GP_MAX) atomicMax(&S.mx, (unsigned long long)dkey(vmax));
+    if (STEP == GP_LEVEL) atomicMin(&S.hi_min, (unsigned long long)dkey(vmin));
+    if (STEP == GP_RANGE) {
+      atomicMin(&S.a, (unsigned long long)dkey(vmin));
+      atomicMax(&S.b, (unsigned long long)dkey(vmax));
+      if (f == 0) atomicAdd(&S.base, (unsigned long long)cnt);
+    }
+    if (STEP == GP_COUNT) atomicAdd(&S.above, (unsigned long long)cnt);
+  }
+  if (STEP == GP_HIST) {
+    __syncthreads();
+    for (int k = threadIdx.x; k < 1024; k += 256)
+      if (hist[k]) atomicAdd(&S.hist[k], hist[k]);
+  }
+}
+
+__global__ void __launch_bounds__(1024) k_gabor_threshold(const Img *imgs, GaborState *state) {
+  __shared__ int hist[1024];
+  const Img im = imgs[blockIdx.x];
+  GaborState &S = state[blockIdx.x * 8 + blockIdx.y + 1];
+  hist[threadIdx.x] = S.hist[threadIdx.x];
+  __syncthreads();
+  const double thr = otsu_threshold(hist, (long)im.h * im.w, dkey_inv(S.a), dkey_inv(S.b));
+  if (threadIdx.x == 0) S.thr = thr;
+}
+
+__global__ void __launch_bounds__(64) k_gabor_ratios(const GaborState *state, OutRef o) {
+  const int f = threadIdx.x;
+  if (f >= 1 && f < 8)
+    o.rows[blockIdx.x][f - 1] = (double)state[blockIdx.x * 8 + f].above / (double)state[blockIdx.x * 8].base;
+}
+
+void launch_gabor_post_exact(const Img *imgs, double *const *energy, float *const *bound, const double *taps,
+                             GaborState *state, int *flags, bool loop_tiles, OutRef o, int nimg, int maxh, int maxw,
+                             hipStream_t s) {
+  const int tiles = loop_tiles ? 1 : ((maxw + GB_TC - 1) / GB_TC) * ((maxh + GB_TR - 1) / GB_TR);
+  const dim3 grid((unsigned)(((long)maxh * maxw + GP_CHUNK - 1) / GP_CHUNK), 8, nimg);
+  auto repair = [&] {
+    k_gabor_repair_list<<<dim3(1, 8, nimg), 64, 0, s>>>(imgs, taps, energy, bound, flags);
+    k_gabor_repair<<<dim3(tiles, 8, nimg), 256, 0, s>>>(imgs, taps, energy, bound, flags, loop_tiles);
+  };
+  k_gabor_init<<<std::min(8 * nimg, 4096), 1024, 0, s>>>(state, flags, 8 * nimg);
+  k_gabor_step<GP_LOW><<<grid, 256, 0, s>>>(imgs, energy, bound, state, flags);
+  k_gabor_step<GP_MARK_TOP><<<grid, 256, 0, s>>>(imgs, energy, bound, state, flags);
+  repair();
+  k_gabor_step<GP_MAX><<<grid, 256, 0, s>>>(imgs, energy, bound, state, flags);
+  k_gabor_step<GP_LEVEL><<<grid, 256, 0, s>>>(imgs, energy, bound, state, flags);
+  k_gabor_step<GP_MARK_LOW><<<grid, 256, 0, s>>>(imgs, energy, bound, state, flags);
+  repair();
+  k_gabor_step<GP_RANGE><<<grid, 256, 0, s>>>(imgs, energy, bound, state, flags);
+  k_gabor_step<GP_MARK_BIN><<<grid, 256, 0, s>>>(imgs, energy, bound, state, flags);
+  repair();
+  k_gabor_step<GP_HIST><<<grid, 256, 0, s>>>(imgs, energy, bound, state, flags);
+  k_gabor_threshold<<<dim3(nimg, 7), 1024, 0, s>>>(imgs, state);
+  k_gabor_step<GP_MARK_THR><<<grid, 256, 0, s>>>(imgs, energy, bound, state, flags);
+  repair();
+  k_gabor_step<GP_COUNT><<<grid, 256, 0, s>>>(imgs, energy, bound, state, flags);
+  k_gabor_ratios<<<nimg, 64, 0, s>>>(state, o);
 }
 
 void launch_gabor(const Img *imgs, const double *kernels, double *const *energy, OutRef o, int nimg, int maxh,
@@ -1384,7 +1400,7 @@ void launch_gabor(const Img *imgs, const double *kernels, double *const *energy,
   k_gabor_post<<<nimg, 1024, 0, s>>>(imgs, energy, o);
 }
 void launch_gabor_certified(const Img *imgs, const double *kernels, const double *factors, const double *wsum,
-                            double slack, double *const *energy, float *const *bound, double *params, int *flags,
+                            double slack, double *const *energy, float *const *bound, GaborState *state, int *flags,
                             OutRef o, int nimg, int maxh, int maxw, hipStream_t s) {
   const int tiles = ((maxw + GB_TC - 1) / GB_TC) * ((maxh + GS_TR - 1) / GS_TR);
   // a CU holds one block: from two blocks per CU on, the input tile is read once
@@ -1392,7 +1408,7 @@ void launch_gabor_certified(const Img *imgs, const double *kernels, const double
   // of 128 x 128: 10 blocks or 80)
   const int per = (long)tiles * nimg >= 512 ? 8 : 1;
   k_gabor_sep<<<dim3(tiles, 8 / per, nimg), 512, 0, s>>>(imgs, factors, kernels, energy, wsum, bound, 4e-13 * slack, per);
-  launch_gabor_post_exact(imgs, energy, bound, kernels, params, flags, slack <= 1.0, o, nimg, maxh, maxw, s);
+  launch_gabor_post_exact(imgs, energy, bound, kernels, state, flags, slack <= 1.0, o, nimg, maxh, maxw, s);
 }
 void launch_gabor_post(const Img *imgs, double *const *energy, OutRef o, int nimg, hipStream_t s) {
   k_gabor_post<<<nimg, 1024, 0, s>>>(imgs, energy, o);

@@ -206,6 +206,13 @@ struct EdgeCounts { int area, hm[8], hd[8]; };
 void launch_edge_final(const Img *mag, const Img *dir, const Stats *st2, const double *medians, EdgeCounts *cnt, OutRef o,
                        int nimg, long maxn, hipStream_t s);
 void launch_gabor_post(const Img *imgs, double *const *energy, OutRef o, int nimg, hipStream_t s);
+// scratch of the exact Gabor post-processing, per (image, filter)
+struct GaborState {
+  unsigned long long lo, mx, hi_min, a, b;  // keys (dkey): lower end of the top, maximum, upper end of the minimum, range of e / mx
+  unsigned long long base, above;           // counts above 0.4 of the maximum (filter 0), above the threshold
+  double thr;
+  int hist[1024];
+};
 // reduced-precision contractions (k_mixed.hip): precision 1 = FP32, 2 = BF16x3 on MFMA.
 // Gabor: FP32 takes float kernels (k0); BF16x3 takes the hi / mid / lo bf16
 // planes (k0, k1, k2); both write per-pixel error bounds and finish with the
@@ -216,9 +223,9 @@ void launch_gabor_post(const Img *imgs, double *const *energy, OutRef o, int nim
 // for bounds that leave few energies open
 void launch_gabor_mixed(int precision, const Img *imgs, const void *k0, const void *k1, const void *k2,
                         const double *wsum, const double *taps64, double *const *energy, float *const *bound,
-                        double *params, int *flags, OutRef o, int nimg, int maxh, int maxw, hipStream_t s);
+                        GaborState *state, int *flags, OutRef o, int nimg, int maxh, int maxw, hipStream_t s);
 void launch_gabor_post_exact(const Img *imgs, double *const *energy, float *const *bound, const double *taps,
-                             double *params, int *flags, bool loop_tiles, OutRef o, int nimg, int maxh, int maxw,
+                             GaborState *state, int *flags, bool loop_tiles, OutRef o, int nimg, int maxh, int maxw,
                              hipStream_t s);
 void launch_gabor(const Img *imgs, const double *kernels, double *const *energy, OutRef o, int nimg, int maxh,
                   int maxw, hipStream_t s);
@@ -226,7 +233,7 @@ void launch_gabor(const Img *imgs, const double *kernels, double *const *energy,
 // with per-energy bounds
 // (scaled by slack >= 1), every count certified by the exact post-processing
 void launch_gabor_certified(const Img *imgs, const double *kernels, const double *factors, const double *wsum,
-                            double slack, double *const *energy, float *const *bound, double *params, int *flags,
+                            double slack, double *const *energy, float *const *bound, GaborState *state, int *flags,
                             OutRef o, int nimg, int maxh, int maxw, hipStream_t s);
 void launch_zernike(const Img *imgs, double *partial, int nchunk, const double *htab, OutRef o, int nimg,
                     hipStream_t s, int precision = 0);
