@@ -2,8 +2,9 @@
 
 A block forms 27 x 64 energies; below 512 blocks it takes one filter, beyond
 all eight; and where its pixels are outside [1e-24, 1e290] (or infinite) it
-adds the 1,444 taps.  The counts are taken over blocks of 8,192 pixels.  They are certified against the reference's sums, so
-every ratio equals the direct path's (WNDGPU_GABOR_DIRECT=1) exactly."""
+adds the 1,444 taps.  The counts are taken over blocks of 8,192 pixels and
+certified against the reference's sums, so every ratio equals the direct
+path's (WNDGPU_GABOR_DIRECT=1) exactly."""
 import numpy as np
 import pytest
 
