@@ -65,3 +65,19 @@ def test_edge_medians(shape, kind):
            'ramp': np.mgrid[0:h, 0:w][1] * 3.0, 'skewed': np.exp(rng.normal(0, 6, shape))}[kind]
     print('edge', shape, kind, flush=True)
     check('Edge Features', img, EDGE_EXACT)
+
+
+def test_more_planes_than_a_grid_dimension_holds():
+    """33,000 images: 66,000 edge planes, and 66,000 object planes over two
+    nodes, in one call (a grid has up to 65,536 blocks in y); every row equal to
+    its image's in a call of 40"""
+    plan = wndcharm.FeatureComputationPlan('many planes')
+    for group in ('Edge Features ()', 'Otsu Object Features ()', 'Otsu Object Features (Edge ())',
+                  'Inverse-Otsu Object Features ()'):
+        plan.add(group)
+    plan.finalize()
+    imgs = [winding(16, 16 + k % 3, seed=k).astype(np.uint8) for k in range(40)]
+    some = wndcharm.compute_features(imgs, plan)
+    print('objects and edges: 33,000 images', flush=True)
+    many = wndcharm.compute_features(imgs * 825, plan)
+    assert np.array_equal(many, np.tile(some, (825, 1)), equal_nan=True)

@@ -502,19 +502,33 @@ __global__ void __launch_bounds__(1024) k_obj_final(const ObjDesc *ods, OutRef o
   }
 }
 
+// Images or planes of a launch whose grid has them in y, which by the device's
+// limits takes up to 65,536: a call may have more (edge features two planes per
+// image, the object features one per node of the plan), so these launches go in
+// slices.
+constexpr int GRID_Y = 65536;
+template <class Launch>
+static void in_slices(int n, Launch launch) {
+  for (int i = 0; i < n; i += GRID_Y) launch(i, std::min(n - i, GRID_Y));
+}
+
 void launch_objects(const Img *imgs, const Stats *st, int invert, const ObjDesc *od, OutRef o, int nimg, long maxn,
                     int maxstrips, hipStream_t s) {
-  const dim3 chunks((unsigned)((maxn + OBJ_CHUNK - 1) / OBJ_CHUNK), nimg);
-  k_obj_init<<<nimg, 1024, 0, s>>>(imgs, st, invert, od);
-  k_obj_hist<<<chunks, 256, 0, s>>>(imgs, st, invert, od);
-  k_obj_thresh<<<nimg, 1024, 0, s>>>(imgs, od);
-  k_obj_strip<<<dim3(maxstrips, nimg), 1024, 0, s>>>(imgs, st, invert, od);
-  if (maxstrips > 1) k_obj_merge<<<dim3(maxstrips - 1, nimg), 256, 0, s>>>(imgs, od);
-  k_obj_flat<<<chunks, 1024, 0, s>>>(imgs, od);
-  k_obj_scan<<<nimg, 1024, 0, s>>>(imgs, od);
-  k_obj_rank<<<chunks, 1024, 0, s>>>(imgs, od);
-  k_obj_area<<<chunks, 1024, 0, s>>>(imgs, od);
-  k_obj_final<<<nimg, 1024, 0, s>>>(od, o);
+  in_slices(nimg, [&](int i, int n) {
+    const Img *im = imgs + i;
+    const ObjDesc *d = od + i;
+    const dim3 chunks((unsigned)((maxn + OBJ_CHUNK - 1) / OBJ_CHUNK), n);
+    k_obj_init<<<n, 1024, 0, s>>>(im, st + i, invert, d);
+    k_obj_hist<<<chunks, 256, 0, s>>>(im, st + i, invert, d);
+    k_obj_thresh<<<n, 1024, 0, s>>>(im, d);
+    k_obj_strip<<<dim3(maxstrips, n), 1024, 0, s>>>(im, st + i, invert, d);
+    if (maxstrips > 1) k_obj_merge<<<dim3(maxstrips - 1, n), 256, 0, s>>>(im, d);
+    k_obj_flat<<<chunks, 1024, 0, s>>>(im, d);
+    k_obj_scan<<<n, 1024, 0, s>>>(im, d);
+    k_obj_rank<<<chunks, 1024, 0, s>>>(im, d);
+    k_obj_area<<<chunks, 1024, 0, s>>>(im, d);
+    k_obj_final<<<n, 1024, 0, s>>>(d, OutRef{o.rows + i});
+  });
 }
 int obj_strips(int h, int w) { return (h + obj_strip_rows(w) - 1) / obj_strip_rows(w); }
 int obj_chunks(long n) { return (int)((n + OBJ_CHUNK - 1) / OBJ_CHUNK); }
@@ -789,12 +803,14 @@ __global__ void __launch_bounds__(64) k_edge_final(const EdgeCounts *cnt, const 
 
 void launch_median(const Img *planes, const Stats *st, SelState *sel, uint64_t *const *keys, double *median, int nplanes,
                    long maxn, hipStream_t s) {
-  const dim3 chunks((unsigned)((maxn + SEL_CHUNK - 1) / SEL_CHUNK), nplanes);
-  k_sel_init<<<nplanes, 1024, 0, s>>>(sel);
-  k_sel_hist<<<chunks, 256, 0, s>>>(planes, st, sel);
-  k_sel_pick<<<nplanes, 1024, 0, s>>>(planes, sel);
-  k_sel_collect<<<chunks, 256, 0, s>>>(planes, st, sel, keys);
-  k_sel_final<<<nplanes, 1024, 0, s>>>(planes, sel, keys, median);
+  in_slices(nplanes, [&](int i, int n) {
+    const dim3 chunks((unsigned)((maxn + SEL_CHUNK - 1) / SEL_CHUNK), n);
+    k_sel_init<<<n, 1024, 0, s>>>(sel + i);
+    k_sel_hist<<<chunks, 256, 0, s>>>(planes + i, st + i, sel + i);
+    k_sel_pick<<<n, 1024, 0, s>>>(planes + i, sel + i);
+    k_sel_collect<<<chunks, 256, 0, s>>>(planes + i, st + i, sel + i, keys + i);
+    k_sel_final<<<n, 1024, 0, s>>>(planes + i, sel + i, keys + i, median + i);
+  });
 }
 void launch_prewitt(const Img *imgs, const Img *mag, const Img *dir, int nimg, long maxn, hipStream_t s) {
   k_prewitt<<<dim3((maxn + 255) / 256, nimg), 256, 0, s>>>(imgs, mag, dir);
