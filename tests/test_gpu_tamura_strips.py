@@ -43,3 +43,16 @@ def test_values(kind):
            'negative': noise - 50, 'tiny': 1.0 + np.round(noise) * 2.0 ** -52,
            'float32': noise.astype(np.float32).astype(np.float64) + 9}[kind]
     check(img)
+
+
+@pytest.mark.parametrize('exponent', [-1074, -1073, -1070, -1060, -1022, -1015])
+def test_window_means_of_subnormal_sums(exponent):
+    """pixels of a few units near the smallest double: subnormal means, where a
+    quotient can lie halfway between two doubles.  The largest pixel is 1, so
+    that normalisation keeps the values, and the last, so that the sums before
+    it stay small."""
+    print('tamura subnormal 2 **', exponent, flush=True)
+    rng = np.random.default_rng(-exponent)
+    img = np.ldexp(rng.integers(0, 40, (70, 150)).astype(np.float64), exponent)
+    img[-1, -1] = 1.0
+    check(img)

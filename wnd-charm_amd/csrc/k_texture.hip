@@ -2549,13 +2549,16 @@ __global__ void __launch_bounds__(64 * SAT_WAVES) k_tam_sat(const Img *imgs, dou
 // the last place of 1 / c.  A quotient is the product with r with the
 // remainder's quotient added, which rounds as the division does because a / c is
 // nowhere nearer than 1 / (2c) units in the last place to the middle between two
-// doubles; an infinite a, whose remainder is no number, is its own quotient.
+// doubles.  Not so where the quotient is subnormal, which can lie in the very
+// middle, or where a is infinite and the remainder no number: these are divided.
 __device__ __forceinline__ double mean_diff(double a0, double c0, double r0, double a1, double c1, double r1) {
+  constexpr int SUBNORMAL = 0x10 | 0x80;  // of either sign, for v_cmp_class
   const double q0 = a0 * r0, q1 = a1 * r1;
   const double m0 = __builtin_fma(__builtin_fma(-c0, q0, a0), r0, q0);
   const double m1 = __builtin_fma(__builtin_fma(-c1, q1, a1), r1, q1);
   double v = fabs(m0 - m1);
-  if (__any(v != v)) v = fabs((__builtin_isinf(a0) ? a0 : m0) - (__builtin_isinf(a1) ? a1 : m1));
+  if (__any(v != v || __builtin_amdgcn_class(m0, SUBNORMAL) || __builtin_amdgcn_class(m1, SUBNORMAL)))
+    v = fabs(a0 / c0 - a1 / c1);
   return v;
 }
 
