@@ -75,3 +75,21 @@ def test_device_io_replays(graph_mode):
         torch.cuda.synchronize()
         assert lib.wndgpu_compute_device(ctx, plan.handle, st, len(dev), ctypes.c_void_p(out.data_ptr()), None) == 0
         assert np.array_equal(out.cpu().numpy(), eager[k], equal_nan=True)
+
+
+def test_replays_pick_the_schur_kernel_by_their_own_tones(graph_mode):
+    """300 images of few tones and 300 with many among few take different Schur
+    kernels; one graph serves both"""
+    import wndcharm
+    plan = wndcharm.FeatureComputationPlan('haralick')
+    plan.add('Haralick Textures ()')
+    plan.finalize()
+    rng = np.random.default_rng(3)
+    few = [rng.integers(0, 9, (24, 32)).astype(np.uint8) * 20 for _ in range(300)]
+    many = [rng.integers(0, 256, (24, 32)).astype(np.uint8) if k % 30 == 0 else few[k] for k in range(300)]
+    graph_mode(0)
+    eager = [wndcharm.compute_features(b, plan) for b in (few, many)]
+    graph_mode(1)
+    for k in (0, 0, 1, 0, 1, 1):
+        got = wndcharm.compute_features((few, many)[k], plan)
+        assert np.array_equal(got, eager[k], equal_nan=True), k

@@ -5,7 +5,8 @@ The small-launch kernel chases a bulge in windows of 16 steps, keeps a band of
 64 columns in a wave and updates rows above a window 64 at a time, so matrix
 orders around multiples of 16 and 64 (order = number of gray tones) exercise
 its remainders; order 256 is the largest, and orders below 3 have no f14.
-Launches of up to 256 matrices, up to 6144 and beyond take different kernels."""
+Launches of up to 256 matrices, up to 6144 and beyond take different kernels,
+and from 1025 to 6144 the tones decide between two of them."""
 import numpy as np
 import pytest
 
@@ -68,3 +69,22 @@ def test_schur_launch_rules_agree():
     one = np.concatenate([wndcharm.compute_features([im], plan) for im in kinds[::9]])
     assert np.array_equal(many, np.concatenate([some] * 16), equal_nan=True)
     assert np.array_equal(one, some[::9], equal_nan=True)
+
+
+@pytest.mark.parametrize('n', [256, 257, 700])
+@pytest.mark.parametrize('kind', ['few', 'spread', 'one'])
+def test_kernel_picked_by_tones(kind, n):
+    """256 entries take four waves per matrix; beyond, entries of few tones take
+    one wave per matrix, and many tones among few ones four; whichever it is,
+    every entry has the bits that it has on its own"""
+    tones = {'few': [12] * 9, 'spread': range(5, 200, 22), 'one': [250] + [9] * 8}[kind]
+    kinds = [toned(ng, k, (24, 32)) for k, ng in enumerate(tones)]
+    plan = wndcharm.FeatureComputationPlan('haralick')
+    plan.add('Haralick Textures ()')
+    plan.finalize()
+    print('schur picked', kind, n, flush=True)
+    got = wndcharm.compute_features([kinds[k % 9] for k in range(n)], plan)
+    work = wndcharm.last_haralick_work()[1]
+    one = np.concatenate([wndcharm.compute_features([im], plan) for im in kinds])
+    assert np.array_equal(got, one[np.arange(n) % 9], equal_nan=True)
+    assert np.array_equal(work, work[np.arange(n) % 9]) and (work > 0).all()

@@ -1062,7 +1062,8 @@ k_har_hess_rows(const HarDesc *hd, const int *order) {
 // iteration is a chain of dependent steps, so many chains with a small LDS
 // window each keep the CU busy; k_har_schur below serves smaller launches.
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
-k_har_qr(const HarDesc *hd, const int *order) {
+k_har_qr(const HarDesc *hd, const int *order, const int *pick) {
+  if (pick && *pick != 0) return;  // uniform: k_har_schur takes the launch
   constexpr int RS = 2;   // window rows per pass of the wave (32 columns per row)
   constexpr int CH = QW;  // rows above the window staged per chunk
   __shared__ double Rw[CH * QWP];
@@ -1665,7 +1666,8 @@ __device__ __forceinline__ void schur_right(unsigned on, const SchurRf *rf, doub
 
 template <int NW>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
-k_har_schur(const HarDesc *hd, const int *order) {
+k_har_schur(const HarDesc *hd, const int *order, const int *pick) {
+  if (pick && *pick == 0) return;  // uniform: k_har_qr takes the launch
   // window t's buffer (t mod 3): slot j first holds row k0+3+j, which wave 0
   // reads at step j, then the finished row k0+j, which it writes at step j;
   // column k0 + l at l
@@ -2317,15 +2319,36 @@ void launch_haralick_prep(const Img *imgs, const Stats *st, const HarDesc *hd, i
 // own, so the order changes no result.  Thread b owns key b = 256 - ng and
 // scans the entries in index order (keys staged in LDS, chunk by chunk), so
 // ties keep index order and the order is the same on every run.
+//
+// order[nimg] (pick_too) tells which kernel finishes a launch of medium size
+// (launch_haralick_qr): 1 for k_har_schur<4>, whose 512 resident matrices make
+// short chains, 0 for k_har_qr, whose 4,096 make three times longer ones but do
+// 1.1 to 2.5 times as many matrices in all.  Both estimates, in ms, are fits to
+// either kernel's times over launches of 4 x 400 .. 4 x 1500 matrices with equal
+// tones (8 .. 240), tones spread evenly from 0 and one entry in 40 of 256 tones.
+// Either kernel gives the same bits.
 constexpr int ORDER_CHUNK = 16384;
-__global__ void __launch_bounds__(320) k_har_order(const int *ng, int nimg, int *order) {
+__global__ void __launch_bounds__(320) k_har_order(const int *ng, int nimg, int *order, int pick_too) {
   __shared__ __align__(16) uint16_t key[ORDER_CHUNK];
   __shared__ int cnt[257];
+  __shared__ double shd[5];
   const int t = threadIdx.x;
   for (int b = t; b < 257; b += blockDim.x) cnt[b] = 0;
   __syncthreads();
   for (int e = t; e < nimg; e += blockDim.x) atomicAdd(&cnt[256 - min(max(ng[e], 0), 256)], 1);
   __syncthreads();
+  if (pick_too) {
+    const double n = 256 - t, m = t < 257 ? 4.0 * cnt[t] : 0.0;
+    const double chain = n * (8.1e-3 + n * (2.05e-4 + n * 1.5e-7));  // one matrix by k_har_schur<4>
+    const double top = block_reduce(m > 0 ? n : 0.0, MaxOp(), shd);
+    const double chains = block_reduce(m * chain, SumOp(), shd);
+    const double work = block_reduce(m * n * n * (1.5e-7 + n * 7.6e-10), SumOp(), shd);
+    if (t == 0) {
+      const double schur = 0.4 * top * (8.1e-3 + top * (2.05e-4 + top * 1.5e-7)) + chains / 512;
+      const double qr = top * (3e-3 + top * (5.4e-4 + top * 8.1e-7)) + 0.5 * work;
+      order[nimg] = schur < qr;
+    }
+  }
   if (t == 0) {
     int sum = 0;
     for (int b = 0; b < 257; b++) {
@@ -2352,8 +2375,10 @@ __global__ void __launch_bounds__(320) k_har_order(const int *ng, int nimg, int 
       }
   }
 }
+// Matrices of a launch that k_har_order picks the kernel for.
+static bool haralick_pick(int nimg) { return 4 * nimg > 1024 && 4 * nimg <= 6144; }
 void launch_haralick_order(const int *ng, int nimg, int *order, hipStream_t s) {
-  k_har_order<<<1, 320, 0, s>>>(ng, nimg, order);
+  k_har_order<<<1, 320, 0, s>>>(ng, nimg, order, haralick_pick(nimg));
 }
 void launch_haralick_hess(const HarDesc *hd, const int *order, int nimg, hipStream_t s) {
   k_har_hess<<<dim3(4, nimg), 512, 0, s>>>(hd, order);
@@ -2361,17 +2386,24 @@ void launch_haralick_hess(const HarDesc *hd, const int *order, int nimg, hipStre
 }
 void launch_haralick_qr(const HarDesc *hd, const int *order, int nimg, hipStream_t s) {
   // Up to 256 matrices every CU has at most one, and the launch lasts as long
-  // as the longest chain of steps: eight waves per matrix.  Up to 6144, four
-  // waves per matrix, two matrices per CU.  Beyond, one wave per matrix and
-  // sixteen matrices per CU: its chain is three times slower, but it does less
-  // work per step, and with that many the work counts.  Nodes of 256 x 256
-  // images (tones 10..256, mean 128), this rule's kernel against the other:
-  // 48 matrices 13.2 against 30.6 ms (four waves: 17.5), 1200 18.3 against
-  // 48.4, 2400 33.0 against 51.6, 4800 62.9 against 69.0; 7200 88.2 against
-  // 93.9, 9600 112.0 against 124.8, 19200 201 against 259.
-  if (4 * nimg <= 256) k_har_schur<8><<<dim3(4, nimg), 512, 0, s>>>(hd, order);
-  else if (4 * nimg <= 6144) k_har_schur<4><<<dim3(4, nimg), 256, 0, s>>>(hd, order);
-  else k_har_qr<<<dim3(4, nimg), 64, 0, s>>>(hd, order);
+  // as the longest chain of steps: eight waves per matrix.  Up to 1024, four
+  // waves per matrix, two matrices per CU: with tones of 8 .. 240, equal or
+  // spread, in no case slower than the kernel before it (240 equal tones, 1024
+  // matrices: 37.3 against 72.4 ms; 64: 2.9 against 5.7; 8: 0.18 against 0.19).
+  // Beyond 6144 one wave per matrix and sixteen matrices per CU: its chain is
+  // three times slower, but it does less work per step, and with that many the
+  // work counts.  Between, it depends on the tones, which only the device knows:
+  // 1600 matrices of 64 equal tones 5.4 ms by four waves and 3.4 by one, of 0 ..
+  // 253 tones 21.4 and 49.9.  Both are launched and one of them returns at once.
+  // Nodes of 256 x 256 images (tones 10..256, mean 128): 48 matrices 12.4 ms (30.6
+  // with one 256-thread block per matrix; four waves: 17.5), 1200 18.3 against
+  // 48.4, 2400 33.0 against 51.6, 4800 62.9 against 69.0; 7200 88.2 by one wave
+  // against 93.9, 9600 112.0 against 124.8, 19200 201 against 259.
+  const dim3 grid(4, nimg);
+  const int *pick = haralick_pick(nimg) ? order + nimg : nullptr;
+  if (4 * nimg <= 256) k_har_schur<8><<<grid, 512, 0, s>>>(hd, order, nullptr);
+  else if (4 * nimg <= 6144) k_har_schur<4><<<grid, 256, 0, s>>>(hd, order, pick);
+  if (pick || 4 * nimg > 6144) k_har_qr<<<grid, 64, 0, s>>>(hd, order, pick);
 }
 void launch_haralick_final(const HarDesc *hd, OutRef o, int nimg, hipStream_t s) {
   k_har_final<<<nimg, 64, 0, s>>>(hd, o);
