@@ -1,8 +1,9 @@
 """GPU: Tamura textures where the summed-area table's strips and the pixel runs meet.
 
 The table is formed in strips of 64 rows, eight at once, in groups of 16
-columns; pixels are taken in runs of 64 columns x 8 rows and their histograms
-in blocks of 16,384.  Planes just below, at and above these sizes against the
+columns; pixels are taken in runs of 64 columns x 8 rows (2 rows in planes of up
+to 4,096 pixels) and their histograms in blocks of 16,384, planes of one block by
+one launch.  Planes just below, at and above these sizes against the
 oracle.  Best scales and phi go through histograms, whose counts are whole
 numbers: a wrong table entry moves a count, i.e. a result by more than 1 / P.
 The rest are sums of P terms in another order, P * 2^-53 < 1e-9 apart."""
@@ -24,7 +25,7 @@ def check(img):
 
 # one strip and less, runs and groups cut short, eight strips, a wave's second
 # strip where it follows after 41 groups (narrow) and after all groups (wide)
-@pytest.mark.parametrize('shape', [(16, 16), (16, 64), (17, 65), (63, 17), (64, 64), (65, 63), (64, 256), (129, 128), (128, 129),
+@pytest.mark.parametrize('shape', [(16, 16), (16, 64), (16, 256), (16, 257), (256, 16), (17, 65), (63, 17), (31, 129), (64, 64), (65, 63), (64, 256), (129, 128), (128, 129),
                                    (511, 40), (512, 17), (513, 33), (577, 593), (576, 594), (1100, 61), (1030, 700)])
 def test_strips_and_runs(shape):
     print('tamura', shape, flush=True)
@@ -56,3 +57,17 @@ def test_window_means_of_subnormal_sums(exponent):
     img = np.ldexp(rng.integers(0, 40, (70, 150)).astype(np.float64), exponent)
     img[-1, -1] = 1.0
     check(img)
+
+
+def test_planes_of_all_kinds_in_one_call():
+    """each plane's features are those that it has on its own, bit for bit"""
+    rng = np.random.default_rng(11)
+    shapes = [(16, 16), (64, 64), (64, 65), (17, 65), (256, 16), (128, 128), (129, 128), (31, 130), (600, 40), (300, 301)]
+    imgs = [rng.integers(0, 4000, s).astype(np.uint16) for s in shapes]
+    plan = wndcharm.FeatureComputationPlan('tamura')
+    plan.add('Tamura Textures ()')
+    plan.finalize()
+    print('tamura', shapes, flush=True)
+    one = np.concatenate([wndcharm.compute_features([im], plan) for im in imgs])
+    assert np.array_equal(wndcharm.compute_features(imgs, plan), one, equal_nan=True)
+    assert np.array_equal(wndcharm.compute_features(imgs[:5], plan), one[:5], equal_nan=True)

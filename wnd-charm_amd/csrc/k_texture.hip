@@ -2444,11 +2444,11 @@ __device__ __forceinline__ double from_lane_below(double v, double first) {
 }
 
 // Sums over a plane that the directionality and contrast need, by wave of
-// k_tam_pix (64 columns x TAM_ROWS rows), then by block of k_tam_hist
+// k_tam_pix (64 columns x tam_rows rows), then by block of TAM_CHUNK pixels
 struct TamPart { double s, sr, pmn, pmx; int ks, kmask; };
 struct TamPart2 { double m2, m4; };
 struct TamSum { double mean, sr, pmn, pmx; long long ks; int kmn, kmx; int hk[3], hd[125]; };
-constexpr int TAM_ROWS = 8, TAM_CHUNK = 16384;
+constexpr int TAM_CHUNK = 16384;
 static_assert(sizeof(TamPart) % 8 == 0 && sizeof(TamPart2) % 8 == 0, "parts are laid out in doubles");
 // scratch of a plane of P pixels, in doubles: [0, P) normalised plane, [P, 2P)
 // row differences and [3P, 4P) corner differences of the summed-area table,
@@ -2456,7 +2456,10 @@ static_assert(sizeof(TamPart) % 8 == 0 && sizeof(TamPart2) % 8 == 0, "parts are 
 // k_tam_pix and of k_tam_hist and a row of the table
 __host__ __device__ inline size_t tam_summary(long P) { return 4 * (size_t)P + ((size_t)P + 1) / 2; }
 __host__ __device__ inline size_t tam_parts(long P) { return tam_summary(P) + (sizeof(TamSum) + 7) / 8; }
-__host__ __device__ inline int tam_runs(int h, int w) { return ((w + 63) / 64) * ((h + TAM_ROWS - 1) / TAM_ROWS); }
+// rows of a wave of k_tam_pix: eight reuse what neighbouring rows share, two make
+// the shorter chain where a plane has few waves (one of 64 x 64: 10.5 us, 29.3 by eight)
+__host__ __device__ inline int tam_rows(int h, int w) { return (long)h * w <= 4096 ? 2 : 8; }
+__host__ __device__ inline int tam_runs(int h, int w) { return ((w + 63) / 64) * ((h + tam_rows(h, w) - 1) / tam_rows(h, w)); }
 __host__ __device__ inline size_t tam_parts2(int h, int w) {
   return tam_parts((long)h * w) + (size_t)tam_runs(h, w) * (sizeof(TamPart) / 8);
 }
@@ -2464,6 +2467,14 @@ __host__ __device__ inline size_t tam_row(int h, int w) {
   return tam_parts2(h, w) + ((size_t)h * w + TAM_CHUNK - 1) / TAM_CHUNK * (sizeof(TamPart2) / 8);
 }
 size_t tamura_scratch(int h, int w) { return tam_row(h, w) + w + 8; }
+// the most waves that a plane of up to maxh x maxw pixels has: more rows make
+// more of them until a plane takes eight rows per wave
+static int tam_max_runs(int maxh, int maxw) {
+  int most = tam_runs(maxh, maxw);
+  for (int w = 16; w <= maxw; w = (w + 63) / 64 * 64 + 1)  // the narrowest of each number of columns of waves
+    most = std::max(most, tam_runs(std::min(maxh, std::max(4096 / w, 1)), w));
+  return most;
+}
 
 // Summed-area table with the reference's exact recurrence
 //   S(y,x) = ((I(y,x) + S(y,x-1)) + S(y-1,x)) - S(y-1,x-1)
@@ -2478,14 +2489,17 @@ size_t tamura_scratch(int h, int w) { return tam_row(h, w) + w + 8; }
 // A wave's next strip begins T groups after its last, T >= 5 nw + 1, and what
 // wave 0 takes from the strip before it passes through a row in memory.  A
 // group's 64 x 16 inputs and results pass through an LDS tile, so that 16 lanes
-// access 128 consecutive bytes of a row.  Three planes of 1388 x 1040 and their
+// access 128 consecutive bytes of a row.  A block has as many waves, and LDS, as
+// the highest plane has strips (2,000 planes of 16 x 16: 20 us, 47 with LDS for
+// eight).  Three planes of 1388 x 1040 and their
 // transforms (18 planes): 1.2 ms, 9.0 ms with one wave per plane that met at
 // two barriers per step; 4,800 planes of up to 256 x 256 (7.6 GB moved): 3.0 ms.
-constexpr int SAT_WAVES = 8;
+constexpr int SAT_WAVES = 8, SAT_GR = 16, SAT_TILE = 64 * (SAT_GR + 1);
 __global__ void __launch_bounds__(64 * SAT_WAVES) k_tam_sat(const Img *imgs, double *const *scr) {
-  constexpr int GR = 16, LAG = 5;
-  __shared__ double tiles[SAT_WAVES][64 * (GR + 1)];
-  __shared__ double rings[SAT_WAVES][64];
+  constexpr int GR = SAT_GR, LAG = 5;
+  extern __shared__ double sat_lds[];  // a tile and a ring per wave
+  double (*const tiles)[SAT_TILE] = (double (*)[SAT_TILE])sat_lds;
+  double (*const rings)[64] = (double (*)[64])(sat_lds + (blockDim.x >> 6) * SAT_TILE);
   const Img im = imgs[blockIdx.x];
   const int H = im.h, W = im.w;
   const long P = (long)H * W;
@@ -2584,13 +2598,12 @@ __global__ void __launch_bounds__(64 * SAT_WAVES) k_tam_sat(const Img *imgs, dou
 // doubles.  Not so where the quotient is subnormal, which can lie in the very
 // middle, or where a is infinite and the remainder no number: these are divided.
 __device__ __forceinline__ double mean_diff(double a0, double c0, double r0, double a1, double c1, double r1) {
-  constexpr int SUBNORMAL = 0x10 | 0x80;  // of either sign, for v_cmp_class
+  constexpr int ODD = 0x3 | 0x10 | 0x80;  // for v_cmp_class: NaN, subnormal of either sign
   const double q0 = a0 * r0, q1 = a1 * r1;
   const double m0 = __builtin_fma(__builtin_fma(-c0, q0, a0), r0, q0);
   const double m1 = __builtin_fma(__builtin_fma(-c1, q1, a1), r1, q1);
   double v = fabs(m0 - m1);
-  if (__any(v != v || __builtin_amdgcn_class(m0, SUBNORMAL) || __builtin_amdgcn_class(m1, SUBNORMAL)))
-    v = fabs(a0 / c0 - a1 / c1);
+  if (__any(__builtin_amdgcn_class(m0, ODD) || __builtin_amdgcn_class(m1, ODD))) v = fabs(a0 / c0 - a1 / c1);
   return v;
 }
 
@@ -2602,7 +2615,7 @@ __device__ __forceinline__ double mean_diff(double a0, double c0, double r0, dou
 // (stop row, start column), of R where the window starts in row 0: one load.
 // Its divisor is full, a power of two, away from the borders.
 //
-// Bound by instruction issue, so a wave takes 64 columns and goes down TAM_ROWS
+// Bound by instruction issue, so a wave takes 64 columns and goes down tam_rows
 // rows: what depends on the row alone is scalar, and the rows' neighbours stay in
 // registers.  4,800 planes of up to 256 x 256: 9.9 ms; 18.0 ms with four table
 // entries per mean, 12.9 ms with one thread per pixel.
@@ -2617,7 +2630,7 @@ __global__ void __launch_bounds__(256, 3) k_tam_pix(const Img *imgs, double *con
   const long P = (long)H * W;
   const int run = __builtin_amdgcn_readfirstlane(blk * 4 + (threadIdx.x >> 6));
   if (run >= tam_runs(H, W)) return;
-  const int nc = (W + 63) / 64, y0 = run / nc * TAM_ROWS, x0 = run % nc * 64 + (threadIdx.x & 63);
+  const int rows = tam_rows(H, W), nc = (W + 63) / 64, y0 = run / nc * rows, x0 = run % nc * 64 + (threadIdx.x & 63);
   const bool own = x0 < W;
   const int x = min(x0, W - 1);
   const gptr<double> N = to_global(scr[ent]);  // global, not FLAT: vector-memory waits only
@@ -2642,7 +2655,7 @@ __global__ void __launch_bounds__(256, 3) k_tam_pix(const Img *imgs, double *con
   }
   TamPart T = {0, 0, 1e308, -1e308, 0, 0};
 #pragma unroll 1
-  for (int y = y0; y < min(y0 + TAM_ROWS, H); y++) {
+  for (int y = y0; y < min(y0 + rows, H); y++) {
     int xi = x;
     __asm__ volatile("" : "+v"(xi));  // formed anew per row: registers held through the loop cost more waves
     // coarseness: argmax over scales of E_h / E_v (tamura.cpp:183-238); the four
@@ -2739,19 +2752,17 @@ __global__ void __launch_bounds__(256, 3) k_tam_pix(const Img *imgs, double *con
   if ((threadIdx.x & 63) == 0) ((TamPart *)(scr[ent] + tam_parts(P)))[run] = T;
 }
 
-// the plane's sums from its parts; clears the histograms
-__global__ void __launch_bounds__(1024) k_tam_mid(const Img *imgs, double *const *scr) {
-  __shared__ double shd[16];
-  __shared__ long long shl[16];
-  __shared__ int shi[16];
-  const Img im = imgs[blockIdx.x];
+// The plane's sums from its parts; clears the histograms.  By one block of 256.
+__device__ __forceinline__ void tam_mid(const Img &im, const double *scr, TamSum &T) {
+  __shared__ double shd[4];
+  __shared__ long long shl[4];
+  __shared__ int shi[4];
   const long P = (long)im.h * im.w;
-  TamSum &T = *(TamSum *)(scr[blockIdx.x] + tam_summary(P));
-  const TamPart *part = (const TamPart *)(scr[blockIdx.x] + tam_parts(P));
+  const TamPart *part = (const TamPart *)(scr + tam_parts(P));
   double s = 0, sr = 0, pmn = 1e308, pmx = -1e308;
   long long ks = 0;
   int km = 0;
-  for (int b = threadIdx.x; b < tam_runs(im.h, im.w); b += 1024) {
+  for (int b = threadIdx.x; b < tam_runs(im.h, im.w); b += 256) {
     const TamPart q = part[b];
     s += q.s;
     sr += q.sr;
@@ -2780,18 +2791,15 @@ __global__ void __launch_bounds__(1024) k_tam_mid(const Img *imgs, double *const
   }
 }
 
-// contrast moments about the mean (Moments4, tamura.cpp:10-28) and the two
-// histograms, by block of TAM_CHUNK pixels
-__global__ void __launch_bounds__(256) k_tam_hist(const Img *imgs, double *const *scr) {
+// Contrast moments about the mean (Moments4, tamura.cpp:10-28) and the two
+// histograms of one TAM_CHUNK of pixels.  By a block of 256.
+__device__ __forceinline__ void tam_hist(const Img &im, const double *scr, int chunk, TamSum &T, TamPart2 *part) {
   __shared__ double shd[4];
   __shared__ int hk[3], hd[125];
-  const Img im = imgs[blockIdx.y];
-  const long P = (long)im.h * im.w, c0 = (long)blockIdx.x * TAM_CHUNK;
-  if (c0 >= P) return;
-  const gptr<const double> N = to_global((const double *)scr[blockIdx.y]);
+  const long P = (long)im.h * im.w, c0 = (long)chunk * TAM_CHUNK;
+  const gptr<const double> N = to_global(scr);
   const gptr<const double> phi = N + 2 * P;
   const gptr<const int> kb = (gptr<const int>)(N + 4 * P);
-  TamSum &T = *(TamSum *)(scr[blockIdx.y] + tam_summary(P));
   const double mean = T.mean, pmn = T.pmn, kmn = T.kmn;
   const double ksc = hist_scale(kmn, (double)T.kmx, 3), psc = hist_scale(pmn, T.pmx, 125);
   if (threadIdx.x < 3) hk[threadIdx.x] = 0;
@@ -2799,7 +2807,7 @@ __global__ void __launch_bounds__(256) k_tam_hist(const Img *imgs, double *const
   __syncthreads();
   double m2 = 0, m4 = 0;
   int wk0 = 0, wk1 = 0, wk2 = 0;
-  for (int r = 0; r < TAM_CHUNK; r += 256 * 4) {
+  for (int r = 0; r < min((long)TAM_CHUNK, P - c0); r += 256 * 4) {
     double v[4], p[4];
     int kk[4];
 #pragma unroll
@@ -2835,18 +2843,16 @@ __global__ void __launch_bounds__(256) k_tam_hist(const Img *imgs, double *const
   if (threadIdx.x < 125 && hd[threadIdx.x]) atomicAdd(&T.hd[threadIdx.x], hd[threadIdx.x]);
   m2 = block_reduce(m2, SumOp(), shd);
   m4 = block_reduce(m4, SumOp(), shd);
-  if (threadIdx.x == 0) ((TamPart2 *)(scr[blockIdx.y] + tam_parts2(im.h, im.w)))[blockIdx.x] = TamPart2{m2, m4};
+  if (threadIdx.x == 0) part[chunk] = TamPart2{m2, m4};
 }
 
-__global__ void __launch_bounds__(64) k_tam_final(const Img *imgs, double *const *scr, OutRef o) {
-  __shared__ double shd[1];
-  const Img im = imgs[blockIdx.x];
+// The features.  By a wave or more of a block.
+__device__ __forceinline__ void tam_final(const Img &im, const TamSum &T, const TamPart2 *part, double *out) {
+  __shared__ double shd[4];
   const int H = im.h, W = im.w;
   const long P = (long)H * W;
-  const TamSum &T = *(const TamSum *)(scr[blockIdx.x] + tam_summary(P));
-  const TamPart2 *part = (const TamPart2 *)(scr[blockIdx.x] + tam_parts2(im.h, im.w));
   double m2 = 0, m4 = 0;
-  for (long b = threadIdx.x; b < (P + TAM_CHUNK - 1) / TAM_CHUNK; b += 64) {
+  for (long b = threadIdx.x; b < (P + TAM_CHUNK - 1) / TAM_CHUNK; b += blockDim.x) {
     m2 += part[b].m2;
     m4 += part[b].m4;
   }
@@ -2856,7 +2862,6 @@ __global__ void __launch_bounds__(64) k_tam_final(const Img *imgs, double *const
     const int *hk = T.hk, *hd = T.hd;
     const long long ks = T.ks;
     const double sr = T.sr;
-    double *out = o.rows[blockIdx.x];
     // coarseness (tamura.cpp:240-262); the divisor is unsigned arithmetic
     const unsigned xD = W, yD = H;
     double sum = (double)ks;
@@ -2886,17 +2891,55 @@ __global__ void __launch_bounds__(64) k_tam_final(const Img *imgs, double *const
   }
 }
 
+// Planes of more than one chunk take three launches.  The others, which would
+// wait for launches more than work, take one, their sums in LDS: 2,000 planes of
+// 16 x 16 46 us, 117 by three launches.
+__device__ __forceinline__ TamSum &tam_sum(const Img &im, double *scr) { return *(TamSum *)(scr + tam_summary((long)im.h * im.w)); }
+__device__ __forceinline__ TamPart2 *tam_part2(const Img &im, double *scr) { return (TamPart2 *)(scr + tam_parts2(im.h, im.w)); }
+__global__ void __launch_bounds__(256) k_tam_mid(const Img *imgs, double *const *scr) {
+  const Img im = imgs[blockIdx.x];
+  if ((long)im.h * im.w > TAM_CHUNK) tam_mid(im, scr[blockIdx.x], tam_sum(im, scr[blockIdx.x]));
+}
+__global__ void __launch_bounds__(256) k_tam_hist(const Img *imgs, double *const *scr) {
+  const Img im = imgs[blockIdx.y];
+  const long P = (long)im.h * im.w;
+  double *const q = scr[blockIdx.y];
+  if (P > TAM_CHUNK && (long)blockIdx.x * TAM_CHUNK < P) tam_hist(im, q, blockIdx.x, tam_sum(im, q), tam_part2(im, q));
+}
+__global__ void __launch_bounds__(64) k_tam_final(const Img *imgs, double *const *scr, OutRef o) {
+  const Img im = imgs[blockIdx.x];
+  double *const q = scr[blockIdx.x];
+  if ((long)im.h * im.w > TAM_CHUNK) tam_final(im, tam_sum(im, q), tam_part2(im, q), o.rows[blockIdx.x]);
+}
+__global__ void __launch_bounds__(256) k_tam_small(const Img *imgs, double *const *scr, OutRef o) {
+  __shared__ TamSum sum;
+  __shared__ TamPart2 part;
+  const Img im = imgs[blockIdx.x];
+  if ((long)im.h * im.w > TAM_CHUNK) return;
+  tam_mid(im, scr[blockIdx.x], sum);
+  __syncthreads();
+  tam_hist(im, scr[blockIdx.x], 0, sum, &part);
+  __syncthreads();
+  tam_final(im, sum, &part, o.rows[blockIdx.x]);
+}
+
 void launch_tamura(const Img *imgs, const Stats *st, double *const *scratch, OutRef o, int nimg, int maxh, int maxw,
                    hipStream_t s) {
   const long maxn = (long)maxh * maxw;
-  const int blocks = (tam_runs(maxh, maxw) + 3) / 4;
-  const int nblocks = (int)((maxn / 4 + 255) / 256);
+  const int blocks = (tam_max_runs(maxh, maxw) + 3) / 4;
+  const int nblocks = (int)((maxn / 4 + 255) / 256), sat = std::min((maxh + 63) / 64, SAT_WAVES);
   k_tam_norm<<<dim3(nblocks < 1 ? 1 : (nblocks > 1024 ? 1024 : nblocks), nimg), 256, 0, s>>>(imgs, st, scratch);
-  k_tam_sat<<<nimg, 64 * std::min((maxh + 63) / 64, SAT_WAVES), 0, s>>>(imgs, scratch);
+  static const bool lds_ok = hipFuncSetAttribute((const void *)k_tam_sat, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                  SAT_WAVES * (SAT_TILE + 64) * sizeof(double)) == hipSuccess;
+  (void)lds_ok;
+  k_tam_sat<<<nimg, 64 * sat, sat * (SAT_TILE + 64) * sizeof(double), s>>>(imgs, scratch);
   k_tam_pix<<<xcd_grid(blocks, nimg), 256, 0, s>>>(imgs, scratch, nimg, blocks);
-  k_tam_mid<<<nimg, 1024, 0, s>>>(imgs, scratch);
-  k_tam_hist<<<dim3((unsigned)((maxn + TAM_CHUNK - 1) / TAM_CHUNK), nimg), 256, 0, s>>>(imgs, scratch);
-  k_tam_final<<<nimg, 64, 0, s>>>(imgs, scratch, o);
+  if (maxn > TAM_CHUNK) {
+    k_tam_mid<<<nimg, 256, 0, s>>>(imgs, scratch);
+    k_tam_hist<<<dim3((unsigned)((maxn + TAM_CHUNK - 1) / TAM_CHUNK), nimg), 256, 0, s>>>(imgs, scratch);
+    k_tam_final<<<nimg, 64, 0, s>>>(imgs, scratch, o);
+  }
+  k_tam_small<<<nimg, 256, 0, s>>>(imgs, scratch, o);
 }
 
 // ================================================================= Comb moments
