@@ -25,10 +25,6 @@ __device__ double otsu_threshold(const int *hist, long n, double mn, double mx) 
   for (int i = threadIdx.x; i < 1024; i += blockDim.x) pf[i] = hist[i] / wh;
   __syncthreads();
   if (threadIdx.x == 0) {
-    // myu[L-1] first (the recurrence below repeats the same operations)
-    double my_last = 0.0;
-    for (int i = 1; i < 1024; i++) my_last = my_last + i * pf[i];
-    my_last_s = my_last;
     double om = pf[0], my = 0.0;
     for (int i = 0; i < 1023; i++) {
       if (i > 0) {
@@ -38,6 +34,7 @@ __device__ double otsu_threshold(const int *hist, long n, double mn, double mx) 
       om_s[i] = om;
       my_s[i] = my;
     }
+    my_last_s = my + 1023 * pf[1023];  // myu[L-1], by the operations of the recurrence
   }
   __syncthreads();
   const double my_last = my_last_s;
@@ -1240,7 +1237,7 @@ __global__ void __launch_bounds__(256) k_gabor_repair(const Img *imgs, const dou
 // pixels.  Bound by memory: 12 bytes per pixel and filter and step.  Three planes
 // of 1388 x 1040: 0.8 ms for all steps, 10.1 ms with one block per (image,
 // filter); 64 planes of 64..1024 pixels a side: 2.6, 8.1 ms; 400 of 256 x 256:
-// 4.3, 4.5 ms; one of 128 x 128: 0.13, 0.12 ms (the threshold's chain of 1,024
+// 4.3, 4.5 ms; one of 128 x 128: 0.115, 0.12 ms (the threshold's chain of 1,024
 // bins and the launches).
 enum GaborStep { GP_LOW, GP_MARK_TOP, GP_MAX, GP_LEVEL, GP_MARK_LOW, GP_RANGE, GP_MARK_BIN, GP_HIST, GP_MARK_THR, GP_COUNT };
 constexpr int GP_CHUNK = 8192;
