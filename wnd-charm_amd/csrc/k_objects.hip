@@ -913,7 +913,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))
 // each: |E - E64| <= 1.8e-13 S + 4u E.  D = coef * tmax * wsum_f + 1e-14 E with
 // coef = 4e-13 times the context's slack, rounded up.  Where a block's largest
 // |x| is so small that D would leave float's range, so large that a sum could
-// overflow, or infinite, its energies are the plain sums over the 1,444 taps.
+// overflow, or infinite, its energies are E64 itself: the 1,444 products, each
+// rounded and added in k_gabor_conv's order, with D = 0.
 //
 // A block takes 27 x 64 outputs, i.e. 64 rows of 101 inputs, and `per` filters.
 // Each of 512 threads forms eight adjacent row sums of both kinds from a sliding
@@ -963,14 +964,18 @@ __global__ void __launch_bounds__(512) k_gabor_sep(const Img *imgs, const double
     if (!sized) {
       const double *K = kernels + (long)f * GB_N * GB_N * 2;
       for (int r = wave; r < GS_TR; r += 8) {
+        const int y = b0 + r, x = a0 + lane;
         double re = 0.0, imv = 0.0;
         for (int j = 0; j < GB_N; j++)
           for (int i = 0; i < GB_N; i++) {
             const double v = tile[r + 37 - j][lane + 37 - i];
-            re = fma(v, K[2 * (j * GB_N + i)], re);
-            imv = fma(v, K[2 * (j * GB_N + i) + 1], imv);
+            re += v * K[2 * (j * GB_N + i)];
+            imv += v * K[2 * (j * GB_N + i) + 1];
           }
-        put(b0 + r, a0 + lane, re, imv);
+        if (y >= im.h || x >= im.w) continue;
+        const double e = sqrt(re * re + imv * imv);
+        E[(long)y * im.w + x] = e;
+        D[(long)y * im.w + x] = e == e ? 0.0f : (float)e;  // (NaN stays undecided, as elsewhere)
       }
       continue;
     }
