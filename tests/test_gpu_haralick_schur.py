@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 import wndcharm
-from helpers import ALG_NAMES, orc_algorithm
+from helpers import ALG_NAMES, features_in_context, orc_algorithm
 
 pytestmark = pytest.mark.gpu
 
@@ -88,3 +88,19 @@ def test_kernel_picked_by_tones(kind, n):
     one = np.concatenate([wndcharm.compute_features([im], plan) for im in kinds])
     assert np.array_equal(got, one[np.arange(n) % 9], equal_nan=True)
     assert np.array_equal(work, work[np.arange(n) % 9]) and (work > 0).all()
+
+
+@pytest.mark.parametrize('n', [1, 100, 300])
+def test_a_wait_in_vain_fails_the_call(n):
+    """no polls: a wave that does not find the reflectors at once gives up, the
+    kernel ends, and the call fails instead of returning what a stale reflector
+    gave; another context is not affected"""
+    imgs = [toned(150, k, (40, 56)) for k in range(3)]
+    plan = wndcharm.FeatureComputationPlan('haralick')
+    plan.add('Haralick Textures ()')
+    plan.finalize()
+    print('schur without polls', n, flush=True)
+    want = wndcharm.compute_features(imgs, plan)
+    with pytest.raises(wndcharm.WndGpuError):
+        features_in_context({'WNDGPU_SCHUR_NO_POLLS': '1'}, [imgs[k % 3] for k in range(n)], plan)
+    assert np.array_equal(wndcharm.compute_features(imgs, plan), want, equal_nan=True)

@@ -369,6 +369,12 @@ struct wndgpu_ctx {
   // gabor_slack (WNDGPU_GABOR_SLACK, >= 1) scales the certification bound.
   bool gabor_direct = false;
   double gabor_slack = 1;
+  // *schur_lost (pinned): a wave of the Schur kernel gave up waiting for
+  // another's result, and the call fails.  They give up after most of a second,
+  // where the result takes microseconds, or at once (WNDGPU_SCHUR_NO_POLLS, for
+  // tests).
+  int *schur_lost = nullptr;
+  bool schur_no_polls = false;
   // Radon projections: order-free sums whose histogram counts are
   // certified (the default), or the reference's sequential sum per bin
   // (radon_direct, WNDGPU_RADON_DIRECT=1 at creation).  radon_slack
@@ -1171,6 +1177,8 @@ static int build_batch(wndgpu_ctx *c, const wndgpu_plan *plan, const Batch &B, A
           c->har_n = ne;
         }
         HarDesc *hdd = A.stage(hd);
+        const bool no_polls = c->schur_no_polls;
+        int *const lost = c->schur_lost;
         push_side(gn + " [co-occurrence, f1-f13, Q]", [=](hipStream_t s2) {
           launch_gather_stats(sts, nst, ne, s2);
           launch_fill_int(lut_all, 256 * (long)ne, 0, s2);
@@ -1178,8 +1186,8 @@ static int build_batch(wndgpu_ctx *c, const wndgpu_plan *plan, const Batch &B, A
           launch_haralick_order(ng_all, ne, order, s2);
         });
         push_side(gn + " [k_har_hess]", [=](hipStream_t s2) { launch_haralick_hess(hdd, order, ne, s2); });
-        push_side(gn + " [k_har_qr]", [=](hipStream_t s2) { launch_haralick_qr(hdd, order, ne, s2); });
-        push_side(gn + " [mean, range]", [=](hipStream_t s2) { launch_haralick_final(hdd, o, ne, s2); });
+        push_side(gn + " [k_har_qr]", [=](hipStream_t s2) { launch_haralick_qr(hdd, order, no_polls, ne, s2); });
+        push_side(gn + " [mean, range]", [=](hipStream_t s2) { launch_haralick_final(hdd, o, lost, ne, s2); });
       } break;
       case A_ZERNIKE: {
         const int nchunk = (int)std::max<long>(1, std::min<long>(64, (maxp + 4095) / 4096));
@@ -1791,11 +1799,13 @@ int wndgpu_create(int device, wndgpu_ctx **out) {
     delete c;
     return WNDGPU_E_DEVICE;
   }
-  if (scratch_address(device, &c->scratch) != hipSuccess) {
+  if (scratch_address(device, &c->scratch) != hipSuccess ||
+      hipHostMalloc((void **)&c->schur_lost, sizeof(int), hipHostMallocDefault) != hipSuccess) {
     release_check(hipStreamDestroy(c->stream), "hipStreamDestroy");
     delete c;
     return WNDGPU_E_DEVICE;
   }
+  *c->schur_lost = 0;
   if (hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess ||
       hipStreamCreateWithFlags(&c->fstream, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&c->fork_ev, hipEventDisableTiming) != hipSuccess ||
@@ -1807,6 +1817,7 @@ int wndgpu_create(int device, wndgpu_ctx **out) {
     if (c->fstream) release_check(hipStreamDestroy(c->fstream), "hipStreamDestroy");
     if (c->side) release_check(hipStreamDestroy(c->side), "hipStreamDestroy");
     release_check(hipStreamDestroy(c->stream), "hipStreamDestroy");
+    release_check(hipHostFree(c->schur_lost), "hipHostFree");
     delete c;
     return WNDGPU_E_DEVICE;
   }
@@ -1824,6 +1835,7 @@ int wndgpu_create(int device, wndgpu_ctx **out) {
   if (const char *cs = getenv("WNDGPU_CF_SLACK")) c->cf_slack = std::max(1.0, atof(cs));
   if (const char *gd = getenv("WNDGPU_GABOR_DIRECT")) c->gabor_direct = atoi(gd) != 0;
   if (const char *gs = getenv("WNDGPU_GABOR_SLACK")) c->gabor_slack = std::max(1.0, atof(gs));
+  if (const char *sp = getenv("WNDGPU_SCHUR_NO_POLLS")) c->schur_no_polls = atoi(sp) != 0;
   if (const char *rd = getenv("WNDGPU_RADON_DIRECT")) c->radon_direct = atoi(rd) != 0;
   if (const char *rs = getenv("WNDGPU_RADON_SLACK")) c->radon_slack = std::max(1.0, atof(rs));
   if (const char *gm = getenv("WNDGPU_GRAPH")) c->graph_mode = std::min(2, std::max(0, atoi(gm)));
@@ -1863,6 +1875,7 @@ void wndgpu_destroy(wndgpu_ctx *c) {
   if (c->dev) release_check(hipFree(c->dev), "hipFree");
   if (c->hdesc) release_check(hipFree(c->hdesc), "hipFree");
   if (c->host) release_check(hipHostFree(c->host), "hipHostFree");
+  release_check(hipHostFree(c->schur_lost), "hipHostFree");
   release_check(hipEventDestroy(c->fork_ev), "hipEventDestroy");
   release_check(hipEventDestroy(c->join_ev), "hipEventDestroy");
   release_check(hipEventDestroy(c->fjoin_ev), "hipEventDestroy");
@@ -2100,6 +2113,7 @@ static int compute_common(wndgpu_ctx *c, const wndgpu_plan *plan, const wndgpu_i
   B.out = dout;
   c->t_table_ms = 0;
   const auto t_run = std::chrono::steady_clock::now();
+  *c->schur_lost = 0;
   int r = run_batch(c, plan, B, getenv("WNDGPU_TIMING") != nullptr);
   c->t_host_ms = ms_since(t_run);
   const auto t_dev = std::chrono::steady_clock::now();
@@ -2138,6 +2152,7 @@ static int compute_common(wndgpu_ctx *c, const wndgpu_plan *plan, const wndgpu_i
     c->times.emplace_back(c->tnames[k], ms);
   }
   c->tnames.clear();
+  if (*c->schur_lost) return fail(c, WNDGPU_E_DEVICE, "Haralick f14: a wave waited in vain for another's result");
   return rejected ? fail(c, WNDGPU_E_IMAGE, "some images were rejected (see status)") : WNDGPU_OK;
 }
 

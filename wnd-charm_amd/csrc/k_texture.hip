@@ -1664,7 +1664,9 @@ __device__ __forceinline__ void schur_right(unsigned on, const SchurRf *rf, doub
   row[PB + 1] = u1;
 }
 
-template <int NW>
+// POLLS: how often a wave looks for another's result before it gives up
+constexpr int SCHUR_POLLS = 1 << 24;  // most of a second
+template <int NW, int POLLS = SCHUR_POLLS>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
 k_har_schur(const HarDesc *hd, const int *order, const int *pick) {
   if (pick && *pick == 0) return;  // uniform: k_har_qr takes the launch
@@ -2206,12 +2208,18 @@ k_har_schur(const HarDesc *hd, const int *order, const int *pick) {
           }
           if (__ballot(act) != 0) {
             const SchurRf *R = rf[par];
-            // wave 0 publishes every step of its window
+            // wave 0 publishes every step of its window, within microseconds.
+            // Should it not, the sweeps end all the same (their number is
+            // limited), on what lies in LDS, and k_har_final fails the call
             auto await = [&](int q) {
-              for (int spin = 0; spin < (1 << 24); spin++) {
+              for (int spin = 0;; spin++) {
                 if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(&R[q].gen, __ATOMIC_RELAXED,
                                                                      __HIP_MEMORY_SCOPE_WORKGROUP)) == base + q + 1)
                   break;
+                if (spin == POLLS) {
+                  H.count[angle] = -1;
+                  break;
+                }
                 __builtin_amdgcn_s_sleep(1);
               }
               __asm__ volatile("" ::: "memory");
@@ -2278,9 +2286,12 @@ k_har_schur(const HarDesc *hd, const int *order, const int *pick) {
 }
 
 // mean and range over the 4 angles, reference output order (haralick.cpp:96-143)
-__global__ void k_har_final(const HarDesc *hd, OutRef o) {
+// *lost: a wave of k_har_schur waited in vain
+__global__ void k_har_final(const HarDesc *hd, OutRef o, int *lost) {
   const HarDesc H = hd[blockIdx.x];
   if (threadIdx.x != 0) return;
+  for (int g = 0; g < 4; g++)
+    if (H.count[g] < 0) __hip_atomic_store(lost, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   double temp[28];
   for (int a = 0; a < 14; a++) {
     double s = 0, mn = kInf, mx = -kInf;
@@ -2384,7 +2395,7 @@ void launch_haralick_hess(const HarDesc *hd, const int *order, int nimg, hipStre
   k_har_hess<<<dim3(4, nimg), 512, 0, s>>>(hd, order);
   k_har_hess_rows<<<dim3(4, nimg, (256 - 2 + RWS - 1) / RWS), 64, 0, s>>>(hd, order);
 }
-void launch_haralick_qr(const HarDesc *hd, const int *order, int nimg, hipStream_t s) {
+void launch_haralick_qr(const HarDesc *hd, const int *order, bool no_polls, int nimg, hipStream_t s) {
   // Up to 256 matrices every CU has at most one, and the launch lasts as long
   // as the longest chain of steps: eight waves per matrix.  Up to 1024, four
   // waves per matrix, two matrices per CU: with tones of 8 .. 240, equal or
@@ -2401,12 +2412,13 @@ void launch_haralick_qr(const HarDesc *hd, const int *order, int nimg, hipStream
   // against 93.9, 9600 112.0 against 124.8, 19200 201 against 259.
   const dim3 grid(4, nimg);
   const int *pick = haralick_pick(nimg) ? order + nimg : nullptr;
-  if (4 * nimg <= 256) k_har_schur<8><<<grid, 512, 0, s>>>(hd, order, nullptr);
+  if (no_polls) k_har_schur<4, 0><<<grid, 256, 0, s>>>(hd, order, nullptr);
+  else if (4 * nimg <= 256) k_har_schur<8><<<grid, 512, 0, s>>>(hd, order, nullptr);
   else if (4 * nimg <= 6144) k_har_schur<4><<<grid, 256, 0, s>>>(hd, order, pick);
-  if (pick || 4 * nimg > 6144) k_har_qr<<<grid, 64, 0, s>>>(hd, order, pick);
+  if (!no_polls && (pick || 4 * nimg > 6144)) k_har_qr<<<grid, 64, 0, s>>>(hd, order, pick);
 }
-void launch_haralick_final(const HarDesc *hd, OutRef o, int nimg, hipStream_t s) {
-  k_har_final<<<nimg, 64, 0, s>>>(hd, o);
+void launch_haralick_final(const HarDesc *hd, OutRef o, int *lost, int nimg, hipStream_t s) {
+  k_har_final<<<nimg, 64, 0, s>>>(hd, o, lost);
 }
 
 // ======================================================================= Tamura
