@@ -1428,8 +1428,5 @@ void launch_gabor_certified(const Img *imgs, const double *kernels, const double
   k_gabor_sep<<<dim3(tiles, 8 / per, nimg), 512, 0, s>>>(imgs, factors, kernels, energy, wsum, bound, 4e-13 * slack, per);
   launch_gabor_post_exact(imgs, energy, bound, kernels, state, flags, slack <= 1.0, o, nimg, maxh, maxw, s);
 }
-void launch_gabor_post(const Img *imgs, double *const *energy, OutRef o, int nimg, hipStream_t s) {
-  k_gabor_post<<<nimg, 1024, 0, s>>>(imgs, energy, o);
-}
 
 }  // namespace wnd

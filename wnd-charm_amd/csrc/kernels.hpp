@@ -207,7 +207,6 @@ void launch_median(const Img *planes, const Stats *st, SelState *sel, uint64_t *
 struct EdgeCounts { int area, hm[8], hd[8]; };
 void launch_edge_final(const Img *mag, const Img *dir, const Stats *st2, const double *medians, EdgeCounts *cnt, OutRef o,
                        int nimg, long maxn, hipStream_t s);
-void launch_gabor_post(const Img *imgs, double *const *energy, OutRef o, int nimg, hipStream_t s);
 // scratch of the exact Gabor post-processing, per (image, filter)
 struct GaborState {
   unsigned long long lo, mx, hi_min, a, b;  // keys (dkey): lower end of the top, maximum, upper end of the minimum, range of e / mx
