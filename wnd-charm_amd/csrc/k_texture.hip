@@ -11,6 +11,7 @@
 #include <utility>
 #include "common.hpp"
 #include "kernels.hpp"
+#include "schur_math.hpp"
 
 namespace wnd {
 
@@ -1581,36 +1582,6 @@ __device__ __forceinline__ double lane_value(double v, int lane) {
   return __longlong_as_double(((long long)hi << 32) | lo);
 }
 
-// a / d and b / d with d's reciprocal y formed once: Newton steps to y, then
-// the quotient corrected by its exact remainder (Markstein).  Operands must
-// lie well inside the normal range (schur_in_range): the results are then the
-// correctly rounded quotients.
-__device__ __forceinline__ double recip_seed(double d) {
-  double y = __builtin_amdgcn_rcp(d);
-  double e = __builtin_fma(-d, y, 1.0);
-  y = __builtin_fma(y, e, y);
-  e = __builtin_fma(-d, y, 1.0);
-  return __builtin_fma(y, e, y);
-}
-__device__ __forceinline__ double quot(double a, double d, double y) {
-  const double q = a * y;
-  const double r = __builtin_fma(-d, q, a);
-  return __builtin_fma(r, y, q);
-}
-// sqrt(a) by a coupled Newton iteration on sqrt and 1 / (2 sqrt) with two
-// remainder corrections, for a well inside the normal range
-__device__ __forceinline__ double root(double a) {
-  const double y = __builtin_amdgcn_rsq(a);
-  double g = a * y, h = y * 0.5;
-  const double r = __builtin_fma(-h, g, 0.5);
-  g = __builtin_fma(g, r, g);
-  h = __builtin_fma(h, r, h);
-  double d = __builtin_fma(-g, g, a);
-  g = __builtin_fma(d, h, g);
-  d = __builtin_fma(-g, g, a);
-  return __builtin_fma(d, h, g);
-}
-
 struct __align__(16) SchurRf {
   double tau, e0, e1;
   int gen, app;  // step number; whether the reflector is applied (beta != 0)
@@ -2012,10 +1983,11 @@ k_har_schur(const HarDesc *hd, const int *order, const int *pick) {
           if (__builtin_expect(__ballot(least >= 0x1p-350) == 0, 0)) return false;
           double tail = x1 * x1;
           tail += x2 * x2;
-          double bb = root(x0 * x0 + tail);
+          const double sq = x0 * x0 + tail;
+          double bb = root(sq, __builtin_amdgcn_rsq(sq));
           if (x0 >= 0) bb = -bb;
           const double den = x0 - bb;
-          const double yd = recip_seed(den), yb = recip_seed(bb);
+          const double yd = recip(den, __builtin_amdgcn_rcp(den)), yb = recip(bb, __builtin_amdgcn_rcp(bb));
           const double e0 = quot(x1, den, yd), e1 = quot(x2, den, yd);
           const double tau = quot(-den, bb, yb);  // bb - x0 = -den exactly
           const schur_d2 o0 = {tau, e0}, o1 = {e1, __longlong_as_double((1ll << 32) | (unsigned)(base + q + 1))};
