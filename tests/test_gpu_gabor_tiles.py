@@ -82,7 +82,9 @@ def test_blocks_of_small_pixels_beside_others(small):
 
 @pytest.mark.parametrize('value', [np.inf, -np.inf, 0.0])
 def test_blocks_with_an_odd_value(value):
-    """in one block's window only; a plane of zeros"""
+    """in one block's window only; a plane of zeros.  An infinite maximum leaves no
+    base count, so the ratios are NaN on both paths: the energies of such blocks are
+    compared by test_energies_next_to_a_level, which takes the same branch."""
     print('gabor tiles:', value, flush=True)
     a = image((90, 200), 4)
     a[40, 100] = value

@@ -4,7 +4,8 @@ bands and launch rules have edges, bit for bit against the oracle.
 The small-launch kernel chases a bulge in windows of 16 steps, keeps a band of
 64 columns in a wave and updates rows above a window 64 at a time, so matrix
 orders around multiples of 16 and 64 (order = number of gray tones) exercise
-its remainders; order 256 is the largest, and orders below 3 have no f14.
+its remainders; the Hessenberg reduction keeps more columns in LDS from 171 and
+129 tones down and updates the rows above 32 at a time; order 256 is the largest, and orders below 3 have no f14.
 Launches of up to 256 matrices, up to 6144 and beyond take different kernels,
 and from 1025 to 6144 the tones decide between two of them."""
 import numpy as np
@@ -32,8 +33,8 @@ def toned(ng, seed, shape=(40, 56)):
     return np.sort(tones)[idx]
 
 
-@pytest.mark.parametrize('ng', [1, 2, 3, 4, 5, 17, 18, 19, 20, 33, 34, 35, 63, 64, 65, 66, 80, 81, 82, 83, 127, 130,
-                                194, 195, 255, 256])
+@pytest.mark.parametrize('ng', [1, 2, 3, 4, 5, 17, 18, 19, 20, 33, 34, 35, 63, 64, 65, 66, 80, 81, 82, 83, 98, 99, 127, 128, 129,
+                                130, 162, 163, 171, 172, 194, 195, 255, 256])
 def test_schur_orders_equal_oracle(ng):
     img = toned(ng, 3, (64, 72) if ng > 128 else (40, 56))
     print('schur order', ng, flush=True)

@@ -81,3 +81,61 @@ def test_more_planes_than_a_grid_dimension_holds():
     print('objects and edges: 33,000 images', flush=True)
     many = wndcharm.compute_features(imgs * 825, plan)
     assert np.array_equal(many, np.tile(some, (825, 1)), equal_nan=True)
+
+
+ODD = {'nan': [np.nan], '+inf': [np.inf], '-inf': [-np.inf], 'all': [np.nan, np.inf, -np.inf]}
+
+
+def odd_pixels(img, kind, seed):
+    """the plane with seven pixels of each odd value"""
+    rng = np.random.default_rng(seed)
+    img = np.array(img, np.float64)
+    for value in ODD[kind]:
+        img.reshape(-1)[rng.permutation(img.size)[:7]] = value
+    return img
+
+
+@pytest.mark.parametrize('kind', list(ODD))
+@pytest.mark.parametrize('shape', [(64, 70), (131, 130)])
+def test_objects_with_odd_pixels(shape, kind):
+    """The range is that of the finite pixels, infinities count in the outermost
+    bins and lie on their side of the threshold, as the finite extremes do that
+    the oracle gets in their place (its histogram converts them to integers, which
+    C leaves undefined); NaN is in no mask."""
+    print('objects', shape, kind, flush=True)
+    img = odd_pixels(winding(*shape, seed=1), kind, 2)
+    finite = img[np.isfinite(img)]
+    oracle_img = np.where(img == np.inf, finite.max(), np.where(img == -np.inf, finite.min(), img))
+    for alg in ('Otsu Object Features', 'Inverse-Otsu Object Features'):
+        got = np.asarray(wndcharm.FeatureAlgorithm(alg).execute(img))
+        want = orc_algorithm(ALG_NAMES.index(alg), oracle_img)
+        assert np.array_equal(got[OBJ_EXACT], want[OBJ_EXACT]), (alg, got, want)
+        assert np.allclose(got, want, rtol=1e-9, atol=1e-9), (alg, got, want)
+
+
+def prewitt(a):
+    """the gradient's magnitude; sums of whole numbers, so in any order"""
+    p = np.pad(a, 1)
+    with np.errstate(invalid='ignore'):
+        sx = sum(p[j:j + a.shape[0], :-2] - p[j:j + a.shape[0], 2:] for j in range(3))
+        sy = sum(p[:-2, k:k + a.shape[1]] - p[2:, k:k + a.shape[1]] for k in range(3))
+        return np.sqrt(sx * sx + sy * sy)
+
+
+@pytest.mark.parametrize('kind', list(ODD))
+@pytest.mark.parametrize('shape', [(64, 70), (63, 71), (131, 130), (131, 131)])
+@pytest.mark.parametrize('crowded', [False, True])
+def test_edge_medians_with_odd_pixels(shape, kind, crowded):
+    """the magnitude's median with infinite and NaN magnitudes among the sorted
+    values: each NaN at the one end or the other by its sign, which depends on
+    whether its pixel was added or subtracted and on the machine, so any number of
+    them below the rest; crowded: most magnitudes are 0 and so in one bin"""
+    print('edge', shape, kind, crowded, flush=True)
+    rng = np.random.default_rng(sum(shape))
+    img = np.full(shape, 50.0) if crowded else np.round(rng.normal(100, 30, shape))
+    img = odd_pixels(img, kind, 3)
+    m = np.sort(prewitt(img).reshape(-1))  # NaN last
+    nans = int(np.isnan(m).sum())
+    got = np.asarray(wndcharm.FeatureAlgorithm('Edge Features').execute(img))[26]
+    want = [(v[(m.size - 1) // 2] + v[m.size // 2]) / 2 for v in (np.roll(m, k) for k in range(nans + 1))]
+    assert got in want, (got, want)

@@ -15,6 +15,7 @@ from helpers import ALG_NAMES, orc_algorithm
 
 pytestmark = pytest.mark.gpu
 ALG = 'Tamura Textures'
+COARSENESS = [0, 1, 2, 5]
 
 
 def check(img):
@@ -71,3 +72,19 @@ def test_planes_of_all_kinds_in_one_call():
     one = np.concatenate([wndcharm.compute_features([im], plan) for im in imgs])
     assert np.array_equal(wndcharm.compute_features(imgs, plan), one, equal_nan=True)
     assert np.array_equal(wndcharm.compute_features(imgs[:5], plan), one[:5], equal_nan=True)
+
+
+@pytest.mark.parametrize('value', [np.nan, np.inf, -np.inf, 1e39])
+def test_odd_pixels(value):
+    """One odd pixel poisons the table's entries right of and below it, and every
+    window mean from them; 1e39 is finite but beyond what the statistics count.
+    Compared are the coarseness and its histogram: contrast and direction add up
+    the odd pixels themselves, which the oracle leaves out."""
+    print('tamura', value, flush=True)
+    rng = np.random.default_rng(8)
+    for at in ((0, 0), (40, 80), (129, 149), (100, 3), (64, 0)):
+        img = np.round(rng.normal(100, 30, (130, 150)))
+        img[at] = value
+        got = np.asarray(wndcharm.FeatureAlgorithm(ALG).execute(img))
+        want = orc_algorithm(ALG_NAMES.index(ALG), img)
+        assert np.allclose(got[COARSENESS], want[COARSENESS], rtol=1e-9, atol=1e-12, equal_nan=True), (at, got, want)
