@@ -33,7 +33,7 @@ def toned(ng, seed, shape=(40, 56)):
     return np.sort(tones)[idx]
 
 
-@pytest.mark.parametrize('ng', [1, 2, 3, 4, 5, 17, 18, 19, 20, 33, 34, 35, 63, 64, 65, 66, 80, 81, 82, 83, 98, 99, 127, 128, 129,
+@pytest.mark.parametrize('ng', [1, 2, 3, 4, 5, 17, 18, 19, 20, 31, 32, 33, 34, 35, 63, 64, 65, 66, 80, 81, 82, 83, 98, 99, 127, 128, 129,
                                 130, 162, 163, 171, 172, 194, 195, 255, 256])
 def test_schur_orders_equal_oracle(ng):
     img = toned(ng, 3, (64, 72) if ng > 128 else (40, 56))

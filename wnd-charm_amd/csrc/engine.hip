@@ -1156,7 +1156,7 @@ static int build_batch(wndgpu_ctx *c, const wndgpu_plan *plan, const Batch &B, A
         int *lut_all = A.dalloc_n<int>(256 * (size_t)ne);
         int *ng_all = A.dalloc_n<int>(ne);
         double *work_all = A.dalloc_n<double>(4 * (size_t)ne);
-        int *order = A.dalloc_n<int>(ne + 1);  // and the kernel picked for the Schur form
+        int *order = A.dalloc_n<int>(ne + ORDER_EXTRA);
         for (int k = 0; k < ne; k++) {
           HarDesc &H = hd[k];
           H.img = nullptr;

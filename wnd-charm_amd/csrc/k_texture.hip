@@ -487,6 +487,12 @@ __device__ __forceinline__ double lane_xor1(double v) {
 constexpr int HT8 = 9;          // padded row of a wave's 32 x 8 staging tile
 constexpr int HTW = 32 * HT8;   // a wave's tile
 constexpr int HCAP = 16384;     // doubles of the matrix kept in LDS
+// k_har_hess takes a CU per matrix.  Where HESS_MANY entries or more have at most
+// HESS_SMALL tones, a launch of one wave and 12 KB of LDS per matrix takes those:
+// 4,000 matrices of 4 tones 72 us (164 by whole CUs, 132 before there were such),
+// of 16 252 (773, 903), of 32 565 (1796, 2133).  It would follow the large ones'
+// launch, though, and fewer small matrices run beside those for nothing.
+constexpr int HESS_SMALL = 32, HESS_MANY = 256;
 // all waves' LDS accesses complete; global stores may be in flight
 __device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -530,19 +536,23 @@ __device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkm
 // 19,200 (0.77 TB at the fabric's 4.6 TB/s), now 132.
 // Eigen's last step (one row below the diagonal) scales by 1 - tau with
 // tau = 0 (a one-element reflector): an exact no-op, not performed.
-__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <int NW, int NMAX>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, NW == 1 ? 4 : 2)))
 k_har_hess(const HarDesc *hd, const int *order) {
-  __shared__ double res[HCAP];          // resident columns
-  __shared__ __align__(16) double tile[8 * HTW];  // per wave: staging; then the squares of its rows' x
-  __shared__ __align__(16) double2 twe[256];      // by column: left dot, essential element of step i
-  __shared__ __align__(16) double2 tun[256];      // by row: tau * right dot of step i, essential of step i (row pass) / i+1 (column pass)
-  __shared__ double lf[256];            // by row: left factor of step i
-  __shared__ double xc[256];            // by row: column i+1 after step i
+  constexpr bool SMALL = NMAX <= 32;    // every column resident, rows and columns of one wave
+  __shared__ double res[SMALL ? NMAX * 32 : HCAP];  // resident columns
+  __shared__ __align__(16) double tile[NW * HTW];  // per wave: staging; then the squares of its rows' x
+  __shared__ __align__(16) double2 twe[NMAX];      // by column: left dot, essential element of step i
+  __shared__ __align__(16) double2 tun[NMAX];      // by row: tau * right dot of step i, essential of step i (row pass) / i+1 (column pass)
+  __shared__ double lf[NMAX];            // by row: left factor of step i
+  __shared__ double xc[NMAX];            // by row: column i+1 after step i
   __shared__ double sc[4];
+  // entries by decreasing n: the large ones, the small ones, those of n < 3 (Hessenberg as they are)
+  const int e = blockIdx.y, first = SMALL ? order[gridDim.y + ORDER_LARGE] : 0;
+  if (e < first || e >= order[gridDim.y + (SMALL ? ORDER_END : ORDER_LARGE)]) return;
   const int angle = blockIdx.x;
   const HarDesc H = hd[order[blockIdx.y]];
   const int n = __builtin_amdgcn_readfirstlane(*H.ng);
-  if (n < 2) return;
   gptr<double> A = to_global(H.Q + (long)angle * n * n);
   gptr<double> Rf = to_global(H.P + (long)angle * n * n);  // reflector store
   const int t = threadIdx.x, lane = t & 63;
@@ -612,26 +622,27 @@ k_har_hess(const HarDesc *hd, const int *order) {
 
   // the resident columns back to global memory, rows from r1 on
   auto flush = [&](int r1) {
-    for (int r = r1 + wave; r < n; r += 8)
+    for (int r = r1 + wave; r < n; r += NW)
       for (int c = max(cK, r1) + lane; c < n; c += 64) AT(r, c) = RES(r, c);
   };
+  // resident columns of R rows
+  auto columns = [](int R) { return SMALL ? 32 : R <= 128 ? 128 : R <= 170 ? 96 : 64; };
   // residency for rows r1..n-1
   auto reside = [&](int r1) {
-    const int R = n - r1;
-    K = R <= 128 ? 128 : R <= 170 ? 96 : 64;
+    K = columns(n - r1);
     cK = max(n - K, 0);
     r0 = r1;
-    for (int ra = r1 + wave; ra < n; ra += 32) {
+    for (int ra = r1 + wave; ra < n; ra += 4 * NW) {
       double v[4][2];
 #pragma unroll
       for (int k = 0; k < 4; k++)
 #pragma unroll
-        for (int j = 0; j < 2; j++) v[k][j] = AT(min(ra + 8 * k, n - 1), min(cK + lane + 64 * j, n - 1));
+        for (int j = 0; j < 2; j++) v[k][j] = AT(min(ra + NW * k, n - 1), min(cK + lane + 64 * j, n - 1));
 #pragma unroll
       for (int k = 0; k < 4; k++)
 #pragma unroll
         for (int j = 0; j < 2; j++)
-          if (ra + 8 * k < n && cK + lane + 64 * j < n && lane + 64 * j < K) RES(ra + 8 * k, cK + lane + 64 * j) = v[k][j];
+          if (ra + NW * k < n && cK + lane + 64 * j < n && lane + 64 * j < K) RES(ra + NW * k, cK + lane + 64 * j) = v[k][j];
     }
   };
 
@@ -747,8 +758,8 @@ k_har_hess(const HarDesc *hd, const int *order) {
   };
 
   // step 0's reflector and left dot
-  for (int r = t; r < 256; r += 512) tun[r] = double2{0.0, 0.0};
-  for (int r = t; r < n; r += 512) {
+  for (int r = t; r < NMAX; r += 64 * NW) tun[r] = double2{0.0, 0.0};
+  for (int r = t; r < n; r += 64 * NW) {
     const double x = AT(r, 0);
     xc[r] = x;
     if (r >= 1) tile[((r - 1) >> 5) * HTW + ((r - 1) & 31)] = x * x;
@@ -762,8 +773,7 @@ k_har_hess(const HarDesc *hd, const int *order) {
   __syncthreads();
   for (int i = 0; i + 2 < n; ++i) {
     const int rem = n - i - 1, m = rem - 1, asz = m & ~1;
-    const int Kn = rem <= 128 ? 128 : rem <= 170 ? 96 : 64;
-    if (Kn != K) {  // fewer rows: more resident columns
+    if (columns(rem) != K) {  // fewer rows: more resident columns
       flush(i + 1);
       __syncthreads();
       reside(i + 1);
@@ -2303,7 +2313,7 @@ void launch_haralick_prep(const Img *imgs, const Stats *st, const HarDesc *hd, i
 // scans the entries in index order (keys staged in LDS, chunk by chunk), so
 // ties keep index order and the order is the same on every run.
 //
-// order[nimg] (pick_too) tells which kernel finishes a launch of medium size
+// order[nimg + ORDER_PICK] (pick_too) tells which kernel finishes a launch of medium size
 // (launch_haralick_qr): 1 for k_har_schur<4>, whose 512 resident matrices make
 // short chains, 0 for k_har_qr, whose 4,096 make three times longer ones but do
 // 1.1 to 2.5 times as many matrices in all.  Both estimates, in ms, are fits to
@@ -2329,7 +2339,7 @@ __global__ void __launch_bounds__(320) k_har_order(const int *ng, int nimg, int 
     if (t == 0) {
       const double schur = 0.4 * top * (8.1e-3 + top * (2.05e-4 + top * 1.5e-7)) + chains / 512;
       const double qr = top * (3e-3 + top * (5.4e-4 + top * 8.1e-7)) + 0.5 * work;
-      order[nimg] = schur < qr;
+      order[nimg + ORDER_PICK] = schur < qr;
     }
   }
   if (t == 0) {
@@ -2341,6 +2351,11 @@ __global__ void __launch_bounds__(320) k_har_order(const int *ng, int nimg, int 
     }
   }
   __syncthreads();
+  if (t == 0) {  // cnt[256 - n]: entries of more than n tones
+    const int end = cnt[256 - 2], large = cnt[256 - HESS_SMALL];
+    order[nimg + ORDER_END] = end;
+    order[nimg + ORDER_LARGE] = end - large >= HESS_MANY ? large : end;
+  }
   int pos = t < 257 ? cnt[t] : 0;
   for (int base = 0; base < nimg; base += ORDER_CHUNK) {
     const int m = min(ORDER_CHUNK, nimg - base), m8 = (m + 7) & ~7;
@@ -2364,7 +2379,8 @@ void launch_haralick_order(const int *ng, int nimg, int *order, hipStream_t s) {
   k_har_order<<<1, 320, 0, s>>>(ng, nimg, order, haralick_pick(nimg));
 }
 void launch_haralick_hess(const HarDesc *hd, const int *order, int nimg, hipStream_t s) {
-  k_har_hess<<<dim3(4, nimg), 512, 0, s>>>(hd, order);
+  k_har_hess<8, 256><<<dim3(4, nimg), 512, 0, s>>>(hd, order);
+  if (nimg >= HESS_MANY) k_har_hess<1, HESS_SMALL><<<dim3(4, nimg), 64, 0, s>>>(hd, order);
   k_har_hess_rows<<<dim3(4, nimg, (256 - 2 + RWS - 1) / RWS), 64, 0, s>>>(hd, order);
 }
 void launch_haralick_qr(const HarDesc *hd, const int *order, bool no_polls, int nimg, hipStream_t s) {
@@ -2383,7 +2399,7 @@ void launch_haralick_qr(const HarDesc *hd, const int *order, bool no_polls, int 
   // 48.4, 2400 33.0 against 51.6, 4800 62.9 against 69.0; 7200 88.2 by one wave
   // against 93.9, 9600 112.0 against 124.8, 19200 201 against 259.
   const dim3 grid(4, nimg);
-  const int *pick = haralick_pick(nimg) ? order + nimg : nullptr;
+  const int *pick = haralick_pick(nimg) ? order + nimg + ORDER_PICK : nullptr;
   if (no_polls) k_har_schur<4, 0><<<grid, 256, 0, s>>>(hd, order, nullptr);
   else if (4 * nimg <= 256) k_har_schur<8><<<grid, 512, 0, s>>>(hd, order, nullptr);
   else if (4 * nimg <= 6144) k_har_schur<4><<<grid, 256, 0, s>>>(hd, order, pick);

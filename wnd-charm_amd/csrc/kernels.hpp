@@ -153,9 +153,11 @@ struct HarDesc {
 // Haralick in four stream-ordered steps: quantise / co-occurrence / f1..f13
 // / Q, Hessenberg reduction of Q, Francis QR (f14), mean and range output
 void launch_haralick_prep(const Img *imgs, const Stats *st, const HarDesc *hd, int nimg, int maxn, hipStream_t s);
-// order [nimg + 1]: the entries by decreasing ng (launch_haralick_order, from
-// the entries' ng values, contiguous), the dispatch order of the Hessenberg and
-// Schur kernels; behind them the Schur kernel picked
+// order [nimg + ORDER_EXTRA]: the entries by decreasing ng (launch_haralick_order,
+// from the entries' ng values, contiguous), the dispatch order of the Hessenberg
+// and Schur kernels.  Behind them the Schur kernel picked, the number of entries
+// that the Hessenberg kernel for large matrices takes, and of those of ng >= 3.
+enum { ORDER_PICK, ORDER_LARGE, ORDER_END, ORDER_EXTRA };
 void launch_haralick_order(const int *ng, int nimg, int *order, hipStream_t s);
 void launch_haralick_hess(const HarDesc *hd, const int *order, int nimg, hipStream_t s);
 // no_polls: the waves of k_har_schur give up at once where they would wait
