@@ -13,9 +13,9 @@ Also reported:
                 launch time measured live in the timed steps (HIP events
                 recorded around every launch on the stream that launch runs
                 on), against MI355X's FP64 peak: k_har_hess does (exactly)
-                hess_flops(Ng) per Q matrix, k_har_qr reports the flops its
-                Francis sweeps issued, k_gabor_conv 8 x 1444 complex taps per
-                pixel; traffic (HBM bytes per launch) is read from the
+                hess_flops(Ng) per Q matrix, the Schur kernels report the flops
+                their Francis sweeps issued, k_gabor_sep 8 x 228 multiply-adds
+                per pixel; traffic (HBM bytes per launch) is read from the
                 rocprofv3 --pmc summary committed under profiles/ when present.
   stage_ms_serial  per-launch times of the serial pass (the kernels' own
                 times, comparable with rocprofv3 under WNDGPU_SERIAL=1).
@@ -167,17 +167,28 @@ def profiled_traffic(kernel):
 
 
 def _gabor_flops(sizes):
-    """k_gabor_conv: 8 filters x 38 x 38 complex taps x 4 flops per root pixel"""
-    return float(8 * 1444 * 4 * sum(h * w for h, w in sizes))
+    """k_gabor_sep: 8 filters x (2 row sums of 38 taps + 2 complex column sums of 38 taps) x 2 flops per root pixel"""
+    return float(8 * 228 * 2 * sum(h * w for h, w in sizes))
+
+
+def schur_kernel(matrices):
+    """the kernel that a launch of so many matrices takes (launch_haralick_qr)"""
+    if matrices <= 256:
+        return 'k_har_schur<8>'
+    if matrices <= 1024:
+        return 'k_har_schur<4>'
+    return 'k_har_schur<4> or k_har_qr, by the tones' if matrices <= 6144 else 'k_har_qr'
 
 
 # launch name (as wndgpu_last_node_times reports it) -> (kernel, roof, work per step)
-# work(ctx) gets {'tones': Ng per Haralick entry, 'schur': Schur flops per matrix, 'root_sizes': [(h, w)]}
+# work(ctx) gets {'tones': Ng per Haralick entry, 'schur': Schur flops per matrix, 'root_sizes': [(h, w)]};
+# the kernel of the Schur stage goes by the matrices of a launch.  [k_har_hess] is that kernel and
+# k_har_hess_rows, Gabor Textures k_gabor_sep and the launches that count its energies.
 KERNEL_MODELS = {
-    'Haralick Textures [k_har_qr]': ('k_har_qr', 'fp64-valu', lambda w: float(w['schur'].sum())),
+    'Haralick Textures [k_har_qr]': (schur_kernel, 'fp64-valu', lambda w: float(w['schur'].sum())),
     'Haralick Textures [k_har_hess]': ('k_har_hess', 'fp64-valu',
                                        lambda w: float(4 * sum(hess_flops(int(n)) for n in w['tones']))),
-    'Gabor Textures': ('k_gabor_conv', 'fp64-valu', lambda w: _gabor_flops(w['root_sizes'])),
+    'Gabor Textures': ('k_gabor_sep', 'fp64-valu', lambda w: _gabor_flops(w['root_sizes'])),
 }
 
 
@@ -676,6 +687,8 @@ def main():
     dom = max((k for k in serial if k in KERNEL_MODELS), key=lambda k: serial[k])
     kname, bound, model = KERNEL_MODELS[dom]
     per_step = cnt[dom] // args.steps  # launches of that kernel per step
+    if callable(kname):
+        kname = kname(4 * len(tones) // per_step)
     flops = model(work)
     launch_ms = acc[dom] / cnt[dom]  # timed steps (two-stream schedule)
     achieved = flops / per_step / (launch_ms * 1e-3) / 1e12
@@ -685,7 +698,7 @@ def main():
             'launches_per_step': per_step, 'flops_per_launch': flops / per_step,
             'note': 'FP64 vector peak (equal to the FP64 matrix peak on MI355X); launch_ms from HIP events in '
                     'the timed steps, launch_ms_serial from the serial pass'}
-    if kname in ('k_har_qr', 'k_har_hess'):
+    if kname.startswith('k_har_'):
         roof['matrices_per_launch'] = 4 * len(tones) / per_step
     biggest = max(serial, key=serial.get)
     if biggest != dom:
