@@ -1577,7 +1577,7 @@ k_har_qr(const HarDesc *hd, const int *order, const int *pick) {
 //
 // What bounds it: the chain, about 100 instructions of wave 0 per step, issued
 // one per four cycles (an FP64 instruction's rate; dependent ones gain nothing
-// on independent ones): 660 cycles per step, 28,000 steps for 240 tones.  With
+// on independent ones): about 650 cycles per step, 28,000 steps for 240 tones.  With
 // one block of 256 threads chasing through an LDS window, as this kernel's
 // predecessor did, a step took 2,500 cycles: three LDS round trips, three IEEE
 // divisions and a square root with their scaling, and the strips in between.
@@ -2320,9 +2320,11 @@ void launch_haralick_prep(const Img *imgs, const Stats *st, const HarDesc *hd, i
 // order[nimg + ORDER_PICK] (pick_too) tells which kernel finishes a launch of medium size
 // (launch_haralick_qr): 1 for k_har_schur<4>, whose 512 resident matrices make
 // short chains, 0 for k_har_qr, whose 4,096 make three times longer ones but do
-// 1.1 to 2.5 times as many matrices in all.  Both estimates, in ms, are fits to
-// either kernel's times over launches of 4 x 400 .. 4 x 1500 matrices with equal
-// tones (8 .. 240), tones spread evenly from 0 and one entry in 40 of 256 tones.
+// 1.1 to 2.5 times as many matrices in all.  The estimates, in ms, follow either
+// kernel's times over 95 launches of 1,056 to 6,000 matrices: equal tones (8 ..
+// 240), tones spread evenly or thinly from 0, two kinds of them, one entry in 40 of
+// 256 tones, and nodes of images.  There the choice is the slower kernel by 2% at
+// most where that is k_har_schur, by 5% where it is k_har_qr.
 // Either kernel gives the same bits.
 constexpr int ORDER_CHUNK = 16384;
 __global__ void __launch_bounds__(320) k_har_order(const int *ng, int nimg, int *order, int pick_too) {
@@ -2334,18 +2336,6 @@ __global__ void __launch_bounds__(320) k_har_order(const int *ng, int nimg, int 
   __syncthreads();
   for (int e = t; e < nimg; e += blockDim.x) atomicAdd(&cnt[256 - min(max(ng[e], 0), 256)], 1);
   __syncthreads();
-  if (pick_too) {
-    const double n = 256 - t, m = t < 257 ? 4.0 * cnt[t] : 0.0;
-    const double chain = n * (8.1e-3 + n * (2.05e-4 + n * 1.5e-7));  // one matrix by k_har_schur<4>
-    const double top = block_reduce(m > 0 ? n : 0.0, MaxOp(), shd);
-    const double chains = block_reduce(m * chain, SumOp(), shd);
-    const double work = block_reduce(m * n * n * (1.5e-7 + n * 7.6e-10), SumOp(), shd);
-    if (t == 0) {
-      const double schur = 0.4 * top * (8.1e-3 + top * (2.05e-4 + top * 1.5e-7)) + chains / 512;
-      const double qr = top * (3e-3 + top * (5.4e-4 + top * 8.1e-7)) + 0.5 * work;
-      order[nimg + ORDER_PICK] = schur < qr;
-    }
-  }
   if (t == 0) {
     int sum = 0;
     for (int b = 0; b < 257; b++) {
@@ -2355,6 +2345,21 @@ __global__ void __launch_bounds__(320) k_har_order(const int *ng, int nimg, int 
     }
   }
   __syncthreads();
+  if (pick_too) {
+    const double n = 256 - t, m = t < 257 ? 4.0 * ((t < 256 ? cnt[t + 1] : nimg) - cnt[t]) : 0.0;
+    const double chain = n * (8.1e-3 + n * (2.05e-4 + n * 1.5e-7));  // one matrix by k_har_schur<4>
+    // its matrices from the largest to order n need so many rounds of 512, none shorter
+    const double rounds = m > 0 ? ceil((t < 256 ? cnt[t + 1] : nimg) / 128.0) * chain : 0.0;
+    const double longest = block_reduce(rounds, MaxOp(), shd);
+    const double chains = block_reduce(m * chain, SumOp(), shd);
+    const double top = block_reduce(m > 0 ? n : 0.0, MaxOp(), shd);
+    const double work = block_reduce(m * n * n * (1.5e-7 + n * 7.6e-10), SumOp(), shd);
+    if (t == 0) {
+      const double schur = fmax(longest, chains / 512);
+      const double qr = top * (3e-3 + top * (5.4e-4 + top * 8.1e-7)) + 0.42 * work;
+      order[nimg + ORDER_PICK] = schur < qr;
+    }
+  }
   if (t == 0) {  // cnt[256 - n]: entries of more than n tones
     const int end = cnt[256 - 2], large = cnt[256 - HESS_SMALL];
     order[nimg + ORDER_END] = end;
@@ -2397,11 +2402,11 @@ void launch_haralick_qr(const HarDesc *hd, const int *order, bool no_polls, int 
   // three times slower, but it does less work per step, and with that many the
   // work counts.  Between, it depends on the tones, which only the device knows:
   // 1600 matrices of 64 equal tones 5.4 ms by four waves and 3.4 by one, of 0 ..
-  // 253 tones 21.4 and 49.9.  Both are launched and one of them returns at once.
-  // Nodes of 256 x 256 images (tones 10..256, mean 128): 48 matrices 12.4 ms (30.6
-  // with one 256-thread block per matrix; four waves: 17.5), 1200 18.3 against
-  // 48.4, 2400 33.0 against 51.6, 4800 62.9 against 69.0; 7200 88.2 by one wave
-  // against 93.9, 9600 112.0 against 124.8, 19200 201 against 259.
+  // 253 tones 21.6 and 49.9.  Both are launched and one of them returns at once.
+  // Nodes of 256 x 256 images (tones 10..256, mean 128): 48 matrices 12.5 ms (30.6
+  // with one 256-thread block per matrix; four waves: 17.5), 1200 18.5 against
+  // 47.4, 2400 33.3 against 51.1, 4800 63.1 against 69.2; 7200 87.7 by one wave
+  // against 93.9, 9600 112.0 against 124.8, 19200 200 against 259.
   const dim3 grid(4, nimg);
   const int *pick = haralick_pick(nimg) ? order + nimg + ORDER_PICK : nullptr;
   if (no_polls) k_har_schur<4, 0><<<grid, 256, 0, s>>>(hd, order, nullptr);
