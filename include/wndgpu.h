@@ -115,6 +115,9 @@ const char *wndgpu_plan_feature_name(const wndgpu_plan *plan, int column);
  * count that its interval leaves open (maximum, minimum, Otsu bin,
  * threshold, base count) is taken on the energy recomputed in FP64 in the
  * plain form's order: integer-valued features equal the plain form's.  The
+ * plain form is the faster one, as it filters along rows and columns (1000
+ * images of 128 x 128: 8 ms for the Gabor group, 25 in FP32, 27 in BF16X3):
+ * the reduced forms are for comparing arithmetic, not for speed.  The
  * Chebyshev and Chebyshev-Fourier histograms and the Zernike sums stay FP64
  * in every precision.  Set the precision on a plan of your own
  * (wndgpu_plan_from_groups): the standard plans are meant to stay plain. */

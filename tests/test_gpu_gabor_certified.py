@@ -1,5 +1,5 @@
 """Gabor textures of the plain form (GaborTextureFilters2D, gabor.cpp:201-231
-in the reference): the energies are convolved with FP64 fused multiply-adds,
+in the reference): the energies are filtered along rows and columns in FP64,
 each with an a-priori bound on its distance from the reference's separate
 multiply-and-add value, and every count is decided from those bounds, the
 energies a decision leaves open being recomputed in the reference's order.

@@ -363,7 +363,7 @@ struct wndgpu_ctx {
   int *cf_open = nullptr;
   int cf_n = 0;
   double cf_slack = 1;
-  // Gabor energies of the plain form: FP64 fused multiply-adds whose counts
+  // Gabor energies of the plain form: FP64 row and column filters whose counts
   // are certified (the default), or the reference's separate multiply and
   // add throughout (gabor_direct, WNDGPU_GABOR_DIRECT=1 at creation).
   // gabor_slack (WNDGPU_GABOR_SLACK, >= 1) scales the certification bound.

@@ -2626,7 +2626,7 @@ __device__ __forceinline__ double mean_diff(double a0, double c0, double r0, dou
 //
 // Bound by instruction issue, so a wave takes 64 columns and goes down tam_rows
 // rows: what depends on the row alone is scalar, and the rows' neighbours stay in
-// registers.  4,800 planes of up to 256 x 256: 9.9 ms; 18.0 ms with four table
+// registers.  4,800 planes of up to 256 x 256: 10.4 ms; 18.0 ms with four table
 // entries per mean, 12.9 ms with one thread per pixel.
 __global__ void __launch_bounds__(256, 3) k_tam_pix(const Img *imgs, double *const *scr, int nimg, int per_img) {
   __shared__ double recip[129];
