@@ -1187,7 +1187,7 @@ static int build_batch(wndgpu_ctx *c, const wndgpu_plan *plan, const Batch &B, A
         });
         push_side(gn + " [k_har_hess]", [=](hipStream_t s2) { launch_haralick_hess(hdd, order, ne, s2); });
         push_side(gn + " [k_har_qr]", [=](hipStream_t s2) { launch_haralick_qr(hdd, order, no_polls, ne, s2); });
-        push_side(gn + " [mean, range]", [=](hipStream_t s2) { launch_haralick_final(hdd, o, lost, ne, s2); });
+        push_side(gn + " [mean, range]", [=](hipStream_t s2) { launch_haralick_final(hdd, order, o, lost, ne, s2); });
       } break;
       case A_ZERNIKE: {
         const int nchunk = (int)std::max<long>(1, std::min<long>(64, (maxp + 4095) / 4096));

@@ -2192,21 +2192,27 @@ k_har_schur(const HarDesc *hd, const int *order, const int *pick) {
             const SchurRf *R = rf[par];
             // wave 0 publishes every step of its window, within microseconds.
             // Should it not, the sweeps end all the same (their number is
-            // limited), on what lies in LDS, and k_har_final finds count < 0 and
-            // fails the call.  How the wave remembers it is a matter of registers:
-            // a store from here costs 13% of four-wave launches of few tones (26
-            // spilled registers for 12), base < 0 as its mark 2% of eight-wave ones.
+            // limited), on what lies in LDS, and k_har_final finds the mark and
+            // fails the call.  What the mark is and where it is set decide which
+            // registers the compiler spills: so, either launch takes 0.7 to 1% more
+            // than without one; with the other's, 1.4 and 1.5%.
+            auto lose = [&] {
+              if (NW == 8) H.count[angle] = -1;
+              else const_cast<int *>(order)[gridDim.y + ORDER_LOST] = 1;
+            };
             auto await = [&](int q) {
-              for (int spin = 0; __builtin_amdgcn_readfirstlane(__hip_atomic_load(
-                                     &R[q].gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) != base + q + 1;
-                   spin++) {
-                if (spin >= POLLS || (NW == 4 && base < 0)) {
-                  if (NW == 4) base = -(1 << 30);
-                  else H.count[angle] = -1;
+              int spin = 0;
+              for (; NW == 8 || spin < POLLS; spin++) {
+                if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(&R[q].gen, __ATOMIC_RELAXED,
+                                                                     __HIP_MEMORY_SCOPE_WORKGROUP)) == base + q + 1)
+                  break;
+                if (NW == 8 && spin == POLLS) {
+                  lose();
                   break;
                 }
                 __builtin_amdgcn_s_sleep(1);
               }
+              if (NW == 4 && __builtin_expect(spin == POLLS, 0)) lose();
               __asm__ volatile("" ::: "memory");
             };
 #pragma unroll
@@ -2267,17 +2273,17 @@ k_har_schur(const HarDesc *hd, const int *order, const int *pick) {
     H.feat[angle * 14 + 13] = f;
     H.work[angle] = work;
   }
-  if (NW == 4 && base < 0 && lane == 0) H.count[angle] = -1;
 #undef AT
 }
 
 // mean and range over the 4 angles, reference output order (haralick.cpp:96-143)
 // *lost: a wave of k_har_schur waited in vain
-__global__ void k_har_final(const HarDesc *hd, OutRef o, int *lost) {
+__global__ void k_har_final(const HarDesc *hd, const int *order, OutRef o, int *lost) {
   const HarDesc H = hd[blockIdx.x];
   if (threadIdx.x != 0) return;
-  for (int g = 0; g < 4; g++)
-    if (H.count[g] < 0) __hip_atomic_store(lost, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  bool hit = order[gridDim.x + ORDER_LOST] != 0;
+  for (int g = 0; g < 4; g++) hit |= H.count[g] < 0;
+  if (hit) __hip_atomic_store(lost, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   double temp[28];
   for (int a = 0; a < 14; a++) {
     double s = 0, mn = kInf, mx = -kInf;
@@ -2363,6 +2369,7 @@ __global__ void __launch_bounds__(320) k_har_order(const int *ng, int nimg, int 
   if (t == 0) {  // cnt[256 - n]: entries of more than n tones
     const int end = cnt[256 - 2], large = cnt[256 - HESS_SMALL];
     order[nimg + ORDER_END] = end;
+    order[nimg + ORDER_LOST] = 0;
     order[nimg + ORDER_LARGE] = end - large >= HESS_MANY ? large : end;
   }
   int pos = t < 257 ? cnt[t] : 0;
@@ -2409,13 +2416,14 @@ void launch_haralick_qr(const HarDesc *hd, const int *order, bool no_polls, int 
   // against 93.9, 9600 112.0 against 124.8, 19200 200 against 259.
   const dim3 grid(4, nimg);
   const int *pick = haralick_pick(nimg) ? order + nimg + ORDER_PICK : nullptr;
-  if (no_polls) k_har_schur<4, 0><<<grid, 256, 0, s>>>(hd, order, nullptr);
+  if (no_polls && 4 * nimg <= 256) k_har_schur<8, 0><<<grid, 512, 0, s>>>(hd, order, nullptr);
+  else if (no_polls) k_har_schur<4, 0><<<grid, 256, 0, s>>>(hd, order, nullptr);
   else if (4 * nimg <= 256) k_har_schur<8><<<grid, 512, 0, s>>>(hd, order, nullptr);
   else if (4 * nimg <= 6144) k_har_schur<4><<<grid, 256, 0, s>>>(hd, order, pick);
   if (!no_polls && (pick || 4 * nimg > 6144)) k_har_qr<<<grid, 64, 0, s>>>(hd, order, pick);
 }
-void launch_haralick_final(const HarDesc *hd, OutRef o, int *lost, int nimg, hipStream_t s) {
-  k_har_final<<<nimg, 64, 0, s>>>(hd, o, lost);
+void launch_haralick_final(const HarDesc *hd, const int *order, OutRef o, int *lost, int nimg, hipStream_t s) {
+  k_har_final<<<nimg, 64, 0, s>>>(hd, order, o, lost);
 }
 
 // ======================================================================= Tamura

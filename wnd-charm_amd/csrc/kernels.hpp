@@ -156,14 +156,16 @@ void launch_haralick_prep(const Img *imgs, const Stats *st, const HarDesc *hd, i
 // order [nimg + ORDER_EXTRA]: the entries by decreasing ng (launch_haralick_order,
 // from the entries' ng values, contiguous), the dispatch order of the Hessenberg
 // and Schur kernels.  Behind them the Schur kernel picked, the number of entries
-// that the Hessenberg kernel for large matrices takes, and of those of ng >= 3.
-enum { ORDER_PICK, ORDER_LARGE, ORDER_END, ORDER_EXTRA };
+// that the Hessenberg kernel for large matrices takes, and of those of ng >= 3;
+// whether a wave of k_har_schur's four-wave form gave up waiting (the other's
+// makes its entry's count negative).
+enum { ORDER_PICK, ORDER_LARGE, ORDER_END, ORDER_LOST, ORDER_EXTRA };
 void launch_haralick_order(const int *ng, int nimg, int *order, hipStream_t s);
 void launch_haralick_hess(const HarDesc *hd, const int *order, int nimg, hipStream_t s);
 // no_polls: the waves of k_har_schur give up at once where they would wait
 void launch_haralick_qr(const HarDesc *hd, const int *order, bool no_polls, int nimg, hipStream_t s);
 // *lost (host memory) becomes 1 if a wave of k_har_schur gave up
-void launch_haralick_final(const HarDesc *hd, OutRef o, int *lost, int nimg, hipStream_t s);
+void launch_haralick_final(const HarDesc *hd, const int *order, OutRef o, int *lost, int nimg, hipStream_t s);
 size_t tamura_scratch(int h, int w);  // doubles per plane
 void launch_tamura(const Img *imgs, const Stats *st, double *const *scratch, OutRef o, int nimg, int maxh, int maxw,
                    hipStream_t s);
